@@ -274,8 +274,9 @@ int wxo_quantize_pack_q8_multi(const float* const* inputs, const uint32_t* Ns, u
 
 /* matmulQ8: output[n*M + m] = (sum_{k<K} a[n*K + k] * sext8(byte k of weight row m)) * scale[m]
  * for n < N (tokens), m < M (weight rows).  a f32 [N, K], weight u32 [M, ceil(K/4)],
- * scale f32 [M], output f32 [N, M].  f32 accumulation on the matrix cores (exact
- * products); |y - y_ref| <= 1e-5 * sum_k |a * q * s| + 1e-7 against the reference's f64
+ * scale f32 [M], output f32 [N, M].  f32 accumulation on the matrix cores (each
+ * activation as a scaled f16 pair, exact to 2^-23, or exactly where it has no
+ * such pair); |y - y_ref| <= 1e-5 * sum_k |a * q * s| + 1e-7 against the reference's f64
  * sum of per-term dequantized products.  K = 0 gives zeros.  K <= 2^22. */
 int wxo_matmul_q8(const float* a, const uint32_t* weight, const float* scale, float* output, uint32_t N,
                   uint32_t M, uint32_t K, wxo_stream_t stream);

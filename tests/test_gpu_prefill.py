@@ -780,3 +780,46 @@ def test_matmul_weight_past_4_gib():
     cols = np.unique(np.concatenate([np.arange(64), np.arange(M - 100, M), rng.integers(0, M, 256)]))
     wsub = w.reshape(M, W)[cols].reshape(-1)
     assert_matmul(np.ascontiguousarray(y[:, cols]), a, wsub, s[cols], T, len(cols), K)
+
+
+@pytest.mark.parametrize("N,M,K,ws", [
+    (40, 300, 1030, False),    # 32-row tiles, two K groups
+    (40, 300, 2100, True),     # the same, K split between workgroups
+    (300, 2048, 520, False),   # 64-row tiles
+    (256, 6144, 200, False),   # 128-row tiles, two K groups
+    (700, 3548, 1030, True),   # 128-row tiles, the last ones' K steps split
+    (512, 6100, 330, False),   # 256-row tiles
+    (510, 11200, 330, False),  # 384-row tiles
+])
+def test_matmul_activations_past_the_f16_window(N, M, K, ws):
+    """Activations that the scaled f16 pair does not hold (large, tiny,
+    subnormal and infinite ones among ordinary ones, and a token tile of tiny
+    ones only) take the exact three-part split.  A third of the weight rows
+    see the tiny ones alone (their other codes are 0), under scales that make
+    those sums of order 1, so the matmulQ8 bar is relative to them."""
+    rng = np.random.default_rng(N + M + K)
+    a = rng.standard_normal((N, K)).astype(np.float32)
+    tiny = rng.choice(K, 24, replace=False)
+    a[:, tiny] *= np.float32(1e-12)
+    a[1, tiny] = np.float32(1e-41)  # subnormal
+    big = rng.choice(np.setdiff1d(np.arange(K), tiny), 8, replace=False)
+    a[::3, big] *= np.float32(3e6)
+    a[5 % N, big[0]] = np.float32(1e36)
+    a[N // 2, big[1]] = np.inf
+    a[7 % N] = 0
+    a[min(N - 1, 64):min(N, 128)] *= np.float32(1e-20)
+    codes = rng.integers(-128, 128, (M, K)).astype(np.int32)
+    lone = np.arange(M) % 3 == 0
+    codes[np.ix_(lone, np.setdiff1d(np.arange(K), tiny))] = 0
+    s = rng.uniform(0.001, 0.05, M).astype(np.float32)
+    s[lone] = np.float32(1e10)
+    w = oracle.pack_q8(codes.reshape(-1), M, K)
+    ba, bw, bs = (wxo_q8.DeviceBuffer.from_array(v) for v in (a.reshape(-1), w, s))
+    out = wxo_q8.DeviceBuffer(4 * N * M)
+    nbytes = wxo_q8.matmul_q8_workspace_bytes() if ws else 0
+    work = wxo_q8.DeviceBuffer(nbytes) if ws else None
+    wxo_q8.matmul_q8_multi_device(ba, [(bw, bs, out, M)], N, K, workspace=work, workspace_bytes=nbytes)
+    wxo_q8.synchronize()
+    print(wxo_q8.last_variant(), flush=True)
+    rows = np.unique(np.r_[np.arange(0, N, 23), 1, 5 % N, 7 % N, N // 2, min(N - 1, 70), N - 1])
+    assert_matmul(out.download(np.float32, N * M), a, w, s, N, M, K, rows=rows)

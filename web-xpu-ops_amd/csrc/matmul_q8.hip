@@ -11,33 +11,32 @@
 // by at most one f32 rounding of each term, 2^-24 of sum |a * q * s|, far
 // inside the 1e-5 bar the tests hold.
 //
-// Exactness on bf16 matrix cores: a code q in [-128, 127] is exact in bf16;
-// each activation a is split by truncation into a = h + m + l, three bf16
-// parts of 8 significant bits each (a non-finite a stays whole in h, with a
-// canonical quiet NaN), so every product q * part is exact in f32 and
-// v_mfma_f32_16x16x32_bf16 sums them in f32.  Each 1024-code slice of K is
-// summed in the matrix-core accumulator (96 accumulations) and then folded
-// into an outer f32 sum, so no rounding chain exceeds ~96 + K/1024 steps:
-// for K = 11008 that is under 110 roundings, 7e-6 of sum |terms|.
+// Numerics on the f16 matrix cores: a code q in [-128, 127] is exact in f16;
+// an activation, scaled by a power of two of its run's, becomes a pair of f16 h
+// + l / 2048 (split2: exact to 2^-23 of it over 30 binades), every product
+// q * part is exact in f32, and v_mfma_f32_16x16x32_f16 sums the two planes in
+// two f32 accumulators.  Each 1024-code slice of K is summed there (32
+// accumulations a plane) and then folded into an outer f32 sum, so no rounding
+// chain exceeds 32 + K/1024 steps.  Values outside the 30 binades (infinite,
+// past 65504 after the scale, or nonzero and under 2^-16) flag their step, and
+// their products come from an exact three-part bf16 split instead (slow_steps),
+// so every f32 activation is taken as precisely as before.  Against 64 bits,
+// 2-norm: 1.69e-7 at K = 2048 to 5632, where three bf16 parts in one
+// accumulator (96 accumulations per fold) had 3.1e-7; and a third less matrix
+// work, LDS traffic and splitting.
 //
-// Tiling: a workgroup of NW = 8 waves (2 over the weight rows x 4 over the
-// tokens; 4 waves, 2 x 2, also build) owns BM = 32 FB weight rows x BN = 64
-// tokens and walks K in steps of 64 codes.  Each step, the threads load the
-// tile's packed codes (one dwordx4 of 16 codes per chunk) and activations
-// (one token's 64 / NW consecutive k per thread), convert them once (codes ->
-// bf16, activations -> three bf16 parts) into LDS, and after one barrier
-// every wave reads its operand fragments with ds_read_b128 and issues
-// FB x (4 / (NW / 2)) x 2 x 3 matrix-core ops.  Two waves per SIMD let one
-// wave's LDS and barrier waits overlap the other's work (measured: 357 ->
-// 310 us for a 512-token layer against 4 waves).
-// The LDS holds two stages: while a wave's matrix cores work on step i, its
-// VALU converts step i + 1 into the other stage, and global loads run two
-// steps ahead of their conversion in two register sets.  The non-finite handling of the split is a wave-uniform branch taken
-// only by waves that hold an Inf or NaN.  Rows of 64 codes (128 bytes of bf16) are
-// stored with their 16-byte pieces XOR-swizzled by row, so the 16 rows one
-// fragment read touches fall in distinct bank groups.
+// Tiling (matmul_q8_kernel, short prompts): a workgroup of two K groups of 8
+// waves (2 over the weight rows x 4 over the tokens) owns BM = 32 FB weight
+// rows x BN = 64 tokens and walks K in steps of 64 codes.  Each step, the
+// threads load the tile's packed codes (one dwordx4 of 16 codes per chunk) and
+// activations (8 consecutive k of one token per thread), convert them once into
+// LDS, and after one barrier every wave reads its operand fragments with
+// ds_read_b128.  The LDS holds two stages: while a wave's matrix cores work on
+// step i, its VALU converts step i + 1 into the other stage, and global loads
+// run four steps ahead of their conversion.  Rows of 64 codes (128 bytes of
+// f16) are stored with their 16-byte pieces swizzled by row (piece_offset).
 //
-// Operand layout of v_mfma_f32_16x16x32_bf16 (probed on gfx950): A lane l
+// Operand layout of v_mfma_f32_16x16x32_{f16,bf16} (probed on gfx950): A lane l
 // holds A[l % 16][8 (l / 16) + e], B lane l holds B[8 (l / 16) + e][l % 16],
 // C lane l holds C[4 (l / 16) + v][l % 16].  A = weight rows (16 features),
 // B = activations (16 tokens), so a lane's C values are 4 consecutive
@@ -60,18 +59,11 @@
 // and scales them.  The stream order between the two launches is the only
 // synchronisation, so every run gives the same bits.
 //
-// Long rows whose tiles make whole rounds of two per CU run one workgroup of
-// 16 waves per two tiles, each group of 8 waves on a tile of its own (the
-// PAIR instances); the sums are the one-group form's.
-//
 // Launches with enough tiles for one workgroup per CU, and short prompts'
-// 256-row tiles split 4 or 8 ways, run matmul_q8_direct_kernel instead: every wave of 8 owns 16 FW weight rows and
-// all 64 tokens of the tile, and loads its rows' codes straight into VGPRs
-// (two dwordx2 per 16-row block and step, in the operand's k order), so only
-// the activation parts pass through LDS.  That removes the codes' LDS writes
-// (gfx950 writes LDS at ~75 B/clk per CU against ~200 for reads) and converts
-// each code once per wave, at the matrix work.  Same sums in the same order
-// as the one-group form, so the same bits; 2-7 % faster than it.
+// 256-row tiles split 4 or 8 ways, run matmul_q8_direct_kernel instead: every
+// wave owns 32 or 48 weight rows and all 64 tokens of the tile, and loads its
+// rows' codes straight into VGPRs (one dwordx4 per 16-row block and step), so
+// only the activation pairs pass through LDS.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -83,6 +75,9 @@ namespace wxo {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
 
@@ -132,24 +127,36 @@ __device__ __forceinline__ uint32_t hi_pair(uint32_t a, uint32_t b) {
     return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 
-// 16 codes (4 packed words) -> 16 bf16 in two 16-byte pieces.
-__device__ __forceinline__ void codes16_to_bf16(u32x4v w, u32x4v& lo, u32x4v& hi) {
-    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+// 4 codes (a packed word) -> 4 f16, exactly: code + 128 is the low byte of the
+// f16 1024 + (code + 128), so a byte permute and one packed add convert two
+// codes (2.5 VALU ops per two codes; through f32 and bf16 it was 3).
+__device__ __forceinline__ void codes4_to_f16(uint32_t w, uint32_t& lo, uint32_t& hi) {
+    const f16x2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    const uint32_t u = w ^ 0x80808080u;
+    lo = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) + bias);
+    hi = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) + bias);
+}
+
+// 16 codes (4 packed words) -> 16 f16 in two 16-byte pieces.
+__device__ __forceinline__ void codes16_to_f16(u32x4v w, u32x4v& lo, u32x4v& hi) {
     uint32_t r[8];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const float c0 = (float)(int8_t)(ws[q]);
-        const float c1 = (float)(int8_t)(ws[q] >> 8);
-        const float c2 = (float)(int8_t)(ws[q] >> 16);
-        const float c3 = (float)((int32_t)ws[q] >> 24);
-        r[2 * q] = hi_pair(__float_as_uint(c0), __float_as_uint(c1));
-        r[2 * q + 1] = hi_pair(__float_as_uint(c2), __float_as_uint(c3));
-    }
+    codes4_to_f16(w.x, r[0], r[1]);
+    codes4_to_f16(w.y, r[2], r[3]);
+    codes4_to_f16(w.z, r[4], r[5]);
+    codes4_to_f16(w.w, r[6], r[7]);
     lo = u32x4v{r[0], r[1], r[2], r[3]};
     hi = u32x4v{r[4], r[5], r[6], r[7]};
 }
 
-// 8 codes (2 packed words) -> 8 bf16.
+// 8 codes (2 packed words) -> 8 f16.
+__device__ __forceinline__ f16x8 codes8_to_f16(uint32_t w0, uint32_t w1) {
+    uint32_t r[4];
+    codes4_to_f16(w0, r[0], r[1]);
+    codes4_to_f16(w1, r[2], r[3]);
+    return __builtin_bit_cast(f16x8, u32x4v{r[0], r[1], r[2], r[3]});
+}
+
+// 8 codes (2 packed words) -> 8 bf16 (the exact three-part step only).
 __device__ __forceinline__ bf16x8 codes8_to_bf16(u32x2v w) {
     const uint32_t ws[2] = {w.x, w.y};
     uint32_t r[4];
@@ -165,19 +172,95 @@ __device__ __forceinline__ bf16x8 codes8_to_bf16(u32x2v w) {
     return __builtin_bit_cast(bf16x8, u32x4v{r[0], r[1], r[2], r[3]});
 }
 
-// Splits activations into bf16 parts h + m + l (bit patterns in the upper
-// halves).  Finite values split exactly by truncation: h keeps the top 8
-// significant bits, r = a - h is exact, m keeps r's top 8, l = r - m is exact
-// with at most 8 significant bits.  A non-finite value keeps all of itself in
-// h (a NaN canonicalised, so truncating its payload cannot make it Inf) and
-// m = l = 0, so Inf and NaN reach the products as IEEE arithmetic has them.
-__device__ __forceinline__ void split3_fast(uint32_t bits, uint32_t& h, uint32_t& m, uint32_t& l, float& r) {
-    h = bits & 0xffff0000u;
-    r = __uint_as_float(bits) - __uint_as_float(h);
-    m = __float_as_uint(r) & 0xffff0000u;
-    l = __float_as_uint(r - __uint_as_float(m));
+// Where 16-byte piece p (8 codes or activations) of a 128-byte LDS row sits:
+// even pieces in the first half and odd ones in the second, so that the four
+// lane groups of a fragment read (pieces 2 g + h, g = 0 .. 3) find theirs side
+// by side, then XOR-swizzled by row.  Reads and writes are then free of bank
+// conflicts (p ^ row alone cost a fifth of the 2048-token launch's cycles).
+__device__ __forceinline__ uint32_t piece_offset(uint32_t p, uint32_t row) {
+    return ((((p & 1u) << 2) | (p >> 1)) ^ (row & 7u)) * 16u;
 }
 
+// Two activations -> their f16 pairs.  t = x * 2^s (s the tile's, exact), h =
+// f16(t) and l = f16(2048 (t - h)), both rounded to nearest: t - h is exact,
+// so h + l / 2048 is t to 2^-23 of it while h is a normal f16, i.e. for
+// 2^-14 <= |t| <= 65504, and to 2^-20 from 2^-16 up.  lo and hi collect the
+// smallest and largest |t|.
+constexpr float kPartScale = 2048.0f;
+constexpr float kPartMin = 1.52587890625e-05f;  // 2^-16
+constexpr float kPartMax = 65504.0f;
+__device__ __forceinline__ void split2(float x0, float x1, float up, uint32_t& h, uint32_t& l, float& lo, float& hi) {
+    const float t0 = x0 * up, t1 = x1 * up;
+    const f16x2 hp = __builtin_convertvector((f32x2v){t0, t1}, f16x2);
+    const float r0 = __builtin_fmaf(x0, up, -(float)hp.x), r1 = __builtin_fmaf(x1, up, -(float)hp.y);
+    const f16x2 lp = __builtin_convertvector((f32x2v){r0 * kPartScale, r1 * kPartScale}, f16x2);
+    h = __builtin_bit_cast(uint32_t, hp);
+    l = __builtin_bit_cast(uint32_t, lp);
+    lo = __builtin_fminf(__builtin_fminf(__builtin_fabsf(t0), __builtin_fabsf(t1)), lo);
+    hi = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(t0), __builtin_fabsf(t1)), hi);
+}
+
+// True (wave-uniform) if the wave holds a value that its pair does not
+// represent: infinite, past 65504 or, not being 0, under 2^-16 after the scale
+// (lo and hi as split2 collected them over v; least: 2^-16, or 0 for a token
+// past the tile's, whose values are all 0).  Such a wave writes zeros and
+// flags the step, and slow_steps adds its tokens' products from the exact
+// three-part split.  NaNs stay: their token's sums are NaN either way.
+__device__ __forceinline__ bool needs_slow(const uint32_t (&v)[8], float least, float down, float lo, float hi) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(lo >= least && hi <= kPartMax)) == 0, 1)) return false;
+    // zeros also read as too small: tell them apart (2 |bits| - 1 wraps for 0)
+    uint32_t small = 0xffffffffu;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) small = min(small, (v[e] << 1) - 1u);
+    const bool bad = small < (__float_as_uint(kPartMin * down) << 1) - 1u || !(hi <= kPartMax);
+    return __builtin_amdgcn_ballot_w64(bad) != 0;
+}
+
+// Eight consecutive activations of one token -> `w` and `w + plane` in LDS
+// (zeros where the step needs slow_steps, which is returned; written over the
+// pairs, so that the conversion stays free of the branch).
+__device__ __forceinline__ bool store_split(const uint32_t (&v)[8], float least, float up, float down, uint8_t* w,
+                                            uint32_t plane) {
+    uint32_t hp[4], lp[4];
+    float lo = kPartMax, hi = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split2(__uint_as_float(v[2 * e]), __uint_as_float(v[2 * e + 1]), up, hp[e], lp[e], lo, hi);
+    *reinterpret_cast<u32x4v*>(w) = u32x4v{hp[0], hp[1], hp[2], hp[3]};
+    *reinterpret_cast<u32x4v*>(w + plane) = u32x4v{lp[0], lp[1], lp[2], lp[3]};
+    const bool bad = needs_slow(v, least, down, lo, hi);
+    if (bad) {
+        *reinterpret_cast<u32x4v*>(w) = u32x4v{0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4v*>(w + plane) = u32x4v{0u, 0u, 0u, 0u};
+    }
+    return bad;
+}
+
+// The tile's power of two, from the sum of |x| over its first 64 x 64
+// activations: their mean lands in [2^6, 2^7), which leaves 2^9 of it above
+// and 2^-22 below before a step takes the slow form.  All zero or not finite:
+// no scaling.  Every power stays far from the f32 range's ends.
+__device__ __forceinline__ int part_exponent(float abssum) {
+    const int e = (int)((__float_as_uint(abssum) >> 23) & 0xffu);
+    if (e == 0 || e == 0xff) return 0;
+    const int s = 6 + 12 - (e - 127);  // the mean is abssum / 2^12
+    return s > 100 ? 100 : (s < -100 ? -100 : s);
+}
+__device__ __forceinline__ float pow2f(int s) { return __uint_as_float((uint32_t)(127 + s) << 23); }
+
+__device__ __forceinline__ float wave_sum(float v) {
+    v += partner_f32<1>(v);
+    v += partner_f32<2>(v);
+    v += partner_f32<4>(v);
+    v += partner_f32<8>(v);
+    v = swap_add<16>(v, v);
+    return swap_add<32>(v, v);
+}
+
+// Three bf16 parts of an activation, exactly, whatever its exponent: h keeps
+// the top 8 significant bits by truncation, m the next 8, l the rest (r = a -
+// h and r - m are exact).  A non-finite value keeps all of itself in h (a NaN
+// canonicalised, so truncating its payload cannot make it Inf) and m = l = 0,
+// so Inf reaches the products as IEEE arithmetic has it.
 __device__ __forceinline__ void split3_any(uint32_t bits, uint32_t& h, uint32_t& m, uint32_t& l) {
     const bool finite = (bits & 0x7f800000u) != 0x7f800000u;
     const bool nan = (bits & 0x7fffffffu) > 0x7f800000u;
@@ -188,25 +271,112 @@ __device__ __forceinline__ void split3_any(uint32_t bits, uint32_t& h, uint32_t&
     l = __float_as_uint(r - __uint_as_float(m));
 }
 
+// One 64-code step of a wave's FW x TB blocks for the tokens whose converting
+// wave flagged it: `groups` bit i stands for the tile's tokens 8 i .. 8 i + 7.
+// Codes and activations come straight from memory, in the operand's k order,
+// the activations split in three; other tokens' values count as 0, so adding
+// the products (add(f, b, block)) completes the step whatever the other waves found.
+template <int FW, int TB, typename Add>
+__device__ __forceinline__ void slow_step(__amdgpu_buffer_rsrc_t wrs, __amdgpu_buffer_rsrc_t ars, uint32_t wm,
+                                          uint32_t wn, uint32_t rowbytes, uint32_t K, uint32_t k0, uint32_t groups,
+                                          Add&& add) {
+    const uint32_t lane = threadIdx.x & 63u, j = lane & 15u, g = lane >> 4;
+#pragma unroll 1
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t k = k0 + 16u * g + 8u * (uint32_t)h;
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            const uint32_t tk = wn + 16u * (uint32_t)b + j;
+            if (((groups >> ((wn >> 3) + 2u * (uint32_t)b)) & 3u) == 0u) continue;  // uniform
+            const bool mine = ((groups >> (tk >> 3)) & 1u) != 0u;
+            uint32_t x[8], hp[4], mp[4], lp[4];
+            const u32x4v x0 = __builtin_amdgcn_raw_buffer_load_b128(ars, (int)((tk * K + k) * 4u), 0, 0);
+            const u32x4v x1 = __builtin_amdgcn_raw_buffer_load_b128(ars, (int)((tk * K + k) * 4u + 16u), 0, 0);
+            x[0] = x0.x; x[1] = x0.y; x[2] = x0.z; x[3] = x0.w;
+            x[4] = x1.x; x[5] = x1.y; x[6] = x1.z; x[7] = x1.w;
+#pragma unroll
+            for (uint32_t e = 0; e < 8u; ++e)
+                if (!mine || k + e >= K) x[e] = 0u;
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                uint32_t h0, m0, l0, h1, m1, l1;
+                split3_any(x[e], h0, m0, l0);
+                split3_any(x[e + 1], h1, m1, l1);
+                hp[e / 2] = hi_pair(h0, h1);
+                mp[e / 2] = hi_pair(m0, m1);
+                lp[e / 2] = hi_pair(l0, l1);
+            }
+            const bf16x8 bh = __builtin_bit_cast(bf16x8, u32x4v{hp[0], hp[1], hp[2], hp[3]});
+            const bf16x8 bm = __builtin_bit_cast(bf16x8, u32x4v{mp[0], mp[1], mp[2], mp[3]});
+            const bf16x8 bl = __builtin_bit_cast(bf16x8, u32x4v{lp[0], lp[1], lp[2], lp[3]});
+#pragma unroll
+            for (int f = 0; f < FW; ++f) {
+                const bf16x8 af = codes8_to_bf16(__builtin_bit_cast(u32x2v, __builtin_amdgcn_raw_buffer_load_b64(
+                    wrs, (int)((wm + 16u * (uint32_t)f + j) * rowbytes + k), 0, 0)));
+                f32x4 p = f32x4{0.f, 0.f, 0.f, 0.f};
+                p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bh, p, 0, 0, 0);
+                p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bm, p, 0, 0, 0);
+                p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bl, p, 0, 0, 0);
+                add(f, b, p);
+            }
+        }
+    }
+}
+
+// sum += (acc + accl / 2048) * down, and both accumulators start again.
+__device__ __forceinline__ void fold(f32x4& sum, f32x4& acc, f32x4& accl, float down) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const float p = __builtin_fmaf(accl[v], 1.0f / kPartScale, acc[v]);
+        sum[v] = __builtin_fmaf(p, down, sum[v]);
+    }
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    accl = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+// The flagged steps among the `count` steps from step `first` (a fold group's,
+// at most 16): `flags` holds a byte per step of the last 32 and converting
+// wave.  Rare, and once a fold group so that the step loop carries no code or
+// registers for it.
+constexpr uint32_t kFlagSteps = 2u * kFoldCodes / 64u;
+template <int FW, int TB, typename Add>
+__device__ __forceinline__ void slow_steps(const uint8_t (&flags)[kFlagSteps][8], __amdgpu_buffer_rsrc_t wrs,
+                                           __amdgpu_buffer_rsrc_t ars, uint32_t wm, uint32_t wn, uint32_t rowbytes,
+                                           uint32_t K, uint32_t s0, uint32_t first, uint32_t count, Add&& add) {
+    const uint32_t lane = threadIdx.x & 63u, step = lane >> 1;
+    const uint32_t fl = step < count ? reinterpret_cast<const uint32_t*>(flags[(first + step) % kFlagSteps])[lane & 1u] : 0u;
+    uint64_t left = __builtin_amdgcn_ballot_w64(fl != 0u);
+#pragma unroll 1
+    while (left != 0u) {  // wave-uniform
+        const int st = __builtin_ctzll(left) >> 1;
+        left &= ~(3ull << (2 * st));
+        uint32_t groups = 0u;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)fl, 2 * st + w);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) groups |= ((v >> (8 * q)) & 1u) << (4 * w + q);
+        }
+        slow_step<FW, TB>(wrs, ars, wm, wn, rowbytes, K, (s0 + first + (uint32_t)st) * 64u, groups, add);
+    }
+}
+
 // SPLIT instances take the split launch above: whole tiles plus split tiles
 // whose K steps are shared by `parts` workgroups (a short prompt's few tiles,
 // which would leave most CUs idle, or the tiles past the last whole round of
 // a long prompt, which would leave some CUs with one tile more than others).
-// PAIR instances (two K groups) run the first P.whole tiles two per
-// workgroup, one whole tile per group, and the rest one per workgroup with
-// the K steps split between the groups.  The other instances run every tile
-// whole, with no branch on it.
-template <int FB, int NW, int BK, int PD, int KS, bool SPLIT = false, bool PAIR = false>
+// The other instances run every tile whole, with no branch on it.
+template <int FB, int NW, int BK, int PD, int KS, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __restrict__ a, MatmulProjections P,
                                                         uint32_t N, uint32_t K, uint32_t W, uint32_t mtiles,
                                                         uint32_t ntiles) {
     constexpr uint32_t BM = 32u * FB;                 // weight rows per workgroup
     constexpr uint32_t kBK = (uint32_t)BK;            // codes per K step
-    constexpr uint32_t kRowBytes = kBK * 2u;          // one LDS row: BK bf16
+    constexpr uint32_t kRowBytes = kBK * 2u;          // one LDS row: BK f16
     constexpr uint32_t kFoldSteps = kFoldCodes / kBK;
     constexpr uint32_t CPR = kBK / 16u;               // 16-code chunks per row and step
     constexpr uint32_t AST = BM * kRowBytes;          // bytes of one A stage
-    constexpr uint32_t BST = 3u * kBN * kRowBytes;    // bytes of one B stage (three parts)
+    constexpr uint32_t BST = 2u * kBN * kRowBytes;    // bytes of one B stage (two planes)
     constexpr uint32_t NT = 64u * NW;                 // threads of one K group
     constexpr uint32_t ACH = BM * CPR;                // 16-code chunks of A per step
     constexpr int AL = (int)((ACH + NT - 1u) / NT);   // A loads per thread per step
@@ -215,13 +385,15 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
     constexpr uint32_t WR = 2u;                        // waves over the rows
     constexpr int TB = (int)(4u * WR / NW);            // 16-token blocks per wave (2 or 1)
     constexpr int FW = (int)(BM / (16u * WR));         // 16-row blocks per wave
-    static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-    static_assert(BK == 64 || BK == 128, "64- or 128-code steps");
+    static_assert(NW == 8 && BK == 64, "a wave converts 8 tokens of a 64-code step, 8 activations a thread");
     static_assert(PD == 2 || PD == 4, "2 or 4 register sets of loads in flight");
     static_assert(kFoldSteps % (uint32_t)PD == 0u, "a fold group starts on register set 0 and stage 0");
     static_assert(KS == 1 || KS == 2, "K split over 1 or 2 groups of NW waves");
     // Per K group: [A0 A1 B0 B1]
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    // [step][wave]: nonzero, the wave's tokens of the step are slow_step's
+    __shared__ __attribute__((aligned(8))) uint8_t flags[KS][kFlagSteps][8];
+    __shared__ float abssum[KS][8];
 
     // XCD-aware tile order: workgroup i runs on XCD i % 8; give each XCD a
     // contiguous run of the tile sequence (tile_coords).  A split launch
@@ -229,25 +401,9 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
     // split tiles' parts, so every XCD holds its share of both and the whole
     // tiles are dispatched first.  Workgroups past the end return whole (no
     // barrier is skipped by part of one).
-    static_assert(!PAIR || (KS == 2 && !SPLIT), "pairs are the two K groups of a whole-tile launch");
     const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
     uint32_t tile, xs = 0u, np = (uint32_t)KS;  // np: runs of this tile's K steps
-    bool pair = false;                          // this group runs a tile of its own
-    if constexpr (PAIR) {
-        const uint32_t pairs = P.whole / 2u, singles = mtiles * ntiles - P.whole;
-        const uint32_t wpx = (pairs + 7u) / 8u;
-        if (slot < wpx) {
-            const uint32_t i = xcd * wpx + slot;
-            if (i >= pairs) return;
-            tile = 2u * i + __builtin_amdgcn_readfirstlane(threadIdx.x / (64u * NW));
-            np = 1u;
-            pair = true;
-        } else {
-            const uint32_t q = xcd * ((singles + 7u) / 8u) + (slot - wpx);
-            if (q >= singles) return;
-            tile = P.whole + q;
-        }
-    } else if constexpr (!SPLIT) {
+    if constexpr (!SPLIT) {
         const uint32_t total = mtiles * ntiles;
         const uint32_t lin = xcd * ((total + 7u) / 8u) + slot;
         if (lin >= total) return;
@@ -340,113 +496,80 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
             v[4 * q + 3] = gb[s][q].w;
         }
     };
-    // The three parts of the thread's FPT activations into stage s: FPT / 8
-    // 16-byte pieces per part, starting at piece bc * FPT / 8 of the row.
-    auto store_b = [&](int s, const uint32_t (&hp)[FPT / 2], const uint32_t (&mp)[FPT / 2],
-                       const uint32_t (&lp)[FPT / 2]) {
-        uint8_t* row = lds + gbase + 2u * AST + (uint32_t)s * BST + btok * kRowBytes;
-#pragma unroll
-        for (uint32_t q = 0; q < FPT / 8u; ++q) {
-            const uint32_t pc = ((bc * (FPT / 8u) + q) ^ (btok & 7u)) * 16u;
-            *reinterpret_cast<u32x4v*>(row + pc) = u32x4v{hp[4 * q], hp[4 * q + 1], hp[4 * q + 2], hp[4 * q + 3]};
-            *reinterpret_cast<u32x4v*>(row + kBN * kRowBytes + pc) =
-                u32x4v{mp[4 * q], mp[4 * q + 1], mp[4 * q + 2], mp[4 * q + 3]};
-            *reinterpret_cast<u32x4v*>(row + 2u * kBN * kRowBytes + pc) =
-                u32x4v{lp[4 * q], lp[4 * q + 1], lp[4 * q + 2], lp[4 * q + 3]};
-        }
-    };
-    // Writes the converted step into stage s and returns the thread's
-    // non-finite indicator.  Row r's 16-byte piece p sits at piece p ^ (r & 7).
-    auto convert_store = [&](int s, int st) -> float {
+    float up = 1.0f, down = 1.0f;  // the tile's power of two and its inverse
+    const float least = btok < ntok ? kPartMin : 0.0f;
+    // Writes the converted step into stage st.
+    auto convert_store = [&](int s, int st, uint32_t step) {
         uint8_t* as = lds + gbase + (uint32_t)st * AST;
 #pragma unroll
         for (int u = 0; u < AL; ++u) {
             if (!(ACH % NT == 0u || t + NT * (uint32_t)u < ACH)) continue;  // wave-uniform
             const uint32_t r = ar + (NT / CPR) * (uint32_t)u;
             u32x4v lo, hi;
-            codes16_to_bf16(ga[s][u], lo, hi);
-            const uint32_t p0 = (2u * ac) ^ (r & 7u), p1 = (2u * ac + 1u) ^ (r & 7u);
-            *reinterpret_cast<u32x4v*>(as + r * kRowBytes + p0 * 16u) = lo;
-            *reinterpret_cast<u32x4v*>(as + r * kRowBytes + p1 * 16u) = hi;
+            codes16_to_f16(ga[s][u], lo, hi);
+            *reinterpret_cast<u32x4v*>(as + r * kRowBytes + piece_offset(2u * ac, r)) = lo;
+            *reinterpret_cast<u32x4v*>(as + r * kRowBytes + piece_offset(2u * ac + 1u, r)) = hi;
         }
         uint32_t v[FPT];
         load_b(s, v);
-        // Split all FPT the fast way.  r = a - h is NaN exactly when a is not
-        // finite, so the sum of the r's tells whether this thread needs the
-        // slower split; the caller redoes the stage for a wave that does
-        // (nonfinite_fixup), outside the block the scheduler interleaves with
-        // the matrix work.
-        uint32_t hp[FPT / 2], mp[FPT / 2], lp[FPT / 2];
-        float rsum = 0.0f;
-#pragma unroll
-        for (int e = 0; e < (int)FPT; e += 2) {
-            uint32_t h0, m0_, l0, h1, m1, l1;
-            float r0, r1;
-            split3_fast(v[e], h0, m0_, l0, r0);
-            split3_fast(v[e + 1], h1, m1, l1, r1);
-            rsum += r0 + r1;
-            hp[e / 2] = hi_pair(h0, h1);
-            mp[e / 2] = hi_pair(m0_, m1);
-            lp[e / 2] = hi_pair(l0, l1);
-        }
-        store_b(st, hp, mp, lp);
-        return rsum;
+        uint8_t* row = lds + gbase + 2u * AST + (uint32_t)st * BST + btok * kRowBytes + piece_offset(bc, btok);
+        const bool bad = store_split(v, least, up, down, row, kBN * kRowBytes);
+        if (lane == 0u) flags[kg][step % kFlagSteps][wv] = bad ? 1u : 0u;
     };
 
-    // The same activation conversion for every value, Inf and NaN included.
-    auto nonfinite_fixup = [&](int s, int st) {
-        uint32_t v[FPT];
-        load_b(s, v);
-        uint32_t hp[FPT / 2], mp[FPT / 2], lp[FPT / 2];
-#pragma unroll
-        for (int e = 0; e < (int)FPT; e += 2) {
-            uint32_t h0, m0_, l0, h1, m1, l1;
-            split3_any(v[e], h0, m0_, l0);
-            split3_any(v[e + 1], h1, m1, l1);
-            hp[e / 2] = hi_pair(h0, h1);
-            mp[e / 2] = hi_pair(m0_, m1);
-            lp[e / 2] = hi_pair(l0, l1);
-        }
-        store_b(st, hp, mp, lp);
-    };
+    const uint32_t steps = (K + kBK - 1u) / kBK;
+    const bool ragged = (K % kBK) != 0u;
+    // This group's steps: [s0, s0 + gs), run xs * KS + kg of np; every group
+    // runs `iters` iterations (the same barriers), skipping the matrix work
+    // past its own steps.
+    constexpr bool kOneRun = KS == 1 && !SPLIT;  // every group takes all the steps: no skip
+    const uint32_t iters = kOneRun ? steps : (steps + np - 1u) / np;
+    const uint32_t s0 = kOneRun ? 0u : (xs * (uint32_t)KS + kg) * iters;
+    const uint32_t gs = kOneRun ? steps : (s0 < steps ? min(iters, steps - s0) : 0u);
 
-    f32x4 acc[FW][TB], sum[FW][TB];
+    f32x4 acc[FW][TB], accl[FW][TB], sum[FW][TB];
 #pragma unroll
     for (int f = 0; f < FW; ++f)
 #pragma unroll
         for (int b = 0; b < TB; ++b) {
             acc[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            accl[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
             sum[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 
-    // Matrix work of one stage: two 32-code substeps.
+    // Matrix work of one stage: two 32-code halves, lane group g taking codes
+    // 16 g + 8 h .. +7 of the step in half h (the sum's k order is free; this
+    // one is the direct kernel's, whose lanes load 16 consecutive codes).
     auto compute = [&](int s) {
         const uint8_t* as = lds + gbase + (uint32_t)s * AST;
         const uint8_t* bs = lds + gbase + 2u * AST + (uint32_t)s * BST;
 #pragma unroll
-        for (int ss = 0; ss < BK / 32; ++ss) {
-            const uint32_t piece = 4u * (uint32_t)ss + g;
-            bf16x8 af[FW], bf[TB][3];
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t piece = 2u * g + (uint32_t)h;
+            f16x8 af[FW], bf[TB][2];
 #pragma unroll
             for (int f = 0; f < FW; ++f) {
                 const uint32_t r = wm + 16u * (uint32_t)f + j;
-                af[f] = *reinterpret_cast<const bf16x8*>(as + r * kRowBytes + ((piece ^ (r & 7u)) * 16u));
+                af[f] = *reinterpret_cast<const f16x8*>(as + r * kRowBytes + piece_offset(piece, r));
             }
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
                 const uint32_t tk = wn + 16u * (uint32_t)b + j;
 #pragma unroll
-                for (int p = 0; p < 3; ++p)
-                    bf[b][p] = *reinterpret_cast<const bf16x8*>(bs + ((uint32_t)p * kBN + tk) * kRowBytes +
-                                                                ((piece ^ (tk & 7u)) * 16u));
+                for (int p = 0; p < 2; ++p)
+                    bf[b][p] = *reinterpret_cast<const f16x8*>(bs + ((uint32_t)p * kBN + tk) * kRowBytes +
+                                                               piece_offset(piece, tk));
             }
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
+            for (int f = 0; f < FW; ++f)
 #pragma unroll
-                for (int f = 0; f < FW; ++f)
+                for (int b = 0; b < TB; ++b)
+                    acc[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[f], bf[b][0], acc[f][b], 0, 0, 0);
 #pragma unroll
-                    for (int b = 0; b < TB; ++b)
-                        acc[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[f], bf[b][p], acc[f][b], 0, 0, 0);
+            for (int f = 0; f < FW; ++f)
+#pragma unroll
+                for (int b = 0; b < TB; ++b)
+                    accl[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[f], bf[b][1], accl[f][b], 0, 0, 0);
         }
     };
 
@@ -457,23 +580,24 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
     // conversion (VALU) and the matrix work are independent, so a wave
     // overlaps them.  Past the last step the conversion writes a stage nobody
     // reads and the loads fall outside the buffer resources (they return 0).
-    const uint32_t steps = (K + kBK - 1u) / kBK;
-    const bool ragged = (K % kBK) != 0u;
-    // This group's steps: [s0, s0 + gs), run xs * KS + kg of np; every group
-    // runs `iters` iterations (the same barriers), skipping the matrix work
-    // past its own steps.
-    constexpr bool kOneRun = KS == 1 && !SPLIT;  // every group takes all the steps: no skip
-    const uint32_t iters = kOneRun ? steps : (steps + np - 1u) / np;
-    const uint32_t s0 = kOneRun || pair ? 0u : (xs * (uint32_t)KS + kg) * iters;
-    const uint32_t gs = kOneRun ? steps : (s0 < steps ? min(iters, steps - s0) : 0u);
-    auto convert_checked = [&](int s, int st) {
-        const float rsum = convert_store(s, st);
-        if (__builtin_amdgcn_ballot_w64(__builtin_isnan(rsum)) != 0) nonfinite_fixup(s, st);  // uniform
-    };
 #pragma unroll
     for (int q = 0; q < PD; ++q) issue(q, (s0 + (uint32_t)q) * kBK);
     if (ragged && s0 + 1u == steps) mask_b(0, s0 * kBK);
-    convert_checked(0, 0);
+    {
+        // the power of two of this group's run, from its first step
+        uint32_t v[FPT];
+        load_b(0, v);
+        float m = 0.0f;
+#pragma unroll
+        for (int e = 0; e < (int)FPT; ++e) m += __builtin_fabsf(__uint_as_float(v[e]));
+        m = wave_sum(m);
+        if (lane == 0u) abssum[kg][wv] = m;
+        __syncthreads();
+        const int e = part_exponent(wave_sum(lane < 8u ? abssum[kg][lane] : 0.0f));
+        up = pow2f(e);
+        down = pow2f(-e);
+    }
+    convert_store(0, 0, 0u);
     issue(0, (s0 + (uint32_t)PD) * kBK);
     __syncthreads();
     // The matrix work comes first in program order: its LDS reads then need
@@ -483,7 +607,7 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
         const int nx = (q + 1) % PD;
         if (ragged && s0 + i + 2u == steps) mask_b(nx, (s0 + i + 1u) * kBK);  // uniform
         if (kOneRun || i < gs) compute(q & 1);                                 // uniform
-        convert_checked(nx, (q + 1) & 1);
+        convert_store(nx, (q + 1) & 1, i + 1u);
         issue(nx, (s0 + i + 1u + (uint32_t)PD) * kBK);
         __syncthreads();
     };
@@ -504,37 +628,33 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
         for (int f = 0; f < FW; ++f)
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
-                sum[f][b] += acc[f][b];
-                acc[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+                fold(sum[f][b], acc[f][b], accl[f][b], down);
             }
+        if (g0 < gs) slow_steps<FW, TB>(flags[kg], wrs, ars, wm, wn, rowbytes, K, s0, g0, min(gend, gs) - g0, [&](int f, int b, f32x4 v) { sum[f][b] += v; });
     }
 
     if constexpr (KS > 1) {
-        // Group 1's sums through LDS (its stages are done) into group 0's;
-        // a pair's groups each store their own tile (`pair` is
-        // workgroup-uniform, and always false outside PAIR instances).
+        // Group 1's sums through LDS (its stages are done) into group 0's.
         constexpr uint32_t E = (uint32_t)(FW * TB * 4);
         static_assert(E * NT * 4u <= 2u * AST + 2u * BST, "the reduction fits in group 0's stages");
-        if (!pair) {
-            float* red = reinterpret_cast<float*>(lds);
-            __syncthreads();
-            if (kg == 1u) {
-#pragma unroll
-                for (int f = 0; f < FW; ++f)
-#pragma unroll
-                    for (int b = 0; b < TB; ++b)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) red[((uint32_t)((f * TB + b) * 4 + v)) * NT + t] = sum[f][b][v];
-            }
-            __syncthreads();
-            if (kg != 0u) return;  // after the last barrier
+        float* red = reinterpret_cast<float*>(lds);
+        __syncthreads();
+        if (kg == 1u) {
 #pragma unroll
             for (int f = 0; f < FW; ++f)
 #pragma unroll
                 for (int b = 0; b < TB; ++b)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) sum[f][b][v] += red[((uint32_t)((f * TB + b) * 4 + v)) * NT + t];
+                    for (int v = 0; v < 4; ++v) red[((uint32_t)((f * TB + b) * 4 + v)) * NT + t] = sum[f][b][v];
         }
+        __syncthreads();
+        if (kg != 0u) return;  // after the last barrier
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) sum[f][b][v] += red[((uint32_t)((f * TB + b) * 4 + v)) * NT + t];
     }
 
     // Epilogue: lane (j, g) of block (f, b) holds features m0 + wm + 16 f +
@@ -570,48 +690,94 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
     }
 }
 
-// The one-group GEMM with each wave's weight codes loaded straight into
-// registers.  A workgroup of 8 waves owns BM = 128 FW weight rows x 64 tokens;
-// wave w owns rows 16 FW w .. +16 FW - 1 and every token of the tile, so
-// nothing it converts is shared and no code passes through LDS.  Per 64-code
-// step, lane (j, g) of 16-row block f loads codes 8g .. 8g+7 and 32+8g ..
-// 32+8g+7 of row 16 f + j (the operand's k order for the step's two 32-code
-// halves) PD steps ahead; the activations go through the same double-buffered,
-// XOR-swizzled LDS stage as matmul_q8_kernel, split into three parts once per
-// workgroup.  Matrix ops, their order and the fold points are the one-group
-// form's, so the bits are too.  SPLIT instances split every tile's K steps
-// into P.parts runs, one workgroup each (P.whole = 0): part 0 stores its
-// unscaled sums into the output, part j >= 1 into workspace block
-// (j - 1) * P.splits + tile, and split_sum_kernel adds them in part order and
-// scales them.
-template <int FW, int PD, bool SPLIT = false>
-__global__ __launch_bounds__(512) void matmul_q8_direct_kernel(const float* __restrict__ a, MatmulProjections P,
-                                                               uint32_t N, uint32_t K, uint32_t W, uint32_t mtiles,
-                                                               uint32_t ntiles) {
-    constexpr uint32_t NW = 8u, TB = 4u;
-    constexpr uint32_t BM = 16u * FW * NW;
-    constexpr uint32_t kRowBytes = 128u;              // one LDS row: 64 codes of bf16
-    constexpr uint32_t BST = 3u * kBN * kRowBytes;    // one stage: three parts of 64 tokens
-    constexpr uint32_t NT = 64u * NW;
-    constexpr uint32_t FPT = kBN * 64u / NT;          // activations per thread per step
-    constexpr int BL = (int)(FPT / 4u);
-    constexpr uint32_t TPT = NT / kBN;                // threads per token
-    constexpr uint32_t kFoldSteps = kFoldCodes / 64u;
-    static_assert(TB * 16u == kBN, "a wave covers the tile's tokens");
-    static_assert(FPT % 8u == 0u, "whole 16-byte pieces per part");
-    static_assert(kFoldSteps % (uint32_t)PD == 0u, "a fold group starts on register set 0 and stage 0");
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+// One-group workgroups of 8 waves keep the folded sums in LDS (touched once
+// per 1024 codes): the 16 FW registers they would take hold the next step's
+// operands instead.
+constexpr bool direct_sums_in_lds(int NW, int KS) { return NW == 8 && KS == 1; }
 
-    // XCD-aware order as matmul_q8_kernel: each XCD a contiguous run of the
-    // sequence (of tiles, or of split tiles' parts, a tile's parts adjacent)
+// The GEMM with each wave's weight codes loaded straight into registers.  A
+// group of NW waves owns BM = 16 FW NW weight rows x 64 tokens; wave w owns rows
+// 16 FW w .. +16 FW - 1 and every token of the tile, so nothing it converts is
+// shared and no code passes through LDS.  Per 64-code step, lane (j, g) of a
+// 16-row block loads codes 16 g .. +15 of row j, one dwordx4, two steps ahead;
+// the activations go through a ring of three LDS stages, split into their f16
+// pairs once per group.  KS = 2: two groups share the tile and split its K steps
+// in halves (their sums meet in LDS), or, as kTilePairs, each take a tile of
+// their own.  kSplitTiles splits the last P.splits tiles' K steps into P.parts
+// runs, one workgroup each: part 0 stores its unscaled sums into the output,
+// part j >= 1 into workspace block (j - 1) * P.splits + tile, and
+// split_sum_kernel adds them in part order and scales them.  Every form sums a
+// run in the same order, so whole tiles have the same bits in all of them.
+//
+// What bounds it: at 2048 x 2048 x 5632 (256 tiles of 256 rows, one per CU) the
+// step takes 1.1 us where its matrix ops alone, at the clock they leave (they
+// sustain 1.5 PFLOP/s), take 0.69; loads, split, code conversion and LDS reads
+// each add about 0.1 us to that (timing bounds with each taken out).  Two parts
+// for three, the ring, and the order below took that shape from 122 to 98 us.
+// One wave per SIMD (4 waves of 64 rows: 133), 32x32x16 matrix ops (109), waves
+// over 4 x 2 row and token halves (113) and code conversion through masks in
+// place of byte permutes (105) are all slower.
+enum : int { kWholeTiles = 0, kSplitTiles = 1, kTilePairs = 2 };
+template <int NW, int FW, int KS, int MODE>
+__global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const float* __restrict__ a,
+                                                                           MatmulProjections P, uint32_t N, uint32_t K,
+                                                                           uint32_t W, uint32_t mtiles,
+                                                                           uint32_t ntiles) {
+    constexpr int TB = 4, NS = 3, PD = 2;             // 16-token blocks per wave, LDS stages, code register sets
+    constexpr int CH = 8 / NW;                        // 8-activation chunks a thread converts per step
+    constexpr int GB = CH == 1 ? 2 : 1;               // activation register sets
+    constexpr uint32_t NT = 64u * NW;                 // threads of one K group
+    constexpr uint32_t BM = 16u * FW * NW;
+    constexpr uint32_t kRowBytes = 128u;              // one LDS row: 64 codes of f16
+    constexpr uint32_t BST = 2u * kBN * kRowBytes;    // one stage: two planes of 64 tokens
+    constexpr uint32_t kFoldSteps = kFoldCodes / 64u;
+    constexpr bool kSumsInLds = direct_sums_in_lds(NW, KS);
+    constexpr bool kOneRun = KS == 1 && MODE == kWholeTiles;  // every workgroup takes all the steps
+    static_assert(NW == 4 || NW == 8, "whole chunks per thread");
+    static_assert(KS == 1 || KS == 2, "one or two K groups");
+    static_assert(MODE != kTilePairs || KS == 2, "pairs are the two groups of a workgroup");
+    static_assert(kFoldSteps % 2u == 0u, "a fold group starts on register set 0");
+    // [stages of group 0][stages of group 1][sums]
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    // [group][step][wave]: nonzero, the wave's tokens of the step are slow_step's
+    __shared__ __attribute__((aligned(8))) uint8_t flags[KS][kFlagSteps][8];
+    __shared__ float abssum[KS][8];
+
+    // XCD-aware order: workgroup i runs on XCD i % 8; each XCD gets a
+    // contiguous run of the tile sequence (tile_coords).  A split launch gives
+    // each XCD a run of the whole tiles first and then a run of the split
+    // tiles' parts (a tile's parts adjacent).  Workgroups past the end return
+    // whole (no barrier is skipped by part of one).
+    const uint32_t kg = KS == 1 ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
     const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
-    const uint32_t parts = SPLIT ? P.parts : 1u;
-    const uint32_t units = mtiles * ntiles * parts;
-    const uint32_t lin = xcd * ((units + 7u) / 8u) + slot;
-    if (lin >= units) return;
-    const uint32_t tile = lin / parts, xs = lin - tile * parts;
+    uint32_t tile, xs = 0u, np = (uint32_t)KS;  // np: runs of this tile's K steps
+    if constexpr (MODE == kTilePairs) {
+        const uint32_t pairs = P.whole / 2u;
+        const uint32_t i = xcd * ((pairs + 7u) / 8u) + slot;
+        if (i >= pairs) return;
+        tile = 2u * i + kg;
+        np = 1u;
+    } else if constexpr (MODE == kWholeTiles) {
+        const uint32_t total = mtiles * ntiles;
+        tile = xcd * ((total + 7u) / 8u) + slot;
+        if (tile >= total) return;
+    } else {
+        const uint32_t wpx = (P.whole + 7u) / 8u;
+        if (slot < wpx) {
+            tile = xcd * wpx + slot;
+            if (tile >= P.whole) return;
+        } else {
+            const uint32_t np_all = P.splits * P.parts;
+            const uint32_t q = xcd * ((np_all + 7u) / 8u) + (slot - wpx);
+            if (q >= np_all) return;
+            tile = P.whole + q / P.parts;
+            xs = q % P.parts;
+            np = (uint32_t)KS * P.parts;
+        }
+    }
     uint32_t mt, nt;
     tile_coords(tile, mtiles, ntiles, mt, nt);
+    // the projection that owns weight-row tile mt (wave-uniform)
     const uint32_t pj = (mt >= P.mt0[1] ? 1u : 0u) + (mt >= P.mt0[2] ? 1u : 0u) + (mt >= P.mt0[3] ? 1u : 0u);
     const uint32_t* __restrict__ weight = P.weight[pj];
     const float* __restrict__ scale = P.scale[pj];
@@ -619,7 +785,7 @@ __global__ __launch_bounds__(512) void matmul_q8_direct_kernel(const float* __re
     const uint32_t M = P.M[pj];
     const uint32_t m0 = (mt - P.mt0[pj]) * BM, n0 = nt * kBN;
 
-    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t t = KS == 1 ? threadIdx.x : threadIdx.x % NT, lane = t & 63u;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const uint32_t wm = wv * (16u * FW);
     const uint32_t j = lane & 15u, g = lane >> 4;
@@ -627,196 +793,295 @@ __global__ __launch_bounds__(512) void matmul_q8_direct_kernel(const float* __re
     const uint32_t rowbytes = W * 4u;
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(weight + (size_t)m0 * W, mrows * rowbytes);
     const __amdgpu_buffer_rsrc_t ars = make_rsrc(a + (size_t)n0 * K, ntok * K * 4u);
-    const uint32_t btok = t / TPT, bc = t % TPT;
-    const int boff = (int)((btok * K + bc * FPT) * 4u);
+    // this thread converts k 8 bc .. +7 of a step for tokens btok (and btok + 8 NW)
+    const uint32_t btok = t >> 3, bc = t & 7u;
+    const int boff = (int)((btok * K + bc * 8u) * 4u), bnext = (int)(8u * NW * K * 4u);
+    uint8_t* const stages = lds + kg * (NS * BST);
+    uint8_t* const brow = stages + btok * kRowBytes + piece_offset(bc, btok);
+    f32x4* const lsum = reinterpret_cast<f32x4*>(lds + KS * NS * BST) + t;  // block i of the thread: lsum[i * NT]
 
-    // PD register sets each of codes (set i % PD: step i, loaded PD steps
-    // before its matrix work) and activations (loaded PD steps before their
-    // conversion, one step ahead of the matrix work).
-    u32x2v ga[PD][FW][2];
-    u32x4v gb[PD][BL];
+    // PD register sets of codes (set i % PD: step i) and GB of activations
+    // (step i, converted two steps before its matrix work).
+    u32x4v ga[PD][FW];
+    u32x4v gb[GB][CH][2];
+    const int aoff = (int)((wm + j) * rowbytes + 16u * g);
     auto issue_a = [&](int b, uint32_t k0) {
 #pragma unroll
         for (int f = 0; f < FW; ++f)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                ga[b][f][h] = __builtin_bit_cast(u32x2v, __builtin_amdgcn_raw_buffer_load_b64(
-                    wrs, (int)((wm + 16u * (uint32_t)f + j) * rowbytes + 8u * g + 32u * (uint32_t)h), (int)k0, 0));
+            ga[b][f] = __builtin_amdgcn_raw_buffer_load_b128(wrs, aoff + (int)(16u * (uint32_t)f * rowbytes), (int)k0, 0);
     };
     auto issue_b = [&](int b, uint32_t k0) {
 #pragma unroll
-        for (int q = 0; q < BL; ++q)
-            gb[b][q] = __builtin_amdgcn_raw_buffer_load_b128(ars, boff + 16 * q, (int)(k0 * 4u), 0);
+        for (int c = 0; c < CH; ++c)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                gb[b][c][q] = __builtin_amdgcn_raw_buffer_load_b128(ars, boff + c * bnext + 16 * q, (int)(k0 * 4u), 0);
     };
     // activations at k >= K of step k0 belong to the next token: zero
     auto mask_b = [&](int s, uint32_t k0) {
-        const uint32_t kb = k0 + bc * FPT;
+        const uint32_t kb = k0 + bc * 8u;
 #pragma unroll
-        for (int q = 0; q < BL; ++q) {
-            if (kb + 4u * (uint32_t)q >= K) gb[s][q].x = 0u;
-            if (kb + 4u * (uint32_t)q + 1u >= K) gb[s][q].y = 0u;
-            if (kb + 4u * (uint32_t)q + 2u >= K) gb[s][q].z = 0u;
-            if (kb + 4u * (uint32_t)q + 3u >= K) gb[s][q].w = 0u;
-        }
-    };
-    auto store_b = [&](int st, const uint32_t (&hp)[FPT / 2], const uint32_t (&mp)[FPT / 2],
-                       const uint32_t (&lp)[FPT / 2]) {
-        uint8_t* row = lds + (uint32_t)st * BST + btok * kRowBytes;
+        for (int c = 0; c < CH; ++c)
 #pragma unroll
-        for (uint32_t q = 0; q < FPT / 8u; ++q) {
-            const uint32_t pc = ((bc * (FPT / 8u) + q) ^ (btok & 7u)) * 16u;
-            *reinterpret_cast<u32x4v*>(row + pc) = u32x4v{hp[4 * q], hp[4 * q + 1], hp[4 * q + 2], hp[4 * q + 3]};
-            *reinterpret_cast<u32x4v*>(row + kBN * kRowBytes + pc) =
-                u32x4v{mp[4 * q], mp[4 * q + 1], mp[4 * q + 2], mp[4 * q + 3]};
-            *reinterpret_cast<u32x4v*>(row + 2u * kBN * kRowBytes + pc) =
-                u32x4v{lp[4 * q], lp[4 * q + 1], lp[4 * q + 2], lp[4 * q + 3]};
-        }
-    };
-    // The three parts of register set s into stage st; a wave holding an Inf
-    // or NaN (r = a - h is NaN exactly then) redoes its part with the split
-    // that handles every value.
-    auto convert_b = [&](int s, int st) {
-        uint32_t v[FPT];
-#pragma unroll
-        for (int q = 0; q < BL; ++q) {
-            v[4 * q] = gb[s][q].x;
-            v[4 * q + 1] = gb[s][q].y;
-            v[4 * q + 2] = gb[s][q].z;
-            v[4 * q + 3] = gb[s][q].w;
-        }
-        uint32_t hp[FPT / 2], mp[FPT / 2], lp[FPT / 2];
-        float rsum = 0.0f;
-#pragma unroll
-        for (int e = 0; e < (int)FPT; e += 2) {
-            uint32_t h0, m0_, l0, h1, m1, l1;
-            float r0, r1;
-            split3_fast(v[e], h0, m0_, l0, r0);
-            split3_fast(v[e + 1], h1, m1, l1, r1);
-            rsum += r0 + r1;
-            hp[e / 2] = hi_pair(h0, h1);
-            mp[e / 2] = hi_pair(m0_, m1);
-            lp[e / 2] = hi_pair(l0, l1);
-        }
-        store_b(st, hp, mp, lp);
-        if (__builtin_amdgcn_ballot_w64(__builtin_isnan(rsum)) != 0) {  // wave-uniform
-#pragma unroll
-            for (int e = 0; e < (int)FPT; e += 2) {
-                uint32_t h0, m0_, l0, h1, m1, l1;
-                split3_any(v[e], h0, m0_, l0);
-                split3_any(v[e + 1], h1, m1, l1);
-                hp[e / 2] = hi_pair(h0, h1);
-                mp[e / 2] = hi_pair(m0_, m1);
-                lp[e / 2] = hi_pair(l0, l1);
+            for (int q = 0; q < 2; ++q) {
+                if (kb + 4u * (uint32_t)q >= K) gb[s][c][q].x = 0u;
+                if (kb + 4u * (uint32_t)q + 1u >= K) gb[s][c][q].y = 0u;
+                if (kb + 4u * (uint32_t)q + 2u >= K) gb[s][c][q].z = 0u;
+                if (kb + 4u * (uint32_t)q + 3u >= K) gb[s][c][q].w = 0u;
             }
-            store_b(st, hp, mp, lp);
+    };
+    float up = 1.0f, down = 1.0f;  // the run's power of two and its inverse
+    constexpr uint32_t kChunkBytes = 8u * NW * kRowBytes;  // from a thread's token to its next in a stage
+    float least[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) least[c] = btok + 8u * NW * (uint32_t)c < ntok ? kPartMin : 0.0f;
+    auto take = [&](int s, int c, uint32_t (&v)[8]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            v[4 * q] = gb[s][c][q].x;
+            v[4 * q + 1] = gb[s][c][q].y;
+            v[4 * q + 2] = gb[s][c][q].z;
+            v[4 * q + 3] = gb[s][c][q].w;
+        }
+    };
+    auto flag = [&](uint32_t step, int c, bool bad) {
+        if (lane == 0u) flags[kg][step % kFlagSteps][wv + NW * (uint32_t)c] = bad ? 1u : 0u;
+    };
+    // The two planes of register set s into the stage at `stage`.
+    auto convert_b = [&](int s, uint32_t stage, uint32_t step) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            uint32_t v[8];
+            take(s, c, v);
+            flag(step, c, store_split(v, least[c], up, down, brow + stage + (uint32_t)c * kChunkBytes, kBN * kRowBytes));
         }
     };
 
-    f32x4 acc[FW][TB], sum[FW][TB];
+    f32x4 acc[FW][TB], accl[FW][TB], sum[kSumsInLds ? 1 : FW][kSumsInLds ? 1 : TB];
 #pragma unroll
     for (int f = 0; f < FW; ++f)
 #pragma unroll
-        for (uint32_t b = 0; b < TB; ++b) {
+        for (int b = 0; b < TB; ++b) {
             acc[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-            sum[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            accl[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (!kSumsInLds) sum[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 
-    // Matrix work of one step: activation parts from stage st, codes from
-    // register set q, two 32-code halves.
-    auto compute = [&](int st, int q) {
-        const uint8_t* bs = lds + (uint32_t)st * BST;
+    // Activation fragments of plane p of half h of a stage: lane group g takes
+    // codes 16 g + 8 h .. +7 of the step, so a lane's 16 consecutive codes feed
+    // both halves.
+    const uint8_t* const brd0 = stages + j * kRowBytes + piece_offset(2u * g, j);
+    const uint8_t* const brd1 = stages + j * kRowBytes + piece_offset(2u * g + 1u, j);
+    auto read_b = [&](uint32_t stage, int h, int p, f16x8 (&bf)[TB]) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t piece = 4u * (uint32_t)h + g;
-            bf16x8 af[FW], bf[TB][3];
-#pragma unroll
-            for (uint32_t b = 0; b < TB; ++b) {
-                const uint32_t tk = 16u * b + j;
-#pragma unroll
-                for (int p = 0; p < 3; ++p)
-                    bf[b][p] = *reinterpret_cast<const bf16x8*>(bs + ((uint32_t)p * kBN + tk) * kRowBytes +
-                                                                ((piece ^ (tk & 7u)) * 16u));
-            }
-#pragma unroll
-            for (int f = 0; f < FW; ++f) af[f] = codes8_to_bf16(ga[q][f][h]);
-#pragma unroll
-            for (int p = 0; p < 3; ++p)
-#pragma unroll
-                for (int f = 0; f < FW; ++f)
-#pragma unroll
-                    for (uint32_t b = 0; b < TB; ++b)
-                        acc[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[f], bf[b][p], acc[f][b], 0, 0, 0);
-        }
+        for (int b = 0; b < TB; ++b)
+            bf[b] = *reinterpret_cast<const f16x8*>((h ? brd1 : brd0) + stage + (uint32_t)p * kBN * kRowBytes +
+                                                    16u * (uint32_t)b * kRowBytes);
     };
-
-    // One barrier per step: iteration i runs step i's matrix work (stage
-    // i & 1, code set i % PD), refills that code set with step i + PD,
-    // converts step i + 1's activations into the other stage and refills
-    // their set with step i + 1 + PD.  Loads past K fall outside the buffer
-    // resources and return 0.
-    // This workgroup's steps: [s0, s0 + gs) (all of them unless SPLIT).
-    // Loads past the run read the next part's steps or past K (0), unused.
-    const uint32_t steps = (K + 63u) / 64u;
-    const bool ragged = (K % 64u) != 0u;
-    const uint32_t iters = (steps + parts - 1u) / parts;
-    const uint32_t s0 = xs * iters;
-    const uint32_t gs = s0 < steps ? min(iters, steps - s0) : 0u;
+    auto codes = [&](int q, int h, f16x8 (&af)[FW]) {
 #pragma unroll
-    for (int q = 0; q < PD; ++q) {
-        issue_a(q, 64u * (s0 + (uint32_t)q));
-        issue_b(q, 64u * (s0 + (uint32_t)q));
-    }
-    if (ragged && s0 + 1u == steps) mask_b(0, 64u * s0);
-    convert_b(0, 0);
-    issue_b(0, 64u * (s0 + (uint32_t)PD));
-    __syncthreads();
-    auto iter = [&](int q, uint32_t i) {
-        const int nx = (q + 1) % PD;
-        if (ragged && s0 + i + 2u == steps) mask_b(nx, (s0 + i + 1u) * 64u);  // uniform
-        compute(q & 1, q);
-        issue_a(q, (s0 + i + (uint32_t)PD) * 64u);
-        convert_b(nx, (q + 1) & 1);
-        issue_b(nx, (s0 + i + 1u + (uint32_t)PD) * 64u);
-        __syncthreads();
+        for (int f = 0; f < FW; ++f)
+            af[f] = h == 0 ? codes8_to_f16(ga[q][f].x, ga[q][f].y) : codes8_to_f16(ga[q][f].z, ga[q][f].w);
     };
-    for (uint32_t g0 = 0; g0 < gs; g0 += kFoldSteps) {
-        const uint32_t gend = min(g0 + kFoldSteps, gs);
-        uint32_t i = g0;
-        for (; i + (uint32_t)PD <= gend; i += (uint32_t)PD) {
-#pragma unroll
-            for (int q = 0; q < PD; ++q) iter(q, i + (uint32_t)q);
-        }
-#pragma unroll
-        for (int q = 0; q < PD - 1; ++q)
-            if (i + (uint32_t)q < gend) iter(q, i + (uint32_t)q);
+    auto matrix = [&](const f16x8 (&af)[FW], const f16x8 (&bf)[TB], f32x4 (&c)[FW][TB]) {
 #pragma unroll
         for (int f = 0; f < FW; ++f)
 #pragma unroll
-            for (uint32_t b = 0; b < TB; ++b) {
-                sum[f][b] += acc[f][b];
-                acc[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int b = 0; b < TB; ++b) c[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[f], bf[b], c[f][b], 0, 0, 0);
+    };
+    // One phase's instruction order: its LDS reads under its first matrix ops,
+    // VALU work in the shadow of each.
+    auto interleave = [&]() {
+#pragma unroll
+        for (int q = 0; q < FW * TB; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);               // a matrix op
+            if (q < TB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // an LDS read
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);               // VALU
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // This group's steps: [s0, s0 + gs), run xs * KS + kg of np; every group
+    // runs `iters` iterations (the same barriers).  Loads past the run read
+    // the next run's steps, the next token's or past the buffer (0), all
+    // unused.
+    const uint32_t steps = (K + 63u) / 64u;
+    const bool ragged = (K % 64u) != 0u;
+    const uint32_t iters = kOneRun ? steps : (steps + np - 1u) / np;
+    const uint32_t s0 = kOneRun || MODE == kTilePairs ? 0u : (xs * (uint32_t)KS + kg) * iters;
+    const uint32_t gs = kOneRun ? steps : (s0 < steps ? min(iters, steps - s0) : 0u);
+
+    issue_b(0, 64u * s0);
+    if constexpr (GB == 2) issue_b(1, 64u * (s0 + 1u));
+#pragma unroll
+    for (int q = 0; q < PD; ++q) issue_a(q, 64u * (s0 + (uint32_t)q));
+    if (ragged && s0 + 1u == steps) mask_b(0, 64u * s0);
+    {
+        // the power of two, from the run's first step
+        float m = 0.0f;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            uint32_t v[8];
+            take(0, c, v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) m += __builtin_fabsf(__uint_as_float(v[e]));
+        }
+        m = wave_sum(m);
+        if (lane == 0u) abssum[kg][wv] = m;
+        __syncthreads();
+        const int e = part_exponent(wave_sum(lane < (uint32_t)NW ? abssum[kg][lane] : 0.0f));
+        up = pow2f(e);
+        down = pow2f(-e);
+    }
+    convert_b(0, 0u, 0u);
+    if constexpr (GB == 2) issue_b(0, 64u * (s0 + 2u));
+    else issue_b(0, 64u * (s0 + 1u));
+    if (ragged && s0 + 2u == steps) mask_b(GB - 1, 64u * (s0 + 1u));
+    convert_b(GB - 1, BST, 1u);
+    if constexpr (GB == 2) issue_b(1, 64u * (s0 + 3u));
+    else issue_b(0, 64u * (s0 + 2u));
+    __syncthreads();
+
+    // One barrier per step.  Iteration i works on stage i % NS, written two
+    // iterations earlier, so the fragments of its first phase are read before
+    // the barrier that starts it: matrix work runs across the barrier.  In
+    // the shadow of the matrix ops it converts step i + 2's activations into
+    // their stage and the codes of the next half, and refills the registers
+    // those came from.  Four phases (half h, plane p), each reading the next
+    // one's fragments.
+    f16x8 bx[TB], by[TB], ax[FW], ay[FW];
+    read_b(0u, 0, 0, bx);
+    codes(0, 0, ax);
+    uint32_t cur = 0u;  // the stage of step i
+    auto iter = [&](int q, uint32_t i) {
+        constexpr uint32_t kEnd = (uint32_t)NS * BST;
+        const int s = q % GB;
+        const uint32_t next = cur + BST == kEnd ? 0u : cur + BST, after = next + BST == kEnd ? 0u : next + BST;
+        if (ragged && s0 + i + 3u == steps) mask_b(s, (s0 + i + 2u) * 64u);  // uniform
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t v[CH][8], hp[CH][4], lp[CH][4];
+        float lo[CH], hi[CH];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            take(s, c, v[c]);
+            lo[c] = kPartMax;
+            hi[c] = 0.0f;
+        }
+        auto split = [&](int e) {  // pair e of the thread's 4 CH
+            const int c = e >> 2, k = e & 3;
+            split2(__uint_as_float(v[c][2 * k]), __uint_as_float(v[c][2 * k + 1]), up, hp[c][k], lp[c][k], lo[c], hi[c]);
+        };
+        read_b(cur, 0, 1, by);
+        matrix(ax, bx, acc);
+        codes(q, 1, ay);
+        interleave();
+        issue_a(q, (s0 + i + (uint32_t)PD) * 64u);
+        read_b(cur, 1, 0, bx);
+        matrix(ax, by, accl);
+#pragma unroll
+        for (int e = 0; e < 2 * CH; ++e) split(e);
+        interleave();
+        read_b(cur, 1, 1, by);
+        matrix(ay, bx, acc);
+#pragma unroll
+        for (int e = 2 * CH; e < 4 * CH; ++e) split(e);
+        interleave();
+        uint8_t* const w = brow + after;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            *reinterpret_cast<u32x4v*>(w + (uint32_t)c * kChunkBytes) = u32x4v{hp[c][0], hp[c][1], hp[c][2], hp[c][3]};
+            *reinterpret_cast<u32x4v*>(w + (uint32_t)c * kChunkBytes + kBN * kRowBytes) =
+                u32x4v{lp[c][0], lp[c][1], lp[c][2], lp[c][3]};
+        }
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const bool bad = needs_slow(v[c], least[c], down, lo[c], hi[c]);
+            if (bad) {  // wave-uniform
+                *reinterpret_cast<u32x4v*>(w + (uint32_t)c * kChunkBytes) = u32x4v{0u, 0u, 0u, 0u};
+                *reinterpret_cast<u32x4v*>(w + (uint32_t)c * kChunkBytes + kBN * kRowBytes) = u32x4v{0u, 0u, 0u, 0u};
             }
+            flag(i + 2u, c, bad);
+        }
+        issue_b(s, (s0 + i + 2u + (uint32_t)GB) * 64u);
+        __builtin_amdgcn_sched_barrier(0);
+        read_b(next, 0, 0, bx);
+        matrix(ay, by, accl);
+        codes(q ^ 1, 0, ax);
+#pragma unroll
+        for (int f = 0; f < FW; ++f) asm volatile("" : "+v"(ax[f]));  // converted here, not past the barrier
+        interleave();
+        cur = next;
+    };
+    for (uint32_t g0 = 0; g0 < iters; g0 += kFoldSteps) {
+        const uint32_t gend = min(g0 + kFoldSteps, iters);
+        for (uint32_t i = g0; i < gend; i += 2u) {
+            if (kOneRun || i < gs) iter(0, i);  // uniform over the group
+            __syncthreads();
+            if (i + 1u < gend) {
+                if (kOneRun || i + 1u < gs) iter(1, i + 1u);
+                __syncthreads();
+            }
+        }
+        if (!kOneRun && g0 >= gs) continue;  // nothing since the last fold
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int b = 0; b < TB; ++b) {
+                if constexpr (kSumsInLds) {
+                    f32x4 v = g0 == 0u ? f32x4{0.f, 0.f, 0.f, 0.f} : lsum[(uint32_t)(f * TB + b) * NT];
+                    fold(v, acc[f][b], accl[f][b], down);
+                    lsum[(uint32_t)(f * TB + b) * NT] = v;
+                } else {
+                    fold(sum[f][b], acc[f][b], accl[f][b], down);
+                }
+            }
+        slow_steps<FW, TB>(flags[kg], wrs, ars, wm, 0u, rowbytes, K, s0, g0, min(gend, gs) - g0, [&](int f, int b, f32x4 v) {
+            if constexpr (kSumsInLds) lsum[(uint32_t)(f * TB + b) * NT] += v;
+            else sum[f][b] += v;
+        });
+    }
+
+    if constexpr (KS > 1 && MODE != kTilePairs) {
+        // group 1's sums through LDS (every stage is done with) into group 0's
+        static_assert(!kSumsInLds && (uint32_t)(FW * TB) * NT * 16u <= NS * BST, "the sums fit in group 0's stages");
+        f32x4* const red = reinterpret_cast<f32x4*>(lds) + t;
+        if (kg == 1u) {
+#pragma unroll
+            for (int f = 0; f < FW; ++f)
+#pragma unroll
+                for (int b = 0; b < TB; ++b) red[(uint32_t)(f * TB + b) * NT] = sum[f][b];
+        }
+        __syncthreads();
+        if (kg != 0u) return;  // after the last barrier
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int b = 0; b < TB; ++b) sum[f][b] += red[(uint32_t)(f * TB + b) * NT];
     }
 
     // lane (j, g) of block (f, b): rows m0 + wm + 16 f + 4 g .. +3 of token
     // n0 + 16 b + j.  A split tile's parts store unscaled sums: part 0 into
     // the output, part xs into its workspace block ([token][row] in the tile).
-    const __amdgpu_buffer_rsrc_t srs = make_rsrc(scale + m0, SPLIT ? 0u : mrows * 4u);
-    float* const blk = SPLIT && xs > 0u ? P.part + ((size_t)(xs - 1u) * P.splits + tile) * (size_t)(BM * kBN) : nullptr;
+    const bool split = MODE == kSplitTiles && tile >= P.whole;
+    const __amdgpu_buffer_rsrc_t srs = make_rsrc(scale + m0, split ? 0u : mrows * 4u);
+    float* const blk = MODE == kSplitTiles && xs > 0u
+        ? P.part + ((size_t)(xs - 1u) * P.splits + (tile - P.whole)) * (size_t)(BM * kBN) : nullptr;
 #pragma unroll
     for (int f = 0; f < FW; ++f) {
         const uint32_t fm = wm + 16u * (uint32_t)f + 4u * g;
-        const u32x4v sv = SPLIT ? u32x4v{0x3f800000u, 0x3f800000u, 0x3f800000u, 0x3f800000u}  // 1.0f
+        const u32x4v sv = split ? u32x4v{0x3f800000u, 0x3f800000u, 0x3f800000u, 0x3f800000u}  // 1.0f
                                 : __builtin_amdgcn_raw_buffer_load_b128(srs, (int)(fm * 4u), 0, 0);
 #pragma unroll
-        for (uint32_t b = 0; b < TB; ++b) {
-            const uint32_t tok = 16u * b + j;
+        for (int b = 0; b < TB; ++b) {
+            const uint32_t tok = 16u * (uint32_t)b + j;
             if (tok >= ntok) continue;
             f32x4 y;
-            y[0] = sum[f][b][0] * __uint_as_float(sv.x);
-            y[1] = sum[f][b][1] * __uint_as_float(sv.y);
-            y[2] = sum[f][b][2] * __uint_as_float(sv.z);
-            y[3] = sum[f][b][3] * __uint_as_float(sv.w);
+            if constexpr (kSumsInLds) y = gs ? lsum[(uint32_t)(f * TB + b) * NT] : f32x4{0.f, 0.f, 0.f, 0.f};
+            else y = sum[f][b];
+            y[0] *= __uint_as_float(sv.x);
+            y[1] *= __uint_as_float(sv.y);
+            y[2] *= __uint_as_float(sv.z);
+            y[3] *= __uint_as_float(sv.w);
             float* o = blk ? blk + tok * BM + fm : out + (size_t)(n0 + tok) * M + m0 + fm;
             if (fm + 3u < mrows) {
                 *reinterpret_cast<f32x4_a4*>(o) = f32x4_a4{y[0], y[1], y[2], y[3]};
@@ -895,32 +1160,33 @@ uint32_t fill_projections(const MatmulProjection* p, uint32_t count, uint32_t BM
     return mtiles;
 }
 
-// One launch of matmul_q8_direct_kernel (128 FW-row tiles, PD register sets)
-// over `count` projections of the same activations.
-// With parts > 1 (a SPLIT instance) every tile's K steps split into `parts`
-// runs, the workspace `part` holding (parts - 1) x tiles blocks of 128 FW x
-// kBN floats, and split_sum_kernel sums them in a second launch.
-template <int FW, int PD, bool SPLIT = false>
+// One launch of matmul_q8_direct_kernel over `count` projections of the same
+// activations.  kSplitTiles: the last `splits` tiles of the sequence have their K
+// steps split into `parts` runs, the workspace `part` holding (parts - 1) x splits
+// blocks of BM x kBN floats, and split_sum_kernel sums them in a second launch.
+template <int NW, int FW, int KS = 1, int MODE = kWholeTiles>
 hipError_t launch_direct(const float* a, const MatmulProjection* p, uint32_t count, uint32_t N, uint32_t K,
-                         hipStream_t stream, float* part = nullptr, uint32_t parts = 1) {
-    constexpr uint32_t BM = 128u * FW;
+                         hipStream_t stream, float* part = nullptr, uint32_t splits = 0, uint32_t parts = 1) {
+    constexpr uint32_t BM = 16u * FW * NW;
     const uint32_t W = (uint32_t)(((uint64_t)K + 3) / 4);
     MatmulProjections P = {};
     const uint32_t mtiles = fill_projections(p, count, BM, P);
     const uint32_t ntiles = (N + kBN - 1u) / kBN;
     const uint32_t tiles = mtiles * ntiles;
     P.part = part;
-    P.whole = 0;
-    P.splits = SPLIT ? tiles : 0u;
-    P.parts = SPLIT ? parts : 1u;
-    const uint32_t grid = ((tiles * P.parts + 7u) / 8u) * 8u;
-    const size_t lds = 2u * 3u * kBN * 128u;
-    hipLaunchKernelGGL((matmul_q8_direct_kernel<FW, PD, SPLIT>), dim3(grid), dim3(512), lds, stream, a, P, N, K, W,
-                       mtiles, ntiles);
-    if constexpr (SPLIT) {
+    P.whole = tiles - splits;
+    P.splits = splits;
+    P.parts = parts;
+    uint32_t grid = ((tiles + 7u) / 8u) * 8u;
+    if constexpr (MODE == kSplitTiles) grid = 8u * ((P.whole + 7u) / 8u + (splits * parts + 7u) / 8u);
+    if constexpr (MODE == kTilePairs) grid = 8u * ((tiles / 2u + 7u) / 8u);
+    const size_t lds = KS * 3u * 2u * kBN * 128u + (direct_sums_in_lds(NW, KS) ? BM * kBN * 4u : 0u);
+    hipLaunchKernelGGL((matmul_q8_direct_kernel<NW, FW, KS, MODE>), dim3(grid), dim3(64 * NW * KS), lds, stream, a, P, N,
+                       K, W, mtiles, ntiles);
+    if constexpr (MODE == kSplitTiles) {
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
-        hipLaunchKernelGGL(split_sum_kernel<BM>, dim3(tiles, BM / 16u), dim3(256), 0, stream, P, N, mtiles);
+        hipLaunchKernelGGL(split_sum_kernel<BM>, dim3(splits, BM / 16u), dim3(256), 0, stream, P, N, mtiles);
     }
     return hipGetLastError();
 }
@@ -930,7 +1196,7 @@ hipError_t launch_direct(const float* a, const MatmulProjection* p, uint32_t cou
 // their K steps split into `parts` runs, with the workspace `part` holding
 // (parts - 1) x splits blocks of BM x kBN floats, and a second launch sums
 // them.
-template <int FB, int NW, int BK, int PD, int KS = 1, bool SPLIT = false, bool PAIR = false>
+template <int FB, int NW, int BK, int PD, int KS = 1, bool SPLIT = false>
 hipError_t launch_fb(const float* a, const MatmulProjection* p, uint32_t count, uint32_t N, uint32_t K,
                      hipStream_t stream, float* part = nullptr, uint32_t splits = 0, uint32_t parts = 1) {
     constexpr uint32_t kRowBytes = (uint32_t)BK * 2u;
@@ -946,13 +1212,8 @@ hipError_t launch_fb(const float* a, const MatmulProjection* p, uint32_t count, 
     P.parts = parts;
     uint32_t grid = ((tiles + 7u) / 8u) * 8u;
     if constexpr (SPLIT) grid = 8u * ((P.whole + 7u) / 8u + (splits * parts + 7u) / 8u);
-    if constexpr (PAIR) {  // `splits` here: the tiles run in pairs (even)
-        P.whole = splits;
-        P.splits = 0;
-        grid = 8u * ((splits / 2u + 7u) / 8u + (tiles - splits + 7u) / 8u);
-    }
-    const size_t lds = (size_t)KS * (2u * BM * kRowBytes + 2u * 3u * kBN * kRowBytes);
-    hipLaunchKernelGGL((matmul_q8_kernel<FB, NW, BK, PD, KS, SPLIT, PAIR>), dim3(grid), dim3(64 * NW * KS), lds, stream, a,
+    const size_t lds = (size_t)KS * (2u * BM * kRowBytes + 2u * 2u * kBN * kRowBytes);
+    hipLaunchKernelGGL((matmul_q8_kernel<FB, NW, BK, PD, KS, SPLIT>), dim3(grid), dim3(64 * NW * KS), lds, stream, a,
                        P, N, K, W, mtiles, ntiles);
     if constexpr (SPLIT) {
         const hipError_t err = hipGetLastError();
@@ -1004,24 +1265,16 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         }
         return hipSuccess;
     }
-    // 128 weight rows per workgroup when that still gives every CU a tile,
-    // otherwise 64 rows with four register sets of loads in flight (6-16 %
-    // faster than two at 64-row tiles from K = 2048 to 11008, and faster than
-    // 128-code steps; with 128-row tiles the extra registers cost more than
-    // they save).  When the tiles fit in one workgroup per CU, two groups of
-    // 8 waves split each tile's K steps (half the serial chain; 8-15 %
-    // faster, 512 x 4096 x 11008 in 172 us against 197); with more tiles the
-    // smaller one-group workgroups (two per CU) win.  Short prompts whose
-    // 32-row tiles still fit one workgroup per CU take those: each tile's
-    // steps move less through LDS and twice the CUs work (64 tokens, 2048 x
-    // 2048: 18.5 -> 16.2 us; 2048 x 5632: 44.7 -> 38.3 us; the same sums in
-    // the same order, so the same bits).  Projections in one launch count
-    // their tiles together.  Launches whose tiles take one K group and no
-    // split run on matmul_q8_direct_kernel (D256, D256.PD2, D128 below).
+    // The direct kernel where its tiles give (most of) the CUs one each, alone
+    // or split through the workspace (D256, D128 and the FB4 forms below); short
+    // prompts' smaller tiles, 64 or 32 rows, through LDS with two groups of 8
+    // waves that split each tile's K steps.  Projections in one launch count
+    // their tiles together.
     const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
     const uint64_t ntiles = (N + kBN - 1u) / kBN;
-    uint64_t t8 = 0, t4 = 0, t2 = 0, t1 = 0;
+    uint64_t t12 = 0, t8 = 0, t4 = 0, t2 = 0, t1 = 0;
     for (uint32_t i = 0; i < n; ++i) {
+        t12 += (uint64_t)((p[i].M + 383u) / 384u) * ntiles;
         t8 += (uint64_t)((p[i].M + 255u) / 256u) * ntiles;
         t4 += (uint64_t)((p[i].M + 127u) / 128u) * ntiles;
         t2 += (uint64_t)((p[i].M + 63u) / 64u) * ntiles;
@@ -1029,24 +1282,27 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     }
     const uint32_t steps = (uint32_t)(((uint64_t)K + 63u) / 64u);
     const char* kname = n > 1 ? "matmul_q8.multi" : "matmul_q8";
-    // 256-row tiles on the direct kernel (8 waves of 32 rows x 64 tokens, codes
-    // straight into registers, four sets in flight), one workgroup per CU,
-    // when those tiles make whole rounds of the CUs or at least 2.75 of them.
-    // The sums and their order are the one-group 128-row form's, so are the
-    // bits.  Same process, us, against 256-row tiles through LDS (4 of 8 waves
-    // over the rows, 64 x 32 each), which had replaced the 128-row one-group
-    // form (1024 x 4096 x 4096 129 -> 113): 1024 x 4096 x 4096 108 -> 98,
-    // 2048 x 2048 x 2048 60 -> 56, 2048 x 6144 x 2048 164 -> 155, 2048 x
-    // 11264 x 2048 304 -> 289, 2048 x 2048 x 5632 145 -> 134, 2048 x 4096 x
-    // 11008 502 -> 475, 4096 x 4096 x 4096 391 -> 363.
-    if (t8 >= cus && (t8 % cus == 0 || 4u * t8 >= 11u * (uint64_t)cus)) {
+    // One workgroup of 8 waves per CU on the direct kernel, each wave 32 or 48
+    // rows x 64 tokens.  The larger tile needs 1.26 times the smaller one's time
+    // for 1.5 times its work (the activations' LDS reads, split and barriers per
+    // step are the same), so the dispatch takes the one whose rounds of the CUs
+    // cost less.  Same process, us, 256 / 384 rows: 512 x 11264 x 2048 (352 / 240
+    // tiles) 65 / 50, 2048 x 11264 x 2048 (1408 / 960) 228 / 198, 512 x 6144 x
+    // 2048 (192 / 128) 35.1 / 43.8, 2048 x 2048 x 5632 (256 / 192) 98.8 / 111.
+    // 128-row tiles, two workgroups of 4 waves per CU, take 0.69 of a 256-row
+    // round per tile and CU (704 tiles 67 us): they are left the launches whose
+    // 256-row tiles would leave a round mostly empty.  The sums and their order
+    // are the same in all three, so are the bits.
+    const uint64_t r8 = (t8 + cus - 1u) / cus, r12 = (t12 + cus - 1u) / cus;
+    const bool rows384 = t4 > 2ull * cus && 126u * r12 < 100u * r8;
+    if (!rows384 && t8 >= cus && 100u * r8 * cus < 69u * t4) {
         set_variant(variant, kname, "D256", 8, 256, 0, (int)kBN, (uint32_t)((t8 + 7u) / 8u * 8u));
-        return launch_direct<2, 4>(a, p, n, N, K, stream);
+        return launch_direct<8, 2>(a, p, n, N, K, stream);
     }
     if (t4 >= cus) {
         if (t4 == cus) {
-            set_variant(variant, kname, "FB4.ksplit2", 16, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
-            return launch_fb<4, 8, 64, 2, 2>(a, p, n, N, K, stream);
+            set_variant(variant, kname, "FB4.ksplit2", 8, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
+            return launch_direct<4, 2, 2>(a, p, n, N, K, stream);
         }
         // Two workgroups per CU.  Between cus and 2 x cus tiles, some CUs
         // take two tiles and the others one (384 tiles: half and half).  With
@@ -1071,11 +1327,11 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         // forms (31.6 -> 45.0).
         if (S > 0 && 3u * t8 >= 2u * (uint64_t)cus) {
             set_variant(variant, kname, "D256.PD2", 8, 256, 0, (int)kBN, (uint32_t)((t8 + 7u) / 8u * 8u));
-            return launch_direct<2, 2>(a, p, n, N, K, stream);
+            return launch_direct<8, 2>(a, p, n, N, K, stream);
         }
         if (workspace && S > 0 && steps >= 8u && S * blk <= workspace_bytes) {
-            set_variant(variant, kname, "FB4.balance2", 8, 128, 0, (int)kBN, (uint32_t)(t4 + S));
-            return launch_fb<4, 8, 64, 2, 1, true>(a, p, n, N, K, stream, workspace, (uint32_t)S, 2u);
+            set_variant(variant, kname, "FB4.balance2", 4, 128, 0, (int)kBN, (uint32_t)(t4 + S));
+            return launch_direct<4, 2, 1, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)S, 2u);
         }
         // Long rows whose tiles make two or more whole rounds of two per CU:
         // one workgroup of 16 waves per two consecutive tiles of the sequence,
@@ -1088,15 +1344,17 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         // at K = 2048 no gain.  The same sums in the same order as the
         // one-group form.
         if (K >= 4096u && t4 >= 4ull * cus && t4 % (2ull * cus) == 0) {
-            set_variant(variant, kname, "FB4.pairs", 16, 128, 0, (int)kBN, (uint32_t)((t4 / 2u + 7u) / 8u * 8u));
-            return launch_fb<4, 8, 64, 2, 2, false, true>(a, p, n, N, K, stream, nullptr, (uint32_t)t4, 1u);
+            set_variant(variant, kname, "FB4.pairs", 8, 128, 0, (int)kBN, (uint32_t)((t4 / 2u + 7u) / 8u * 8u));
+            return launch_direct<4, 2, 2, kTilePairs>(a, p, n, N, K, stream);
         }
-        // Otherwise the 128-row tiles on the direct kernel, two workgroups per
-        // CU.  Same process, us, against the one-group form through LDS: 768
-        // tokens q, k, v 86.1 -> 82.9, 1024 tokens 94.8 -> 92.4, 512 x 11008 x
-        // 4096 166.6 -> 161.7.
-        set_variant(variant, kname, "D128", 8, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
-        return launch_direct<1, 2>(a, p, n, N, K, stream);
+        // Otherwise whole 128-row units: three per workgroup by the rule above,
+        // or one per workgroup of 4 waves, two workgroups per CU.
+        if (rows384) {
+            set_variant(variant, kname, "D128", 8, 384, 0, (int)kBN, (uint32_t)((t12 + 7u) / 8u * 8u));
+            return launch_direct<8, 3>(a, p, n, N, K, stream);
+        }
+        set_variant(variant, kname, "D128", 4, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
+        return launch_direct<4, 2>(a, p, n, N, K, stream);
     }
     // With a workspace, 256-row tiles on the direct kernel with every tile's
     // K steps split into 4 or 8 parts, one workgroup each, when that fills
@@ -1112,7 +1370,7 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
             (xs - 1u) * t8 * blk <= workspace_bytes) {
             set_variant(variant, kname, xs == 4u ? "D256.split4" : "D256.split8", 8, 256, 0, (int)kBN,
                         (uint32_t)(t8 * xs));
-            return launch_direct<2, 2, true>(a, p, n, N, K, stream, workspace, xs);
+            return launch_direct<8, 2, 1, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)t8, xs);
         }
     }
     // 128-row tiles that fill most of the CUs, one per CU with two K groups,
@@ -1122,8 +1380,8 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // 256 tokens q, k, v (192 tiles) 38.9 -> 33.2; with 128 tiles (half the
     // CUs) they lose (512 tokens o: 29.6 -> 31.4, one box and process).
     if (5u * t4 >= 3u * cus) {
-        set_variant(variant, kname, "FB4.ksplit2", 16, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
-        return launch_fb<4, 8, 64, 2, 2>(a, p, n, N, K, stream);
+        set_variant(variant, kname, "FB4.ksplit2", 8, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
+        return launch_direct<4, 2, 2>(a, p, n, N, K, stream);
     }
     // With a workspace, 128-row tiles whose K steps split in 2 or 4 fill
     // (nearly) every CU, as long as each K group keeps at least 10 steps
@@ -1137,9 +1395,9 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         const size_t blk = (size_t)128u * kBN * 4u;
         if (workspace && t4 * xs <= cus && 8u * t4 * xs > 7u * cus && steps >= 20u * xs &&
             (xs - 1u) * t4 * blk <= workspace_bytes) {
-            set_variant(variant, kname, xs == 4u ? "FB4.ksplit2.wgsplit4" : "FB4.ksplit2.wgsplit2", 16, 128, 0, (int)kBN,
+            set_variant(variant, kname, xs == 4u ? "FB4.ksplit2.wgsplit4" : "FB4.ksplit2.wgsplit2", 8, 128, 0, (int)kBN,
                         (uint32_t)(t4 * xs));
-            return launch_fb<4, 8, 64, 2, 2, true>(a, p, n, N, K, stream, workspace, (uint32_t)t4, xs);
+            return launch_direct<4, 2, 2, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)t4, xs);
         }
     }
     if (t1 <= cus) {
