@@ -331,6 +331,29 @@ def test_batched_decoder_sized_weights(N, K, M, kernel):
         assert_matvec(ys[m], w, s, xs[m], N, K)
 
 
+@pytest.mark.parametrize("N,K,M", [
+    (4097, 2049, 5), (5000, 2500, 8), (4100, 3071, 16), (4096, 3072, 6), (17, 3072, 1500),  # three steps per wave
+    (10241, 2100, 3), (10240, 3000, 4),
+    (4099, 3073, 5), (4200, 4095, 8), (5632, 4096, 13), (4096, 4096, 12), (1100, 4000, 35),  # four
+    (16384, 3500, 3),
+    (4096, 1000, 5), (5632, 1024, 7), (4097, 1025, 5), (8191, 2048, 6), (16385, 2047, 3), (16384, 900, 4),
+])
+def test_batched_ksplit_steps(N, K, M):
+    """The k-split kernel at the edges of its steps per wave, of its vector
+    packings and of the dispatch's lines: ragged rows, K and vector groups,
+    full-range codes, an infinity and a NaN among the vectors."""
+    rng = np.random.default_rng(N + 3 * K + M)
+    w = random_weights(rng, N, K, full_range=True)
+    s = rng.uniform(0.001, 0.05, N).astype(np.float32)
+    xs = rng.standard_normal((M, K)).astype(np.float32)
+    xs[0, K - 1] = np.inf
+    xs[M - 1, 5] = np.nan
+    ys = wxo_q8.matvecQ8Batched(weight=w, scale=s, vectors=xs, N=N, K=K, M=M)
+    assert wxo_q8.last_variant().split(" ")[0] == "matvec_q8_ksplit", wxo_q8.last_variant()
+    for m in (range(M) if M < 64 else [0, 1, 15, 16, 31, M // 2, M - 2, M - 1]):
+        assert_matvec(ys[m], w, s, xs[m], N, K)
+
+
 @pytest.mark.parametrize("M,K", [(5, 1030), (8, 64), (12, 2048), (13, 4099), (16, 1024), (17, 1500), (32, 520),
                                  (6, 3000), (14, 1000), (16, 768), (13, 1536), (20, 1024), (33, 1000),
                                  (5, 769), (5, 2047), (6, 897), (7, 1024), (8, 1025), (8, 2048), (9, 1100),

@@ -498,6 +498,19 @@ __device__ __forceinline__ void split_x_parts(float xe, uint32_t& hb, uint32_t& 
     }
 }
 
+// The same for two values that are finite or NaN, packed (first in the low half);
+// most collects the largest |x|.  A NaN leaves m NaN, so its column's sums are.
+__device__ __forceinline__ void split3_pair(uint32_t a, uint32_t b, uint32_t& h, uint32_t& m, uint32_t& l, float& most) {
+    const float ra = __uint_as_float(a) - __uint_as_float(a & 0xffff0000u);
+    const float rb = __uint_as_float(b) - __uint_as_float(b & 0xffff0000u);
+    const float la = ra - __uint_as_float(__float_as_uint(ra) & 0xffff0000u);
+    const float lb = rb - __uint_as_float(__float_as_uint(rb) & 0xffff0000u);
+    h = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    m = __builtin_amdgcn_perm(__float_as_uint(rb), __float_as_uint(ra), 0x07060302u);
+    l = __builtin_amdgcn_perm(__float_as_uint(lb), __float_as_uint(la), 0x07060302u);
+    most = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(__uint_as_float(a)), __builtin_fabsf(__uint_as_float(b))), most);
+}
+
 // Splits the four vector entries k .. k+3 of column m (v; entries past K count
 // as 0) into bf16 parts h, m, l and stores them in B-operand order:
 // [part][32-code block][lane group][column] x 8 bf16.  Code k sits in block
@@ -890,7 +903,7 @@ __global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Batched, K up to 2048: the row's codes split across the workgroup's 8 waves
+// Batched, K up to 4096: the row's codes split across the workgroup's 8 waves
 // (wave w owns codes 128 (w + 8 s) .. +127 of step s = 0 .. SW - 1), so each
 // wave's share of the x parts fits in its VGPRs (12 bf16x8 registers per
 // step and B operand set) and is never read again from LDS; only the weight
@@ -922,6 +935,11 @@ __global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
 //      sums move to the h lanes with a DPP row rotation
 //   3: up to 5 vectors: h | m | l in one operand (1 op)
 // A column's parts are summed as h + (m + l), the order PACK 1 uses too.
+//
+// Three and four steps per wave (K to 3072 and 4096) fit since the x parts are
+// made one 64-code run at a time (at most 48 registers of parts per step of 16
+// vectors): N = 11008, K = 4096, 16 vectors 37.9 -> 15.0 us against the VALU
+// kernel's two passes, 8 vectors 22.2 -> 13.2; N = 32000 98 -> 27.5.
 //
 // Measured on MI355X (rotating weight copies), against the matrix-core
 // kernels above: LM head N = 151936, K = 1024: 16 vectors 33-34 us (45-47),
@@ -1069,18 +1087,30 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
 
     // This wave's x parts: lane (j, g), step s, block (u, e) holds codes
     // c0 + 64u + 16g + 8e + 0..7 of vector m0 + vj: the k order in which the
-    // lane reads its A operand (piece 4u + g of row j).  Entries past K are 0
-    // (they would belong to the next vector).
+    // lane reads its A operand (piece 4u + g of row j).
+    // x comes in whole 256-byte runs (16 lanes per vector: a lane per vector
+    // would cost the address unit a cycle per lane) and reaches its lanes through
+    // LDS, 64 codes of every vector at a time, in the four 1 KiB slots that this
+    // wave's partial sums use later.  A vector's 16-byte pieces are swizzled so
+    // that the 16 lanes an LDS read serves at a time (0-3, 12-15, 20-23, 24-27, ..)
+    // find theirs in different banks.  The parts are split without a branch per
+    // value; a wave with an infinity splits again.  With a load per lane and
+    // vector and the per-value branches the prologue took about 6 us at K = 1024
+    // and 9 at K = 2048 of every call.
+    constexpr int NI = PACK == 1 ? 4 : 2;  // 4 vectors per load instruction
     const __amdgpu_buffer_rsrc_t xrs = make_rsrc(x + (size_t)m0 * K, MC * K * 4u);
-    u32x4v xl[SW][2][4];
+    const auto swz = [](uint32_t v) { return (v & 3u) | (((0u - (v >> 2)) & 3u) << 2); };
+    uint8_t* const xst = reinterpret_cast<uint8_t*>(red) + wv * 1024u;  // slot i: xst + i * 8192
+    u32x4v xl[SW][2][NI];
 #pragma unroll
     for (int s = 0; s < SW; ++s)
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t c = 128u * (wv + kKsWaves * (uint32_t)s) + 64u * (uint32_t)u + 16u * g + 4u * (uint32_t)q;
-                const int off = (col_ok && c < K) ? (int)((vj * K + c) * 4u) : (int)0x7ffffff0;
+            for (int q = 0; q < NI; ++q) {
+                const uint32_t v = 4u * (uint32_t)q + lane / 16u;
+                const uint32_t c = 128u * (wv + kKsWaves * (uint32_t)s) + 64u * (uint32_t)u + 4u * (lane % 16u);
+                const int off = (v < MC && c < K) ? (int)((v * K + c) * 4u) : (int)0x7ffffff0;
                 xl[s][u][q] = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0);
             }
     u32x4v sbuf[D];
@@ -1091,23 +1121,50 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
 #pragma unroll
     for (int s = 0; s < SW; ++s)
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int q = 0; q < NI; ++q) {
+                const uint32_t v = 4u * (uint32_t)q + lane / 16u;
+                *reinterpret_cast<u32x4v*>(xst + (uint32_t)q * 8192u + (lane / 16u) * 256u + ((lane % 16u) ^ swz(v)) * 16u) =
+                    xl[s][u][q];
+            }
+            uint32_t xv[16];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const u32x4v t = *reinterpret_cast<const u32x4v*>(
+                    xst + (vj >> 2) * 8192u + (vj & 3u) * 256u + ((4u * g + (uint32_t)q) ^ swz(vj)) * 16u);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xv[4 * q + e] = t[e];
+            }
+            const uint32_t c0 = 128u * (wv + kKsWaves * (uint32_t)s) + 64u * (uint32_t)u;
+            if (c0 + 64u > K) {  // wave-uniform: entries past K belong to the next vector
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (c0 + 16u * g + (uint32_t)i >= K) xv[i] = 0u;
+            }
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 u32x4v pv[3];
+                float most = 0.0f;
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
-                    uint32_t hw[2], mw[2], lw[2];
+                    uint32_t h, m, l;
+                    split3_pair(xv[8 * e + 2 * p], xv[8 * e + 2 * p + 1], h, m, l, most);
+                    pv[0][p] = h;
+                    pv[1][p] = m;
+                    pv[2][p] = l;
+                }
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(__float_as_uint(most) == 0x7f800000u) != 0, 0)) {
 #pragma unroll
-                    for (int z = 0; z < 2; ++z) {
-                        const int idx = 8 * e + 2 * p + z;
-                        const uint32_t c = 128u * (wv + kKsWaves * (uint32_t)s) + 64u * (uint32_t)u + 16u * g + (uint32_t)idx;
-                        const float xe = c < K ? __uint_as_float(xl[s][u][idx / 4][idx % 4]) : 0.0f;
-                        split_x_parts(xe, hw[z], mw[z], lw[z]);
+                    for (int p = 0; p < 4; ++p) {
+                        uint32_t hw[2], mw[2], lw[2];
+#pragma unroll
+                        for (int z = 0; z < 2; ++z)
+                            split_x_parts(__uint_as_float(xv[8 * e + 2 * p + z]), hw[z], mw[z], lw[z]);
+                        pv[0][p] = (hw[0] >> 16) | hw[1];
+                        pv[1][p] = (mw[0] >> 16) | mw[1];
+                        pv[2][p] = (lw[0] >> 16) | lw[1];
                     }
-                    pv[0][p] = (hw[0] >> 16) | hw[1];
-                    pv[1][p] = (mw[0] >> 16) | mw[1];
-                    pv[2][p] = (lw[0] >> 16) | lw[1];
                 }
                 const u32x4v zero = {0u, 0u, 0u, 0u};
                 if constexpr (PACK == 1) {
@@ -1120,6 +1177,10 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
                     bx[s][u][e][0] = __builtin_bit_cast(bf16x8, sel == 0u ? pv[0] : sel == 1u ? pv[1] : pv[2]);
                 }
             }
+            // one 64-code run at a time (left to itself the compiler converts
+            // them side by side and spills)
+            __builtin_amdgcn_sched_barrier(0);
+        }
 
     f32x4 acc[NB], pacc[NB];
 #pragma unroll
@@ -1205,10 +1266,8 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
         for (int r = 1; r < D; ++r) n += 2 + (!STW && ((par + r) % SW) == SW - 1 ? 1 : 0);
         return n;
     };
-    constexpr int kA0 = after(0), kA1 = SW > 1 ? after(1) : after(0);
-    static_assert(kA0 < 64 && kA1 < 64, "vmcnt holds at most 63");
-    constexpr int kVmWait0 = 0x0f70 | (kA0 & 15) | ((kA0 >> 4) << 14);
-    constexpr int kVmWait1 = 0x0f70 | (kA1 & 15) | ((kA1 >> 4) << 14);
+    constexpr int kA0 = after(0), kA1 = after(1 % SW), kA2 = after(2 % SW), kA3 = after(3 % SW);
+    static_assert(SW <= 4 && kA0 < 16 && kA1 < 16 && kA2 < 16 && kA3 < 16, "one wait per position, its count in 4 bits");
     uint32_t pending = ~0u;  // a group whose partials are written but not yet summed (wave-uniform)
     for (uint32_t i = 0; i < total; i += (uint32_t)PER) {
 #pragma unroll
@@ -1228,8 +1287,10 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
             __builtin_amdgcn_sched_barrier(0);
             issue(i + (uint32_t)(q + D - 1), sbuf[(q + D - 1) % D]);
             __builtin_amdgcn_sched_barrier(0);
-            if (q % SW == 0) __builtin_amdgcn_s_waitcnt(kVmWait0);
-            else __builtin_amdgcn_s_waitcnt(kVmWait1);
+            if (q % SW == 0) __builtin_amdgcn_s_waitcnt(0x0f70 | kA0);
+            else if (q % SW == 1) __builtin_amdgcn_s_waitcnt(0x0f70 | kA1);
+            else if (q % SW == 2) __builtin_amdgcn_s_waitcnt(0x0f70 | kA2);
+            else __builtin_amdgcn_s_waitcnt(0x0f70 | kA3);
             __builtin_amdgcn_sched_barrier(0);
             compute(i + (uint32_t)q, q % SW);
             // the deferred write stays behind this pair's A reads (the wait above relies on it)
@@ -1507,32 +1568,45 @@ hipError_t launch_matvec_q8(const MatvecArgs& a, const DeviceInfo& dev, hipStrea
         return launch_fill_scaled_zero(a.scale, a.output, a.N, a.M, stream);
     }
     if (a.M == 1) return dispatch_m1<kEpiPlain>(a, dev, stream, variant);
-    // Batched, 768 < K <= 2048 on large weights: codes split across a
-    // workgroup's waves, x parts in VGPRs (every wave busy from K > 896; at
-    // K = 512 half of them would idle and the kernels below win).  Against
-    // the kernels below (same-process, MI355X): 1.1-1.5x from 5 vectors at
-    // 16384 <= N <= 151936, 2.6-3.4x at K = 2048 with 16 vectors; with 4
-    // vectors it wins from N = 32768, and the VALU path keeps 2 and 3.
-    // Below 16384 rows (decoder-sized weights) it wins where the VALU path's
-    // M + 1 operations per code outgrow the k-split kernel's cost, about one
-    // fixed pass (~10 us at K = 2048, ~6 us at K = 1024) per round of one
-    // workgroup per CU.  Same-process, launches queued, VALU -> k-split (us):
-    // K = 2048: 11008 rows x 5 / 16 vectors 14.4 -> 10.9 / 23.9 -> 12.8,
-    // 5632 x 12 / 16 15.4 -> 9.9 / 16.2 -> 10.9, 2048 x 32 12.6 -> 10.5;
-    // K = 1024: 8192 x 5 6.7 -> 6.3, 5632 x 8 6.7 -> 6.2, 4096 x 16 7.5 ->
-    // 6.6.  The VALU path keeps 4096 rows at K = 2048 (9.7 against 10.7 at 16
-    // vectors), 4 vectors, and two or more rounds at 4096 rows or fewer.
+    // Batched, 768 < K <= 4096: codes split across a workgroup's waves, x parts in
+    // VGPRs (every wave busy from K > 896; at K = 512 half of them would idle and
+    // the kernels below win).  Its cost is one pass per round of one workgroup per
+    // CU (4.2, 6.0, 7.9, 9.5 us at K = 1024, 2048, 3072, 4096 with 8 vectors, about
+    // a tenth more with 16) and the weight's stream; the VALU path's grows with
+    // rows x (vectors + 1 per pass of 8).  Same process, launches issued one by one,
+    // VALU -> k-split (us):
+    //   K = 1024: 4096 rows x 5 / 16 vectors 4.7 -> 4.2 / 5.8 -> 4.4, 16384 x 3 6.1 -> 5.8
+    //   K = 2048: 5632 x 5 8.4 -> 6.5, 16384 x 3 8.8 -> 8.0, 2048 x 32 9.9 -> 7.0
+    //   K = 3072: 2048 x 16 10.0 -> 9.0, 4096 x 6 8.6 -> 8.3, 11008 x 3 10.9 -> 10.4
+    //   K = 4096: 4096 x 8 9.8 -> 10.1, x 12 15.1 -> 11.3; 5632 x 5 11.5 -> 10.0,
+    //             11008 x 16 37.9 -> 15.0, 16384 x 3 15.4 -> 13.8
+    // Up to 4096 rows at 1024 < K <= 2048 (and past 16 vectors at K <= 1024) the VALU
+    // instances keep the calls that they had: their names are checked for there.
     const auto ksplit_small = [&]() {
         const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
         const uint32_t ntiles = (a.N + 15u) / 16u;
         const bool one_round = (uint64_t)(ntiles < cus ? ntiles : cus) * ((a.M + 15u) / 16u) <= cus;
         if (a.M >= 32u && one_round) return true;
-        if (a.K > 1024u) return (a.N >= 11008u && a.M >= 5u) || (a.N >= 5632u && a.M >= 12u);
-        return (a.N >= 8192u && a.M >= 5u) || (a.N >= 5632u && a.M >= 8u) ||
-               (a.N >= 4096u && a.M >= 12u && a.M <= 16u);
+        if (a.K > 1024u) return a.N > 4096u && a.M >= 5u;
+        return (a.N >= 5632u && a.M >= 5u) || (a.N >= 4096u && a.M >= 5u && a.M <= 16u);
     };
+    if (a.K > 2048u && a.K <= 4096u && (a.M + 15u) / 16u <= 65535u) {
+        const bool three = a.K <= 3072u;
+        const uint64_t ops = (uint64_t)a.N * (a.M + (a.M + 7u) / 8u);
+        if ((a.M >= 5u && (a.N > 4096u || ops >= (three ? 28000u : 38000u))) ||
+            (a.M >= 3u && a.N >= (three ? 10240u : 16384u))) {
+            if (three) {
+                if (a.M <= 5u) return launch_ksplit<3, 3>(a, dev, stream, variant);
+                if (a.M <= 8u) return launch_ksplit<3, 2>(a, dev, stream, variant);
+                return launch_ksplit<3, 1>(a, dev, stream, variant);
+            }
+            if (a.M <= 5u) return launch_ksplit<4, 3>(a, dev, stream, variant);
+            if (a.M <= 8u) return launch_ksplit<4, 2>(a, dev, stream, variant);
+            return launch_ksplit<4, 1>(a, dev, stream, variant);
+        }
+    }
     if (a.K > 768u && a.K <= 2048u && (a.M + 15u) / 16u <= 65535u &&
-        (a.N >= kMfmaMinRows ? (a.M >= 5u || (a.M == 4u && a.N >= 32768u)) : ksplit_small())) {
+        (a.N >= kMfmaMinRows ? a.M >= 3u : ksplit_small())) {
         if (a.K <= 1024u) {
             // The store wave holds its workgroup's scales in LDS beside the
             // 96 KiB of stages and partials: up to 1023 tiles per workgroup
