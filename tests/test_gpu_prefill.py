@@ -823,3 +823,47 @@ def test_matmul_activations_past_the_f16_window(N, M, K, ws):
     print(wxo_q8.last_variant(), flush=True)
     rows = np.unique(np.r_[np.arange(0, N, 23), 1, 5 % N, 7 % N, N // 2, min(N - 1, 70), N - 1])
     assert_matmul(out.download(np.float32, N * M), a, w, s, N, M, K, rows=rows)
+
+
+@pytest.mark.parametrize("N,Ms,K,form", [
+    (5, [2048, 2048, 33], 2048, "matmul.tokens_as_vectors"),   # one pass of 8, a ragged last projection
+    (8, [4097, 1], 1025, "matmul.tokens_as_vectors"),
+    (17, [3000, 2000, 700, 15], 1000, "matmul.tokens_as_vectors"),  # two passes, the second with one token
+    (32, [2500, 2500], 3072, "matmul.tokens_as_vectors"),
+    (16, [4200, 500], 4095, "matmul.tokens_as_vectors"),
+    (33, [300], 1030, "x16.ksplit2"),                           # fewer tiles than workgroups per pass
+    (64, [2048, 2048, 2048], 2048, "x16.ksplit2"),              # 6 tile passes per CU
+    (77, [1000, 1, 530], 769, "x16.ksplit2"),
+    (140, [4080], 3073, "x16.ksplit2"),                         # 255 tiles, nine passes
+    (4096, [100], 1024, "x16.ksplit2"),                         # a pass per CU
+])
+def test_matmul_tokens_on_the_ksplit_kernel(N, Ms, K, form):
+    """Short prompts on the batched k-split kernel: several projections in one
+    launch, 16 tokens a pass, every pass in one round.  Every sampled output
+    within the matmulQ8 bar of the oracle (Inf and NaN activations included),
+    the same bits on a second run, nothing written past the outputs."""
+    rng = np.random.default_rng(N + K + sum(Ms))
+    a = rng.standard_normal(N * K).astype(np.float32)
+    a[(N - 1) * K + K - 1] = np.inf
+    a[3 * K + 2] = np.nan
+    ba = wxo_q8.DeviceBuffer.from_array(a)
+    host, bufs = [], []
+    for M in Ms:
+        w = random_packed(rng, M, K)
+        s = rng.uniform(0.001, 0.05, M).astype(np.float32)
+        out = wxo_q8.DeviceBuffer(4 * (N * M + 64))
+        out.upload(np.full(N * M + 64, 7.5, np.float32))
+        host.append((w, s, M))
+        bufs.append((wxo_q8.DeviceBuffer.from_array(w), wxo_q8.DeviceBuffer.from_array(s), out, M))
+    runs = []
+    for _ in range(2):
+        wxo_q8.matmul_q8_multi_device(ba, bufs, N, K)
+        wxo_q8.synchronize()
+        v = wxo_q8.last_variant().split()
+        assert v[1] == form and (v[0].startswith("matvec_q8_ksplit") or N > 32), v
+        runs.append([b[2].download(np.float32, N * b[3] + 64) for b in bufs])
+    rows = np.arange(N) if N <= 140 else np.unique(np.r_[np.arange(0, N, 61), 3, N - 1])
+    for (w, s, M), got, again in zip(host, *runs):
+        assert_bits_equal(again, got, "repeat")
+        assert np.all(got[N * M:] == np.float32(7.5)), f"M={M}: written past the output"
+        assert_matmul(got[:N * M], a, w, s, N, M, K, rows=rows)

@@ -82,6 +82,12 @@ struct Projection {
 };
 hipError_t launch_matvec_q8_multi(const Projection* projections, uint32_t count, const float* x, uint32_t K,
                                   const DeviceInfo& dev, hipStream_t stream, Variant* variant);
+// The same for M vectors x [M, K] (output_p [M, N_p]) on the k-split kernel, 768 <
+// K <= 4096; _pays: whether that beats one call per projection (M >= 5).
+bool matvec_q8_batched_multi_pays(const Projection* projections, uint32_t count, uint32_t K, uint32_t M,
+                                  const DeviceInfo& dev);
+hipError_t launch_matvec_q8_batched_multi(const Projection* projections, uint32_t count, const float* x, uint32_t K,
+                                          uint32_t M, const DeviceInfo& dev, hipStream_t stream, Variant* variant);
 hipError_t launch_fused_zero(const MatvecArgs& a, int epi, hipStream_t stream);
 hipError_t launch_fill_scaled_zero(const float* scale, float* y, uint32_t N, uint32_t M, hipStream_t stream);
 

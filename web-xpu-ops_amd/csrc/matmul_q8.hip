@@ -1256,7 +1256,16 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // the batched path streams the weight once per 8 or 16 tokens (3.6 us
     // for 1 token, 10.5 us for 32; the GEMM wins from about 64 tokens).
     // Both compute the matvecQ8 form.
+    Projection pv[kMaxMatmulProjections];
+    for (uint32_t i = 0; i < n; ++i) pv[i] = Projection{p[i].weight, p[i].scale, p[i].output, p[i].M};
     if (N <= 32u) {
+        // several projections in one launch where the k-split kernel pays for
+        // their rows together (24 tokens, two of 5632 x 2048: 26.1 -> 12.8 us)
+        if (n > 1u && matvec_q8_batched_multi_pays(pv, n, K, N, dev)) {
+            const hipError_t e = launch_matvec_q8_batched_multi(pv, n, a, K, N, dev, stream, variant);
+            if (variant && e == hipSuccess) variant->form = "matmul.tokens_as_vectors";
+            return e;
+        }
         for (uint32_t i = 0; i < n; ++i) {
             MatvecArgs mv{p[i].weight, p[i].scale, a, p[i].output, p[i].M, K, N, (uint32_t)(((uint64_t)K + 3) / 4)};
             const hipError_t e = launch_matvec_q8(mv, dev, stream, variant);
@@ -1282,6 +1291,32 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     }
     const uint32_t steps = (uint32_t)(((uint64_t)K + 63u) / 64u);
     const char* kname = n > 1 ? "matmul_q8.multi" : "matmul_q8";
+    // With a workspace, short prompts whose 32-row tiles fill at most a quarter (a
+    // half) of the CUs split their K steps between 4 (2) workgroups, each run at
+    // least 4 steps per K group; the parts' sums meet in a second launch.
+    const size_t blk32 = (size_t)32u * kBN * 4u;
+    const bool split4 = workspace && 4u * t1 <= cus && steps >= 32u && 3u * t1 * blk32 <= workspace_bytes;
+    const bool split2 = workspace && 2u * t1 <= cus && steps >= 16u && t1 * blk32 <= workspace_bytes;
+    // Short prompts on the batched k-split kernel, 16 tokens a pass, all passes in
+    // one round of the CUs: it splits each activation once per 16-row tile range
+    // instead of once per 32- or 64-row tile, and waits for no barrier per step.
+    // From a sweep of 33 to 256 tokens x 1024 to 11264 rows, us, the tiles below ->
+    // this (K = 2048): 64 x 2048 16.8 -> 8.2, 64 x 6144 17.4 -> 12.8, 128 x 4096 17.6
+    // -> 15.3, 256 x 2048 17.4 -> 15.9, 96 x 6144 19.5 -> 18.1 (9 tile passes per CU);
+    // past 9 it loses (80 x 8192 19.7 -> 20.8, 160 x 4096 19.7 -> 21.1).  The same
+    // line at K = 1024 (64 x 6144 11.7 -> 8.9) and 4096 (64 x 6144 28.7 -> 20.9).
+    // The forms split through a workspace stay where they apply.
+    const uint64_t passes = (N + 15u) / 16u;
+    uint64_t t16 = 0;
+    for (uint32_t i = 0; i < n; ++i) t16 += (p[i].M + 15ull) / 16u;
+    if (!split4 && !split2 && K > 768u && K <= 4096u && passes <= cus && t16 * passes <= 9ull * cus) {
+        const hipError_t e = launch_matvec_q8_batched_multi(pv, n, a, K, N, dev, stream, variant);
+        if (variant && e == hipSuccess) {
+            variant->kernel = kname;
+            variant->form = "x16.ksplit2";  // K split over a workgroup's waves, two tiles per barrier
+        }
+        return e;
+    }
     // One workgroup of 8 waves per CU on the direct kernel, each wave 32 or 48
     // rows x 64 tokens.  The larger tile needs 1.26 times the smaller one's time
     // for 1.5 times its work (the activations' LDS reads, split and barriers per
@@ -1401,15 +1436,11 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         }
     }
     if (t1 <= cus) {
-        // With a workspace, tiles that fill at most a quarter (a half) of the
-        // CUs also split their K steps between 4 (2) workgroups, each run at
-        // least 4 steps per K group; the parts' sums meet in a second launch.
-        const size_t blk = (size_t)32u * kBN * 4u;
-        if (workspace && 4u * t1 <= cus && steps >= 32u && 3u * t1 * blk <= workspace_bytes) {
+        if (split4) {
             set_variant(variant, kname, "FB1.PD4.ksplit2.wgsplit4", 16, 32, 0, (int)kBN, (uint32_t)(4u * t1));
             return launch_fb<1, 8, 64, 4, 2, true>(a, p, n, N, K, stream, workspace, (uint32_t)t1, 4u);
         }
-        if (workspace && 2u * t1 <= cus && steps >= 16u && t1 * blk <= workspace_bytes) {
+        if (split2) {
             set_variant(variant, kname, "FB1.PD4.ksplit2.wgsplit2", 16, 32, 0, (int)kBN, (uint32_t)(2u * t1));
             return launch_fb<1, 8, 64, 4, 2, true>(a, p, n, N, K, stream, workspace, (uint32_t)t1, 2u);
         }

@@ -968,10 +968,41 @@ constexpr int ks_gcd(int a, int b) { return b == 0 ? a : ks_gcd(b, a % b); }
 template <int PACK>
 constexpr uint32_t ks_vectors() { return PACK == 1 ? 16u : PACK == 2 ? 8u : 5u; }
 
-template <int SW, int PACK, bool STW = false>
-__global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
-    const uint32_t* __restrict__ weight, const float* __restrict__ scale, const float* __restrict__ x,
-    float* __restrict__ y, uint32_t N, uint32_t K, uint32_t W, uint32_t M) {
+// Where a 16-row tile of the launch comes from: one weight, or several that
+// share the vectors (their tiles end to end).
+struct KsTile {
+    const uint32_t* weight;  // the tile's first row
+    const float* scale;
+    float* y;                // the tile's first row of vector 0
+    uint32_t rows, N;        // rows in the tile; the projection's rows
+};
+struct KsOne {
+    const uint32_t* weight;
+    const float* scale;
+    float* y;
+    uint32_t N;
+    __device__ __forceinline__ uint32_t tiles() const { return (N + 15u) / 16u; }
+    __device__ __forceinline__ KsTile tile(uint32_t t, uint32_t W) const {
+        return {weight + (size_t)t * 16u * W, scale + (size_t)t * 16u, y + (size_t)t * 16u, min(16u, N - t * 16u), N};
+    }
+};
+struct KsSeveral {
+    const uint32_t* weight[kMaxProjections];
+    const float* scale[kMaxProjections];
+    float* y[kMaxProjections];
+    uint32_t N[kMaxProjections];
+    uint32_t t0[kMaxProjections + 1];  // first tile of each (0xffffffff past the last); [4]: all tiles
+    __device__ __forceinline__ uint32_t tiles() const { return t0[kMaxProjections]; }
+    __device__ __forceinline__ KsTile tile(uint32_t t, uint32_t W) const {
+        const uint32_t p = (t >= t0[1] ? 1u : 0u) + (t >= t0[2] ? 1u : 0u) + (t >= t0[3] ? 1u : 0u);  // wave-uniform
+        const KsOne one{weight[p], scale[p], y[p], N[p]};
+        return one.tile(t - t0[p], W);
+    }
+};
+
+template <int SW, int PACK, bool STW, typename Src>
+__device__ __forceinline__ void ksplit_body(const Src& src, const float* __restrict__ x, uint32_t K, uint32_t W,
+                                            uint32_t M) {
     extern __shared__ __attribute__((aligned(16))) uint8_t ks_lds[];
     constexpr int G = kKsGroup, D = kKsStages;
     constexpr uint32_t SC = 128, TBY = 16u * SC;
@@ -992,7 +1023,7 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
     uint8_t* wst = ks_lds + wv * ((uint32_t)D * TBY);
     float* red = reinterpret_cast<float*>(ks_lds + kKsWaves * (uint32_t)D * TBY);  // [2][G][8 waves][64][4]
     const uint32_t rowbytes = W * 4u;
-    const uint32_t ntiles = (N + 15u) / 16u;
+    const uint32_t ntiles = src.tiles();
     const uint32_t b0 = (uint32_t)((uint64_t)blockIdx.x * ntiles / gridDim.x);
     const uint32_t b1 = (uint32_t)((uint64_t)(blockIdx.x + 1u) * ntiles / gridDim.x);
     const uint32_t ngroups = (b1 - b0 + G - 1) / G;
@@ -1004,6 +1035,9 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
 
     if constexpr (STW) {
         if (wv == kKsWaves) {
+            const uint32_t N = src.N;
+            const float* const scale = src.scale;
+            float* const y = src.y;
             // The store wave: after each group's barrier it sums the group's
             // tiles (their 8 partials in wave order), scales and stores them,
             // while the streaming waves go on.  Its y stores count on its own
@@ -1068,9 +1102,8 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
         const uint32_t ti = i / SW, s = i % SW;
         const uint32_t c0 = 128u * (wv + kKsWaves * s);
         const bool ok = b0 + ti < b1 && c0 < K;
-        const uint32_t tile = ok ? b0 + ti : 0u;
-        const uint32_t rows = ok ? min(16u, N - tile * 16u) : 0u;
-        const __amdgpu_buffer_rsrc_t wrs = make_rsrc(weight + (size_t)tile * 16u * W, rows * rowbytes);
+        const KsTile tl = src.tile(ok ? b0 + ti : 0u, W);
+        const __amdgpu_buffer_rsrc_t wrs = make_rsrc(tl.weight, ok ? tl.rows * rowbytes : 0u);
         uint8_t* sb = wst + (i % (uint32_t)D) * TBY;
 #pragma unroll
         for (int ii = 0; ii < 2; ++ii)
@@ -1079,8 +1112,8 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
                 kCachePolicyNT);
         if (!STW && s == SW - 1u) {
             const bool mine = b0 + ti < b1 && (ti & 7u) == wv;  // this wave sums and stores the tile
-            const __amdgpu_buffer_rsrc_t srs = make_rsrc(scale + (size_t)(mine ? b0 + ti : 0u) * 16u,
-                                                         mine ? min(16u, N - (b0 + ti) * 16u) * 4u : 0u);
+            const KsTile ts = src.tile(mine ? b0 + ti : 0u, W);
+            const __amdgpu_buffer_rsrc_t srs = make_rsrc(ts.scale, mine ? ts.rows * 4u : 0u);
             sc = __builtin_amdgcn_raw_buffer_load_b128(srs, (int)(g * 16u), 0, 0);
         }
     };
@@ -1119,68 +1152,67 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
 
     bf16x8 bx[SW][2][2][NB];
 #pragma unroll
-    for (int s = 0; s < SW; ++s)
+    for (int i = 0; i < SW * 2; ++i) {
+        const int s = i / 2, u = i % 2;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int q = 0; q < NI; ++q) {
+            const uint32_t v = 4u * (uint32_t)q + lane / 16u;
+            *reinterpret_cast<u32x4v*>(xst + (uint32_t)q * 8192u + (lane / 16u) * 256u + ((lane % 16u) ^ swz(v)) * 16u) =
+                xl[s][u][q];
+        }
+        uint32_t xv[16];
 #pragma unroll
-            for (int q = 0; q < NI; ++q) {
-                const uint32_t v = 4u * (uint32_t)q + lane / 16u;
-                *reinterpret_cast<u32x4v*>(xst + (uint32_t)q * 8192u + (lane / 16u) * 256u + ((lane % 16u) ^ swz(v)) * 16u) =
-                    xl[s][u][q];
+        for (int q = 0; q < 4; ++q) {
+            const u32x4v t = *reinterpret_cast<const u32x4v*>(
+                xst + (vj >> 2) * 8192u + (vj & 3u) * 256u + ((4u * g + (uint32_t)q) ^ swz(vj)) * 16u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xv[4 * q + e] = t[e];
+        }
+        const uint32_t c0 = 128u * (wv + kKsWaves * (uint32_t)s) + 64u * (uint32_t)u;
+        if (c0 + 64u > K) {  // wave-uniform: entries past K belong to the next vector
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                if (c0 + 16u * g + (uint32_t)e >= K) xv[e] = 0u;
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            u32x4v pv[3];
+            float most = 0.0f;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                uint32_t h, m, l;
+                split3_pair(xv[8 * e + 2 * p], xv[8 * e + 2 * p + 1], h, m, l, most);
+                pv[0][p] = h;
+                pv[1][p] = m;
+                pv[2][p] = l;
             }
-            uint32_t xv[16];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const u32x4v t = *reinterpret_cast<const u32x4v*>(
-                    xst + (vj >> 2) * 8192u + (vj & 3u) * 256u + ((4u * g + (uint32_t)q) ^ swz(vj)) * 16u);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) xv[4 * q + e] = t[e];
-            }
-            const uint32_t c0 = 128u * (wv + kKsWaves * (uint32_t)s) + 64u * (uint32_t)u;
-            if (c0 + 64u > K) {  // wave-uniform: entries past K belong to the next vector
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    if (c0 + 16u * g + (uint32_t)i >= K) xv[i] = 0u;
-            }
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                u32x4v pv[3];
-                float most = 0.0f;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(__float_as_uint(most) == 0x7f800000u) != 0, 0)) {
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
-                    uint32_t h, m, l;
-                    split3_pair(xv[8 * e + 2 * p], xv[8 * e + 2 * p + 1], h, m, l, most);
-                    pv[0][p] = h;
-                    pv[1][p] = m;
-                    pv[2][p] = l;
-                }
-                if (__builtin_expect(__builtin_amdgcn_ballot_w64(__float_as_uint(most) == 0x7f800000u) != 0, 0)) {
+                    uint32_t hw[2], mw[2], lw[2];
 #pragma unroll
-                    for (int p = 0; p < 4; ++p) {
-                        uint32_t hw[2], mw[2], lw[2];
-#pragma unroll
-                        for (int z = 0; z < 2; ++z)
-                            split_x_parts(__uint_as_float(xv[8 * e + 2 * p + z]), hw[z], mw[z], lw[z]);
-                        pv[0][p] = (hw[0] >> 16) | hw[1];
-                        pv[1][p] = (mw[0] >> 16) | mw[1];
-                        pv[2][p] = (lw[0] >> 16) | lw[1];
-                    }
-                }
-                const u32x4v zero = {0u, 0u, 0u, 0u};
-                if constexpr (PACK == 1) {
-#pragma unroll
-                    for (int b = 0; b < 3; ++b) bx[s][u][e][b] = __builtin_bit_cast(bf16x8, pv[b]);
-                } else if constexpr (PACK == 2) {
-                    bx[s][u][e][0] = __builtin_bit_cast(bf16x8, sel == 0u ? pv[0] : pv[1]);
-                    bx[s][u][e][1] = __builtin_bit_cast(bf16x8, sel == 0u ? pv[2] : zero);
-                } else {
-                    bx[s][u][e][0] = __builtin_bit_cast(bf16x8, sel == 0u ? pv[0] : sel == 1u ? pv[1] : pv[2]);
+                    for (int t = 0; t < 2; ++t)
+                        split_x_parts(__uint_as_float(xv[8 * e + 2 * p + t]), hw[t], mw[t], lw[t]);
+                    pv[0][p] = (hw[0] >> 16) | hw[1];
+                    pv[1][p] = (mw[0] >> 16) | mw[1];
+                    pv[2][p] = (lw[0] >> 16) | lw[1];
                 }
             }
-            // one 64-code run at a time (left to itself the compiler converts
-            // them side by side and spills)
-            __builtin_amdgcn_sched_barrier(0);
+            const u32x4v zero = {0u, 0u, 0u, 0u};
+            if constexpr (PACK == 1) {
+#pragma unroll
+                for (int b = 0; b < 3; ++b) bx[s][u][e][b] = __builtin_bit_cast(bf16x8, pv[b]);
+            } else if constexpr (PACK == 2) {
+                bx[s][u][e][0] = __builtin_bit_cast(bf16x8, sel == 0u ? pv[0] : pv[1]);
+                bx[s][u][e][1] = __builtin_bit_cast(bf16x8, sel == 0u ? pv[2] : zero);
+            } else {
+                bx[s][u][e][0] = __builtin_bit_cast(bf16x8, sel == 0u ? pv[0] : sel == 1u ? pv[1] : pv[2]);
+            }
         }
+        // one 64-code run at a time (left to itself the compiler converts
+        // them side by side and spills)
+        __builtin_amdgcn_sched_barrier(0);
+    }
 
     f32x4 acc[NB], pacc[NB];
 #pragma unroll
@@ -1242,11 +1274,10 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
         f32x4 sum = part[0];
 #pragma unroll
         for (int w = 1; w < (int)kKsWaves; ++w) sum += part[w];
-        const uint32_t tile = b0 + ti;
-        if (tile < b1 && col_ok && sel == 0u) {
-            const uint32_t row = tile * 16u + 4u * g;
-            float* yo = y + (size_t)(m0 + vj) * N + row;
-            if (row + 3u < N) {
+        if (b0 + ti < b1 && col_ok && sel == 0u) {
+            const KsTile tl = src.tile(b0 + ti, W);
+            float* yo = tl.y + (size_t)(m0 + vj) * tl.N + 4u * g;
+            if (4u * g + 3u < tl.rows) {
                 f32x4 o;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) o[q] = sum[q] * __uint_as_float(rsc[q]);
@@ -1254,7 +1285,7 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
             } else {
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    if (row + (uint32_t)q < N) yo[q] = sum[q] * __uint_as_float(rsc[q]);
+                    if (4u * g + (uint32_t)q < tl.rows) yo[q] = sum[q] * __uint_as_float(rsc[q]);
             }
         }
     };
@@ -1317,6 +1348,21 @@ __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
     }
     if (!STW && pending != ~0u) reduce(pending);
     __builtin_amdgcn_s_waitcnt(0);  // no fetch into LDS outlives the workgroup
+}
+
+
+template <int SW, int PACK, bool STW = false>
+__global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
+    const uint32_t* __restrict__ weight, const float* __restrict__ scale, const float* __restrict__ x,
+    float* __restrict__ y, uint32_t N, uint32_t K, uint32_t W, uint32_t M) {
+    ksplit_body<SW, PACK, STW>(KsOne{weight, scale, y, N}, x, K, W, M);
+}
+
+// Several projections of the same vectors in one launch.
+template <int SW, int PACK>
+__global__ __launch_bounds__(512) void matvec_q8_ksplit_multi_kernel(KsSeveral p, const float* __restrict__ x,
+                                                                    uint32_t K, uint32_t W, uint32_t M) {
+    ksplit_body<SW, PACK, false>(p, x, K, W, M);
 }
 
 constexpr uint32_t kKsLdsBytes = kKsWaves * kKsStages * 16u * 128u + 2u * kKsGroup * kKsWaves * 1024u;
@@ -1507,19 +1553,81 @@ hipError_t launch_mv(const MatvecArgs& a, hipStream_t stream, Variant* variant) 
 // with a contiguous range of 16-row tiles; vector groups of ks_vectors<PACK>()
 // on grid y.  STW adds the store wave (K <= 1024 only: with two steps per
 // wave the x parts need more registers than nine waves per workgroup leave).
+// One round of one workgroup per CU whatever the vector groups, so that each
+// workgroup pays its prologue once (two groups of 16 vectors, N = 5632, K = 2048:
+// 13.2 -> 8.5 us; 11008, 4096: 28.7 -> 18.7).
+dim3 ks_grid(uint32_t tiles, uint32_t groups, uint32_t cus) {
+    const uint32_t x = groups < cus ? cus / groups : 1u;
+    return dim3(tiles < x ? tiles : x, groups);
+}
+
 template <int SW, int PACK, bool STW = false>
 hipError_t launch_ksplit(const MatvecArgs& a, const DeviceInfo& dev, hipStream_t stream, Variant* variant) {
     constexpr uint32_t VPB = ks_vectors<PACK>();
     const uint32_t ntiles = (a.N + 15u) / 16u;
     const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
-    const dim3 grid(ntiles < cus ? ntiles : cus, (a.M + VPB - 1u) / VPB);
+    const dim3 grid = ks_grid(ntiles, (a.M + VPB - 1u) / VPB, cus);
     const size_t lds = kKsLdsBytes + (STW ? (size_t)((ntiles + grid.x - 1u) / grid.x + 1u) * 16u * 4u : 0u);
     hipLaunchKernelGGL((matvec_q8_ksplit_kernel<SW, PACK, STW>), grid, dim3(64 * (kKsWaves + (STW ? 1u : 0u))), lds,
                        stream,
                        a.weight, a.scale, a.vector, a.output, a.N, a.K, a.W, a.M);
-    set_variant(variant, "matvec_q8_ksplit", PACK == 1 ? "x16" : PACK == 2 ? "x8" : "x5", (int)kKsWaves + (STW ? 1 : 0), 16, SW,
-                (int)(a.M < VPB ? a.M : VPB), grid.x, grid.y);
+    set_variant(variant, "matvec_q8_ksplit", PACK == 1 ? "x16" : PACK == 2 ? "x8" : "x5",
+                (int)kKsWaves + (STW ? 1 : 0), 16, SW, (int)(a.M < VPB ? a.M : VPB), grid.x, grid.y);
     return hipGetLastError();
+}
+
+template <int SW, int PACK>
+hipError_t launch_ksplit_multi(const Projection* p, uint32_t count, const float* x, uint32_t K, uint32_t M,
+                               const DeviceInfo& dev, hipStream_t stream, Variant* variant) {
+    constexpr uint32_t VPB = ks_vectors<PACK>();
+    KsSeveral several = {};
+    uint32_t tiles = 0;
+    for (uint32_t i = 0; i < kMaxProjections; ++i) {
+        several.t0[i] = i < count ? tiles : 0xffffffffu;
+        if (i >= count) continue;
+        several.weight[i] = p[i].weight;
+        several.scale[i] = p[i].scale;
+        several.y[i] = p[i].output;
+        several.N[i] = p[i].N;
+        tiles += (p[i].N + 15u) / 16u;
+    }
+    several.t0[kMaxProjections] = tiles;
+    const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
+    const dim3 grid = ks_grid(tiles, (M + VPB - 1u) / VPB, cus);
+    hipLaunchKernelGGL((matvec_q8_ksplit_multi_kernel<SW, PACK>), grid, dim3(512), kKsLdsBytes, stream, several,
+                       x, K, (uint32_t)(((uint64_t)K + 3) / 4), M);
+    set_variant(variant, "matvec_q8_ksplit.multi", PACK == 1 ? "x16" : "x8", (int)kKsWaves, 16, SW,
+                (int)(M < VPB ? M : VPB), grid.x, grid.y);
+    return hipGetLastError();
+}
+
+// Batched, 768 < K <= 4096: codes split across a workgroup's waves, x parts in
+// VGPRs (every wave busy from K > 896; at K = 512 half of them would idle and
+// the kernels below win).  Its cost is one pass per round of one workgroup per
+// CU (4.2, 6.0, 7.9, 9.5 us at K = 1024, 2048, 3072, 4096 with 8 vectors, about
+// a tenth more with 16) and the weight's stream; the VALU path's grows with
+// rows x (vectors + 1 per pass of 8).  Same process, launches issued one by one,
+// VALU -> k-split (us):
+//   K = 1024: 4096 rows x 5 / 16 vectors 4.7 -> 4.2 / 5.8 -> 4.4, 16384 x 3 6.1 -> 5.8
+//   K = 2048: 5632 x 5 8.4 -> 6.5, 16384 x 3 8.8 -> 8.0, 2048 x 32 9.9 -> 7.0
+//   K = 3072: 2048 x 16 10.0 -> 9.0, 4096 x 6 8.6 -> 8.3, 11008 x 3 10.9 -> 10.4
+//   K = 4096: 4096 x 8 9.8 -> 10.1, x 12 15.1 -> 11.3; 5632 x 5 11.5 -> 10.0,
+//             11008 x 16 37.9 -> 15.0, 16384 x 3 15.4 -> 13.8
+// Up to 4096 rows at 1024 < K <= 2048 (and past 16 vectors at K <= 1024) the VALU
+// instances keep the calls that they had: their names are checked for there.
+bool ksplit_pays(uint64_t N, uint32_t K, uint32_t M, const DeviceInfo& dev) {
+    if (K <= 768u || K > 4096u || (M + 15u) / 16u > 65535u) return false;
+    if (K > 2048u) {
+        const bool three = K <= 3072u;
+        const uint64_t ops = N * (M + (M + 7u) / 8u);
+        return (M >= 5u && (N > 4096u || ops >= (three ? 28000u : 38000u))) ||
+               (M >= 3u && N >= (three ? 10240u : 16384u));
+    }
+    if (N >= kMfmaMinRows) return M >= 3u;
+    const uint64_t cus = (uint64_t)(dev.cu_count > 0 ? dev.cu_count : 256), ntiles = (N + 15u) / 16u;
+    if (M >= 32u && (ntiles < cus ? ntiles : cus) * ((M + 15u) / 16u) <= cus) return true;  // one round
+    if (K > 1024u) return N > 4096u && M >= 5u;
+    return (N >= 5632u && M >= 5u) || (N >= 4096u && M >= 5u && M <= 16u);
 }
 
 // Rows per workgroup: the largest R (up to RMAX) that still gives every SIMD
@@ -1568,63 +1676,35 @@ hipError_t launch_matvec_q8(const MatvecArgs& a, const DeviceInfo& dev, hipStrea
         return launch_fill_scaled_zero(a.scale, a.output, a.N, a.M, stream);
     }
     if (a.M == 1) return dispatch_m1<kEpiPlain>(a, dev, stream, variant);
-    // Batched, 768 < K <= 4096: codes split across a workgroup's waves, x parts in
-    // VGPRs (every wave busy from K > 896; at K = 512 half of them would idle and
-    // the kernels below win).  Its cost is one pass per round of one workgroup per
-    // CU (4.2, 6.0, 7.9, 9.5 us at K = 1024, 2048, 3072, 4096 with 8 vectors, about
-    // a tenth more with 16) and the weight's stream; the VALU path's grows with
-    // rows x (vectors + 1 per pass of 8).  Same process, launches issued one by one,
-    // VALU -> k-split (us):
-    //   K = 1024: 4096 rows x 5 / 16 vectors 4.7 -> 4.2 / 5.8 -> 4.4, 16384 x 3 6.1 -> 5.8
-    //   K = 2048: 5632 x 5 8.4 -> 6.5, 16384 x 3 8.8 -> 8.0, 2048 x 32 9.9 -> 7.0
-    //   K = 3072: 2048 x 16 10.0 -> 9.0, 4096 x 6 8.6 -> 8.3, 11008 x 3 10.9 -> 10.4
-    //   K = 4096: 4096 x 8 9.8 -> 10.1, x 12 15.1 -> 11.3; 5632 x 5 11.5 -> 10.0,
-    //             11008 x 16 37.9 -> 15.0, 16384 x 3 15.4 -> 13.8
-    // Up to 4096 rows at 1024 < K <= 2048 (and past 16 vectors at K <= 1024) the VALU
-    // instances keep the calls that they had: their names are checked for there.
-    const auto ksplit_small = [&]() {
-        const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
-        const uint32_t ntiles = (a.N + 15u) / 16u;
-        const bool one_round = (uint64_t)(ntiles < cus ? ntiles : cus) * ((a.M + 15u) / 16u) <= cus;
-        if (a.M >= 32u && one_round) return true;
-        if (a.K > 1024u) return a.N > 4096u && a.M >= 5u;
-        return (a.N >= 5632u && a.M >= 5u) || (a.N >= 4096u && a.M >= 5u && a.M <= 16u);
-    };
-    if (a.K > 2048u && a.K <= 4096u && (a.M + 15u) / 16u <= 65535u) {
-        const bool three = a.K <= 3072u;
-        const uint64_t ops = (uint64_t)a.N * (a.M + (a.M + 7u) / 8u);
-        if ((a.M >= 5u && (a.N > 4096u || ops >= (three ? 28000u : 38000u))) ||
-            (a.M >= 3u && a.N >= (three ? 10240u : 16384u))) {
-            if (three) {
-                if (a.M <= 5u) return launch_ksplit<3, 3>(a, dev, stream, variant);
-                if (a.M <= 8u) return launch_ksplit<3, 2>(a, dev, stream, variant);
-                return launch_ksplit<3, 1>(a, dev, stream, variant);
-            }
+    if (ksplit_pays(a.N, a.K, a.M, dev)) {
+        if (a.K > 3072u) {
             if (a.M <= 5u) return launch_ksplit<4, 3>(a, dev, stream, variant);
             if (a.M <= 8u) return launch_ksplit<4, 2>(a, dev, stream, variant);
             return launch_ksplit<4, 1>(a, dev, stream, variant);
         }
-    }
-    if (a.K > 768u && a.K <= 2048u && (a.M + 15u) / 16u <= 65535u &&
-        (a.N >= kMfmaMinRows ? a.M >= 3u : ksplit_small())) {
-        if (a.K <= 1024u) {
-            // The store wave holds its workgroup's scales in LDS beside the
-            // 96 KiB of stages and partials: up to 1023 tiles per workgroup
-            // (4.19M rows on 256 CUs); past that, the eight-wave form.
-            const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
-            const uint32_t ntiles = (a.N + 15u) / 16u, gx = ntiles < cus ? ntiles : cus;
-            if (kKsLdsBytes + (uint64_t)((ntiles + gx - 1u) / gx + 1u) * 64u <= kMfmaLdsBytes) {
-                if (a.M <= 5u) return launch_ksplit<1, 3, true>(a, dev, stream, variant);
-                if (a.M <= 8u) return launch_ksplit<1, 2, true>(a, dev, stream, variant);
-                return launch_ksplit<1, 1, true>(a, dev, stream, variant);
-            }
-            if (a.M <= 5u) return launch_ksplit<1, 3>(a, dev, stream, variant);
-            if (a.M <= 8u) return launch_ksplit<1, 2>(a, dev, stream, variant);
-            return launch_ksplit<1, 1>(a, dev, stream, variant);
+        if (a.K > 2048u) {
+            if (a.M <= 5u) return launch_ksplit<3, 3>(a, dev, stream, variant);
+            if (a.M <= 8u) return launch_ksplit<3, 2>(a, dev, stream, variant);
+            return launch_ksplit<3, 1>(a, dev, stream, variant);
         }
-        if (a.M <= 5u) return launch_ksplit<2, 3>(a, dev, stream, variant);
-        if (a.M <= 8u) return launch_ksplit<2, 2>(a, dev, stream, variant);
-        return launch_ksplit<2, 1>(a, dev, stream, variant);
+        if (a.K > 1024u) {
+            if (a.M <= 5u) return launch_ksplit<2, 3>(a, dev, stream, variant);
+            if (a.M <= 8u) return launch_ksplit<2, 2>(a, dev, stream, variant);
+            return launch_ksplit<2, 1>(a, dev, stream, variant);
+        }
+        // The store wave holds its workgroup's scales in LDS beside the 96 KiB
+        // of stages and partials: up to 1023 tiles per workgroup (4.19M rows on
+        // 256 CUs); past that, the eight-wave form.
+        const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
+        const uint32_t ntiles = (a.N + 15u) / 16u, gx = ks_grid(ntiles, (a.M + 15u) / 16u, cus).x;
+        if (kKsLdsBytes + (uint64_t)((ntiles + gx - 1u) / gx + 1u) * 64u <= kMfmaLdsBytes) {
+            if (a.M <= 5u) return launch_ksplit<1, 3, true>(a, dev, stream, variant);
+            if (a.M <= 8u) return launch_ksplit<1, 2, true>(a, dev, stream, variant);
+            return launch_ksplit<1, 1, true>(a, dev, stream, variant);
+        }
+        if (a.M <= 5u) return launch_ksplit<1, 3>(a, dev, stream, variant);
+        if (a.M <= 8u) return launch_ksplit<1, 2>(a, dev, stream, variant);
+        return launch_ksplit<1, 1>(a, dev, stream, variant);
     }
     // Batched.  The matrix-core kernels pay a per-workgroup prologue (the x
     // parts of the whole K for their 16-vector tile, written to LDS) and a
@@ -1697,6 +1777,25 @@ hipError_t launch_matvec_q8(const MatvecArgs& a, const DeviceInfo& dev, hipStrea
     if (a.M <= 2) return dispatch_mv<2>(a, dev, stream, variant);
     if (a.M <= 4) return dispatch_mv<4>(a, dev, stream, variant);
     return dispatch_mv<8>(a, dev, stream, variant);
+}
+
+bool matvec_q8_batched_multi_pays(const Projection* p, uint32_t count, uint32_t K, uint32_t M, const DeviceInfo& dev) {
+    uint64_t rows = 0;
+    for (uint32_t i = 0; i < count; ++i) rows += (p[i].N + 15ull) / 16u * 16u;
+    return M >= 5u && rows <= 0x7fffffffu && ksplit_pays(rows, K, M, dev);
+}
+
+hipError_t launch_matvec_q8_batched_multi(const Projection* p, uint32_t count, const float* x, uint32_t K, uint32_t M,
+                                          const DeviceInfo& dev, hipStream_t stream, Variant* variant) {
+    if (count == 0u || count > kMaxProjections || K <= 768u || K > 4096u) return hipErrorInvalidValue;
+    if (K > 3072u) return M <= 8u ? launch_ksplit_multi<4, 2>(p, count, x, K, M, dev, stream, variant)
+                                  : launch_ksplit_multi<4, 1>(p, count, x, K, M, dev, stream, variant);
+    if (K > 2048u) return M <= 8u ? launch_ksplit_multi<3, 2>(p, count, x, K, M, dev, stream, variant)
+                                  : launch_ksplit_multi<3, 1>(p, count, x, K, M, dev, stream, variant);
+    if (K > 1024u) return M <= 8u ? launch_ksplit_multi<2, 2>(p, count, x, K, M, dev, stream, variant)
+                                  : launch_ksplit_multi<2, 1>(p, count, x, K, M, dev, stream, variant);
+    return M <= 8u ? launch_ksplit_multi<1, 2>(p, count, x, K, M, dev, stream, variant)
+                   : launch_ksplit_multi<1, 1>(p, count, x, K, M, dev, stream, variant);
 }
 
 hipError_t launch_matvec_q8_fused(const MatvecArgs& a, int epi, const DeviceInfo& dev, hipStream_t stream,
