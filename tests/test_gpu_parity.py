@@ -354,6 +354,30 @@ def test_batched_ksplit_steps(N, K, M):
         assert_matvec(ys[m], w, s, xs[m], N, K)
 
 
+@pytest.mark.parametrize("N,K,M,kernel", [
+    (5632, 4097, 9, "matvec_q8_ksplit.multi"), (5000, 6143, 8, "matvec_q8_ksplit.multi"),   # two passes
+    (4100, 6144, 16, "matvec_q8_ksplit.multi"), (4099, 6145, 17, "matvec_q8_ksplit.multi"),  # two, three
+    (3001, 11008, 33, "matvec_q8_ksplit.multi"), (16390, 9219, 5, "matvec_q8_ksplit.multi"),  # four
+    (2048, 4100, 2048, "matvec_q8_ksplit.multi"), (2049, 4100, 2048, "matvec_q8_mv"),  # 64, 65 tiles per workgroup
+    (150, 65536, 140, "matvec_q8_mv"), (300, 65536, 140, "matvec_q8_ksplit.multi"), (300, 65537, 140, "matvec_q8_mv"),
+    (2048, 5632, 16, "matvec_q8_mv"), (8192, 5632, 4, "matvec_q8_mv"),
+])
+def test_batched_ksplit_long_rows(N, K, M, kernel):
+    """Rows longer than one pass of the k-split kernel: the last pass ragged, the
+    sums kept between passes for one to 64 tiles per workgroup, the dispatch's
+    lines; an infinity in the last pass and a NaN in the first."""
+    rng = np.random.default_rng(N + 3 * K + M)
+    w = random_weights(rng, N, K, full_range=True)
+    s = rng.uniform(0.001, 0.05, N).astype(np.float32)
+    xs = rng.standard_normal((M, K)).astype(np.float32)
+    xs[0, K - 1] = np.inf
+    xs[M - 1, 5] = np.nan
+    ys = wxo_q8.matvecQ8Batched(weight=w, scale=s, vectors=xs, N=N, K=K, M=M)
+    assert wxo_q8.last_variant().split(" ")[0] == kernel, wxo_q8.last_variant()
+    for m in (range(M) if M < 20 else [0, 1, 15, 16, 31, M // 2, M - 2, M - 1]):
+        assert_matvec(ys[m], w, s, xs[m], N, K)
+
+
 @pytest.mark.parametrize("M,K", [(5, 1030), (8, 64), (12, 2048), (13, 4099), (16, 1024), (17, 1500), (32, 520),
                                  (6, 3000), (14, 1000), (16, 768), (13, 1536), (20, 1024), (33, 1000),
                                  (5, 769), (5, 2047), (6, 897), (7, 1024), (8, 1025), (8, 2048), (9, 1100),

@@ -23,7 +23,7 @@
 //
 // The small-M batched VALU kernel reuses every loaded word for up to 8
 // vectors (one unpack per code, one FMA per vector, the vector slices in
-// VGPRs); large weights with 5 or more vectors go to the matrix cores.
+// VGPRs); larger weights with 3 or 5 vectors and more go to the matrix cores.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -903,7 +903,7 @@ __global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Batched, K up to 4096: the row's codes split across the workgroup's 8 waves
+// Batched: the row's codes (up to 4096 at a time) split across the workgroup's 8 waves
 // (wave w owns codes 128 (w + 8 s) .. +127 of step s = 0 .. SW - 1), so each
 // wave's share of the x parts fits in its VGPRs (12 bf16x8 registers per
 // step and B operand set) and is never read again from LDS; only the weight
@@ -1000,9 +1000,21 @@ struct KsSeveral {
     }
 };
 
-template <int SW, int PACK, bool STW, typename Src>
+constexpr uint32_t kKsLdsBytes = kKsWaves * kKsStages * 16u * 128u + 2u * kKsGroup * kKsWaves * 1024u;
+
+// LONG: rows longer than a workgroup's 1024 SW codes, `Kc` codes (a multiple of
+// 1024) at a time: the whole tile range for each, the sums so far in LDS, 1 KiB
+// per tile behind the partials (a tile is summed by the same wave every time, so a
+// lane reads back what it wrote).  A pass costs about 9 us at 3072 codes, most of
+// it the vectors' load and split, which the next tiles share: 16 x 4096 x 11008
+// 51.2 -> 37.0 us against the VALU kernel, 16 x 11008 x 8192 95.3 -> 37.5.  At 4096
+// codes a pass the 16-vector form spills 33 registers (38.6, 35.7; 16 x 2048 x 5632
+// 25.3 against 18.9).
+template <int SW, int PACK, bool STW, bool LONG, typename Src>
 __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restrict__ x, uint32_t K, uint32_t W,
-                                            uint32_t M) {
+                                            uint32_t M, uint32_t Kc) {
+    static_assert(!(LONG && STW), "the streaming waves sum long rows");
+    uint32_t kc0 = 0u, Kl = LONG ? min(K, Kc) : K;  // this pass: codes kc0 .. kc0 + Kl - 1 of every row
     extern __shared__ __attribute__((aligned(16))) uint8_t ks_lds[];
     constexpr int G = kKsGroup, D = kKsStages;
     constexpr uint32_t SC = 128, TBY = 16u * SC;
@@ -1101,14 +1113,14 @@ __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restr
     auto issue = [&](uint32_t i, u32x4v& sc) {
         const uint32_t ti = i / SW, s = i % SW;
         const uint32_t c0 = 128u * (wv + kKsWaves * s);
-        const bool ok = b0 + ti < b1 && c0 < K;
+        const bool ok = b0 + ti < b1 && c0 < Kl;
         const KsTile tl = src.tile(ok ? b0 + ti : 0u, W);
         const __amdgpu_buffer_rsrc_t wrs = make_rsrc(tl.weight, ok ? tl.rows * rowbytes : 0u);
         uint8_t* sb = wst + (i % (uint32_t)D) * TBY;
 #pragma unroll
         for (int ii = 0; ii < 2; ++ii)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                wrs, (__attribute__((address_space(3))) void*)(sb + (uint32_t)ii * 1024u), 16, voff[ii], (int)c0, 0,
+                wrs, (__attribute__((address_space(3))) void*)(sb + (uint32_t)ii * 1024u), 16, voff[ii], (int)(LONG && !ok ? 0u : kc0 + c0), 0,
                 kCachePolicyNT);
         if (!STW && s == SW - 1u) {
             const bool mine = b0 + ti < b1 && (ti & 7u) == wv;  // this wave sums and stores the tile
@@ -1134,6 +1146,7 @@ __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restr
     const __amdgpu_buffer_rsrc_t xrs = make_rsrc(x + (size_t)m0 * K, MC * K * 4u);
     const auto swz = [](uint32_t v) { return (v & 3u) | (((0u - (v >> 2)) & 3u) << 2); };
     uint8_t* const xst = reinterpret_cast<uint8_t*>(red) + wv * 1024u;  // slot i: xst + i * 8192
+    for (;;) {  // passes (one unless LONG)
     u32x4v xl[SW][2][NI];
 #pragma unroll
     for (int s = 0; s < SW; ++s)
@@ -1143,7 +1156,7 @@ __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restr
             for (int q = 0; q < NI; ++q) {
                 const uint32_t v = 4u * (uint32_t)q + lane / 16u;
                 const uint32_t c = 128u * (wv + kKsWaves * (uint32_t)s) + 64u * (uint32_t)u + 4u * (lane % 16u);
-                const int off = (v < MC && c < K) ? (int)((v * K + c) * 4u) : (int)0x7ffffff0;
+                const int off = (v < MC && c < Kl) ? (int)((v * K + kc0 + c) * 4u) : (int)0x7ffffff0;
                 xl[s][u][q] = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0);
             }
     u32x4v sbuf[D];
@@ -1169,10 +1182,10 @@ __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restr
             for (int e = 0; e < 4; ++e) xv[4 * q + e] = t[e];
         }
         const uint32_t c0 = 128u * (wv + kKsWaves * (uint32_t)s) + 64u * (uint32_t)u;
-        if (c0 + 64u > K) {  // wave-uniform: entries past K belong to the next vector
+        if (c0 + 64u > Kl) {  // wave-uniform: entries past K belong to the next vector
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-                if (c0 + 16u * g + (uint32_t)e >= K) xv[e] = 0u;
+                if (c0 + 16u * g + (uint32_t)e >= Kl) xv[e] = 0u;
         }
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
@@ -1274,18 +1287,28 @@ __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restr
         f32x4 sum = part[0];
 #pragma unroll
         for (int w = 1; w < (int)kKsWaves; ++w) sum += part[w];
+        if constexpr (LONG) {
+            if (b0 + ti >= b1) return;
+            f32x4* const so_far = reinterpret_cast<f32x4*>(ks_lds + kKsLdsBytes + ti * 1024u) + lane;
+            if (kc0 != 0u) sum += *so_far;
+            if (kc0 + Kl < K) {
+                *so_far = sum;
+                return;
+            }
+        }
         if (b0 + ti < b1 && col_ok && sel == 0u) {
             const KsTile tl = src.tile(b0 + ti, W);
             float* yo = tl.y + (size_t)(m0 + vj) * tl.N + 4u * g;
-            if (4u * g + 3u < tl.rows) {
-                f32x4 o;
+            const bool whole = 4u * g + 3u < tl.rows;
+            f32x4 o;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) o[q] = sum[q] * __uint_as_float(rsc[q]);
+            for (int q = 0; q < 4; ++q) o[q] = sum[q] * __uint_as_float(rsc[q]);
+            if (whole) {
                 *reinterpret_cast<f32x4_a4*>(yo) = o;
             } else {
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    if (4u * g + (uint32_t)q < tl.rows) yo[q] = sum[q] * __uint_as_float(rsc[q]);
+                    if (4u * g + (uint32_t)q < tl.rows) yo[q] = o[q];
             }
         }
     };
@@ -1347,7 +1370,16 @@ __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restr
         }
     }
     if (!STW && pending != ~0u) reduce(pending);
-    __builtin_amdgcn_s_waitcnt(0);  // no fetch into LDS outlives the workgroup
+    __builtin_amdgcn_s_waitcnt(0);  // no fetch into LDS outlives the pass
+    if constexpr (LONG) {
+        kc0 += Kl;
+        if (kc0 >= K) break;
+        Kl = min(K - kc0, Kc);
+        __builtin_amdgcn_s_barrier();  // every partial is read before the slots hold x again
+    } else {
+        break;
+    }
+    }
 }
 
 
@@ -1355,17 +1387,15 @@ template <int SW, int PACK, bool STW = false>
 __global__ __launch_bounds__(STW ? 576 : 512) void matvec_q8_ksplit_kernel(
     const uint32_t* __restrict__ weight, const float* __restrict__ scale, const float* __restrict__ x,
     float* __restrict__ y, uint32_t N, uint32_t K, uint32_t W, uint32_t M) {
-    ksplit_body<SW, PACK, STW>(KsOne{weight, scale, y, N}, x, K, W, M);
+    ksplit_body<SW, PACK, STW, false>(KsOne{weight, scale, y, N}, x, K, W, M, K);
 }
 
 // Several projections of the same vectors in one launch.
-template <int SW, int PACK>
+template <int SW, int PACK, bool LONG = false>
 __global__ __launch_bounds__(512) void matvec_q8_ksplit_multi_kernel(KsSeveral p, const float* __restrict__ x,
-                                                                    uint32_t K, uint32_t W, uint32_t M) {
-    ksplit_body<SW, PACK, false>(p, x, K, W, M);
+                                                                    uint32_t K, uint32_t W, uint32_t M, uint32_t Kc) {
+    ksplit_body<SW, PACK, false, LONG>(p, x, K, W, M, Kc);
 }
-
-constexpr uint32_t kKsLdsBytes = kKsWaves * kKsStages * 16u * 128u + 2u * kKsGroup * kKsWaves * 1024u;
 
 // ---------------------------------------------------------------------------
 // Host-side dispatch.
@@ -1576,7 +1606,7 @@ hipError_t launch_ksplit(const MatvecArgs& a, const DeviceInfo& dev, hipStream_t
     return hipGetLastError();
 }
 
-template <int SW, int PACK>
+template <int SW, int PACK, bool LONG = false>
 hipError_t launch_ksplit_multi(const Projection* p, uint32_t count, const float* x, uint32_t K, uint32_t M,
                                const DeviceInfo& dev, hipStream_t stream, Variant* variant) {
     constexpr uint32_t VPB = ks_vectors<PACK>();
@@ -1594,14 +1624,18 @@ hipError_t launch_ksplit_multi(const Projection* p, uint32_t count, const float*
     several.t0[kMaxProjections] = tiles;
     const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
     const dim3 grid = ks_grid(tiles, (M + VPB - 1u) / VPB, cus);
-    hipLaunchKernelGGL((matvec_q8_ksplit_multi_kernel<SW, PACK>), grid, dim3(512), kKsLdsBytes, stream, several,
-                       x, K, (uint32_t)(((uint64_t)K + 3) / 4), M);
+    // LONG: the fewest passes, of even length in whole 1024s
+    const uint32_t passes = (K + 1024u * SW - 1u) / (1024u * SW);
+    const uint32_t Kc = (K + 1024u * passes - 1u) / (1024u * passes) * 1024u;
+    const uint32_t lds = kKsLdsBytes + (LONG ? (tiles + grid.x - 1u) / grid.x * 1024u : 0u);
+    hipLaunchKernelGGL((matvec_q8_ksplit_multi_kernel<SW, PACK, LONG>), grid, dim3(512), lds, stream, several,
+                       x, K, (uint32_t)(((uint64_t)K + 3) / 4), M, Kc);
     set_variant(variant, "matvec_q8_ksplit.multi", PACK == 1 ? "x16" : "x8", (int)kKsWaves, 16, SW,
                 (int)(M < VPB ? M : VPB), grid.x, grid.y);
     return hipGetLastError();
 }
 
-// Batched, 768 < K <= 4096: codes split across a workgroup's waves, x parts in
+// Batched, K > 768: codes split across a workgroup's waves, x parts in
 // VGPRs (every wave busy from K > 896; at K = 512 half of them would idle and
 // the kernels below win).  Its cost is one pass per round of one workgroup per
 // CU (4.2, 6.0, 7.9, 9.5 us at K = 1024, 2048, 3072, 4096 with 8 vectors, about
@@ -1616,7 +1650,21 @@ hipError_t launch_ksplit_multi(const Projection* p, uint32_t count, const float*
 // Up to 4096 rows at 1024 < K <= 2048 (and past 16 vectors at K <= 1024) the VALU
 // instances keep the calls that they had: their names are checked for there.
 bool ksplit_pays(uint64_t N, uint32_t K, uint32_t M, const DeviceInfo& dev) {
-    if (K <= 768u || K > 4096u || (M + 15u) / 16u > 65535u) return false;
+    if (K <= 768u || (M + 15u) / 16u > 65535u) return false;
+    if (K > 4096u) {
+        // Passes of at most 3072 codes; each tile's sums take 1 KiB of LDS between
+        // them.  A pass is a fixed cost per round, the VALU path's the operations
+        // (VALU -> k-split, us): vectors x rows x codes 8 x 5632 x 5632 21.8 -> 17.2,
+        // 5 x 8192 x 5632 24.7 -> 16.9, 16 x 4096 x 4160 24.0 -> 19.9, 12 x 4096 x
+        // 8192 33.5 -> 27.3, 8 x 32000 x 8192 135 -> 57.5; below the line 8 x 4096 x
+        // 11008 28.8 -> 32.2, 16 x 2048 x 5632 16.5 -> 18.9, 16 x 1000 x 20000 47.7 -> 61.3.
+        if (M < 5u || K > 65536u) return false;
+        const uint64_t cus = (uint64_t)(dev.cu_count > 0 ? dev.cu_count : 256), tiles = (N + 15u) / 16u;
+        const uint64_t groups = (M + 15u) / 16u, gx = ks_grid((uint32_t)tiles, (uint32_t)groups, (uint32_t)cus).x;
+        if (kKsLdsBytes + (tiles + gx - 1u) / gx * 1024u > kMfmaLdsBytes) return false;
+        const uint64_t ops = N * K * (M + (M + 7u) / 8u), passes = (K + 3071u) / 3072u;
+        return ops >= passes * 125000000u;
+    }
     if (K > 2048u) {
         const bool three = K <= 3072u;
         const uint64_t ops = N * (M + (M + 7u) / 8u);
@@ -1677,6 +1725,10 @@ hipError_t launch_matvec_q8(const MatvecArgs& a, const DeviceInfo& dev, hipStrea
     }
     if (a.M == 1) return dispatch_m1<kEpiPlain>(a, dev, stream, variant);
     if (ksplit_pays(a.N, a.K, a.M, dev)) {
+        if (a.K > 4096u) {
+            const Projection one = {a.weight, a.scale, a.output, a.N};
+            return launch_matvec_q8_batched_multi(&one, 1u, a.vector, a.K, a.M, dev, stream, variant);
+        }
         if (a.K > 3072u) {
             if (a.M <= 5u) return launch_ksplit<4, 3>(a, dev, stream, variant);
             if (a.M <= 8u) return launch_ksplit<4, 2>(a, dev, stream, variant);
@@ -1787,7 +1839,9 @@ bool matvec_q8_batched_multi_pays(const Projection* p, uint32_t count, uint32_t 
 
 hipError_t launch_matvec_q8_batched_multi(const Projection* p, uint32_t count, const float* x, uint32_t K, uint32_t M,
                                           const DeviceInfo& dev, hipStream_t stream, Variant* variant) {
-    if (count == 0u || count > kMaxProjections || K <= 768u || K > 4096u) return hipErrorInvalidValue;
+    if (count == 0u || count > kMaxProjections || K <= 768u || K > 65536u) return hipErrorInvalidValue;
+    if (K > 4096u) return M <= 8u ? launch_ksplit_multi<3, 2, true>(p, count, x, K, M, dev, stream, variant)
+                                  : launch_ksplit_multi<3, 1, true>(p, count, x, K, M, dev, stream, variant);
     if (K > 3072u) return M <= 8u ? launch_ksplit_multi<4, 2>(p, count, x, K, M, dev, stream, variant)
                                   : launch_ksplit_multi<4, 1>(p, count, x, K, M, dev, stream, variant);
     if (K > 2048u) return M <= 8u ? launch_ksplit_multi<3, 2>(p, count, x, K, M, dev, stream, variant)
