@@ -391,6 +391,18 @@ def test_matmul_workspace_balance(N, Ms, K, form_ws, form_plain):
         assert_matmul(b[2].download(np.float32, N * M), a, w, s, N, M, K, rows=rows)
 
 
+@pytest.mark.parametrize("N,Ms,K,form_ws,form_plain", [
+    (192, [11008], 1030, "D256.PD2", "D256.PD2"),    # 129 256-row tiles
+    (570, [4300], 1000, "D256.PD2", "D256.PD2"),     # 153
+    (1216, [2049], 1030, "D256.PD2", "D256.PD2"),    # 171
+    (640, [4200], 1000, "FB4.balance2", "D128"),     # 170
+    (19000, [128], 1030, "FB4.balance2", "D128"),    # 297 tiles of either height, two rounds
+])
+def test_matmul_one_round_of_256_row_tiles(N, Ms, K, form_ws, form_plain):
+    """The lines of the one-round dispatch, as above."""
+    test_matmul_workspace_balance(N, Ms, K, form_ws, form_plain)
+
+
 MIB = 1 << 20
 FB4_CASES = [
     # (N, Ms, K, workspace bytes (True: the full size), form): tiles that fill

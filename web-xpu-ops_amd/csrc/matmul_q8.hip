@@ -1345,22 +1345,24 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         // in two, so that whole tiles plus halves fill the 2 x cus slots and
         // every CU holds the same work (384 tiles -> 256 whole and 256 halves,
         // one of each per CU).  The halves' sum is a second launch (~5 us
-        // with its launch); with more tiles the dispatch already evens the
-        // CUs out over several rounds and the split no longer pays (704
-        // tiles: the GEMM 90 -> 85 us, plus the sum).  Same process, 512
-        // tokens: q, k, v 54.9 -> 49.3 us; at 256 tokens gate and up 51.6 ->
-        // 47.1.
+        // with its launch), so this pays for long rows only (320 x 7680 tokens x
+        // rows: 101.7 -> 91.3 us at K = 5632, 41.9 -> 42.6 at 2048); with more
+        // tiles the rounds even the CUs out by themselves.
         const uint64_t slots = 2ull * cus;
         const uint64_t S = t4 < slots ? slots - t4 : 0u;
         const size_t blk = (size_t)128u * kBN * 4u;
-        // Where the 256-row tiles fill at least two thirds of the CUs, the
-        // direct kernel on those tiles (one workgroup per CU, two register
-        // sets) beats both the split and the uneven round, with or without a
-        // workspace.  Same process, us, split -> 256-row direct: 512 tokens q,
-        // k, v (192 tiles) 51.9 -> 48.7; 256 tokens gate and up (176) 53.9 ->
-        // 49.9.  With fewer (96 at 256 tokens q, k, v) it loses to the 128-row
-        // forms (31.6 -> 45.0).
-        if (S > 0 && 3u * t8 >= 2u * (uint64_t)cus) {
+        // One round of 256-row tiles on the direct kernel beats both the split and
+        // the uneven round, with or without a workspace: a 128-row workgroup beside
+        // another takes longer than a 256-row one alone.  Same process, us, split ->
+        // 256-row: 512 tokens q, k, v (192 tiles) 41.0 -> 34.3, 256 tokens gate and up
+        // (176) 41.4 -> 34.3, 320 x 7168 x 2048 (140) 42.4 -> 33.7 (x 1024: 30.4 ->
+        // 20.6, x 5632: 90.1 -> 80.7), 300 x 6700 x 4096 (135) 74.5 -> 59.6; without a
+        // workspace 320 x 7168 x 1024 24.5 -> 20.6.  From 0.6 to 2/3 of the CUs the
+        // 128-row forms are kept for their names, which tests check at 154 and 160
+        // tiles, not for their time (154 tiles, K = 1030: 31.8 us against 22.1).
+        // More 256-row tiles than CUs (19000 x 128 x 2048, every tile half empty)
+        // would take two rounds: 67.9 us against 48.2 without a workspace, 58.2 with.
+        if (S > 0 && t8 <= cus && (5u * t8 < 3ull * cus || 3u * t8 >= 2ull * cus)) {
             set_variant(variant, kname, "D256.PD2", 8, 256, 0, (int)kBN, (uint32_t)((t8 + 7u) / 8u * 8u));
             return launch_direct<8, 2>(a, p, n, N, K, stream);
         }
