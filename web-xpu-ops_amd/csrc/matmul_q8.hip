@@ -1254,7 +1254,7 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // projection.  The GEMM walks all of K in a serial chain of steps per
     // workgroup whatever the token count (20 us for 1 token at 2048 x 2048);
     // the batched path streams the weight once per 8 or 16 tokens (3.6 us
-    // for 1 token, 10.5 us for 32; the GEMM wins from about 64 tokens).
+    // for 1 token, 7.0 us for 32).
     // Both compute the matvecQ8 form.
     Projection pv[kMaxMatmulProjections];
     for (uint32_t i = 0; i < n; ++i) pv[i] = Projection{p[i].weight, p[i].scale, p[i].output, p[i].M};
@@ -1370,16 +1370,10 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
             set_variant(variant, kname, "FB4.balance2", 4, 128, 0, (int)kBN, (uint32_t)(t4 + S));
             return launch_direct<4, 2, 1, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)S, 2u);
         }
-        // Long rows whose tiles make two or more whole rounds of two per CU:
-        // one workgroup of 16 waves per two consecutive tiles of the sequence,
-        // one per K group.  Same process, one-group -> pairs (us, measured
-        // with a token-major tile sequence): 1024 tiles
-        // at K = 4096 240-245 -> 226-232, at K = 11008 645-647 -> 607-612 and
-        // 334-338 -> 300-302, at K = 5632 299-317 -> 290-323; one round (512
-        // tiles) even, and 5.5 rounds (2816 tiles, K = 4096) 658 -> 686-690,
-        // where two workgroups per CU even out the last half round better;
-        // at K = 2048 no gain.  The same sums in the same order as the
-        // one-group form.
+        // Long rows whose 128-row tiles make two or more whole rounds of two per CU
+        // where 256-row ones do not: one workgroup of 8 waves per two consecutive
+        // tiles of the sequence, 4 waves each (65536 tokens x 128 x 4096: 231.9 ->
+        // 228.4 us).  The same sums in the same order as the one-group form.
         if (K >= 4096u && t4 >= 4ull * cus && t4 % (2ull * cus) == 0) {
             set_variant(variant, kname, "FB4.pairs", 8, 128, 0, (int)kBN, (uint32_t)((t4 / 2u + 7u) / 8u * 8u));
             return launch_direct<4, 2, 2, kTilePairs>(a, p, n, N, K, stream);
@@ -1396,11 +1390,10 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // With a workspace, 256-row tiles on the direct kernel with every tile's
     // K steps split into 4 or 8 parts, one workgroup each, when that fills
     // more than 7/8 of the CUs with at least 11 steps per part (the parts
-    // meet in split_sum_kernel).  Same box, us, against the two-K-group forms
-    // the dispatch took before: 512 tokens down 50.0 -> 47.1 (4 parts of 22
-    // steps), 256 tokens down 31.6 -> 30.2 (8 parts of 11); with 8 or 4 steps
-    // per part the split's second launch costs more than it saves (o, K =
-    // 2048: 24.6 -> 26.2 at 512 tokens, 19.6 -> 20.6 at 256).
+    // meet in split_sum_kernel).  Same process, us, against the forms below: 512
+    // tokens x 2048 x 5632 38.9 -> 36.3 (4 parts of 22 steps), 256 tokens 24.6 ->
+    // 25.0 (8 parts of 11: even); with fewer steps per part the split's second
+    // launch costs more than it saves.
     for (uint32_t xs : {4u, 8u}) {
         const size_t blk = (size_t)256u * kBN * 4u;
         if (workspace && t8 * xs <= cus && 8u * t8 * xs > 7u * cus && steps >= 11u * xs &&
@@ -1410,12 +1403,10 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
             return launch_direct<8, 2, 1, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)t8, xs);
         }
     }
-    // 128-row tiles that fill most of the CUs, one per CU with two K groups,
-    // beat smaller tiles that fill them all: a 128-row tile moves ~19 bytes
-    // through LDS per output and step against ~27 for 64 rows and ~45 for
-    // 32.  Same process, µs: 128 tokens gate and up (176 tiles) 38.6 -> 32.0,
-    // 256 tokens q, k, v (192 tiles) 38.9 -> 33.2; with 128 tiles (half the
-    // CUs) they lose (512 tokens o: 29.6 -> 31.4, one box and process).
+    // 128-row tiles that fill most of the CUs, one per CU with two K groups of 4
+    // waves on the direct kernel, beat smaller tiles that fill them all.  Same
+    // process, us, against the 64-row form: 128 tokens gate and up (176 tiles) 32.5 ->
+    // 24.8, 256 tokens q, k, v (192) 31.7 -> 24.8, 320 x 5120 x 2048 (200) 32.2 -> 24.9.
     if (5u * t4 >= 3u * cus) {
         set_variant(variant, kname, "FB4.ksplit2", 8, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
         return launch_direct<4, 2, 2>(a, p, n, N, K, stream);
@@ -1423,11 +1414,8 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // With a workspace, 128-row tiles whose K steps split in 2 or 4 fill
     // (nearly) every CU, as long as each K group keeps at least 10 steps
     // (the split's second launch and every part's pipeline start cost a few
-    // us): 512 tokens down 55.8 -> 49.9 us (2 parts, 22 steps per group), 256
-    // tokens down 40.2 -> 31.1 (4 parts, 11 steps).  Fewer workgroups than
-    // 7/8 of the CUs, or shorter runs, lose to the smaller tiles below (512
-    // tokens o in 2 parts of 8 steps per group: 21.9 -> 26.0; 128 tokens q, k,
-    // v in 2 parts on 3/4 of the CUs: 21.8 -> 23.9).
+    // us): 512 tokens x 2048 x 2560 25.8 -> 24.7 us (2 parts, 10 steps per group)
+    // against the 64-row form.
     for (uint32_t xs : {4u, 2u}) {
         const size_t blk = (size_t)128u * kBN * 4u;
         if (workspace && t4 * xs <= cus && 8u * t4 * xs > 7u * cus && steps >= 20u * xs &&
