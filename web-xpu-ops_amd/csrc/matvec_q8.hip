@@ -1299,7 +1299,10 @@ __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restr
         if (b0 + ti < b1 && col_ok && sel == 0u) {
             const KsTile tl = src.tile(b0 + ti, W);
             float* yo = tl.y + (size_t)(m0 + vj) * tl.N + 4u * g;
-            const bool whole = 4u * g + 3u < tl.rows;
+            // rows from this lane's first on (4 g + q against the row count would
+            // be kept in registers through the loop, and the longest rows' form spill)
+            const int left = (int)tl.rows - (int)(4u * g);
+            const bool whole = left > 3;
             f32x4 o;
 #pragma unroll
             for (int q = 0; q < 4; ++q) o[q] = sum[q] * __uint_as_float(rsc[q]);
@@ -1308,7 +1311,7 @@ __device__ __forceinline__ void ksplit_body(const Src& src, const float* __restr
             } else {
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    if (4u * g + (uint32_t)q < tl.rows) yo[q] = o[q];
+                    if (q < left) yo[q] = o[q];
             }
         }
     };
