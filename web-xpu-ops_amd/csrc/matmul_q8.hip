@@ -660,13 +660,16 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
     // Epilogue: lane (j, g) of block (f, b) holds features m0 + wm + 16 f +
     // 4 g .. +3 of token n0 + wn + 16 b + j.  A split tile stores unscaled
     // sums: part 0 into the output, part xs into its workspace block.
+    // The lane group is read again: kept from the start it costs the 64-row form on
+    // two K groups (128 registers a lane) a spill.
+    const uint32_t ge = __lane_id() >> 4;
     const bool split = SPLIT && tile >= P.whole;
     const __amdgpu_buffer_rsrc_t srs = make_rsrc(scale + m0, split ? 0u : mrows * 4u);
     float* const blk = SPLIT && xs > 0u
         ? P.part + ((size_t)(xs - 1u) * P.splits + (tile - P.whole)) * (size_t)(BM * kBN) : nullptr;
 #pragma unroll
     for (int f = 0; f < FW; ++f) {
-        const uint32_t fm = wm + 16u * (uint32_t)f + 4u * g;  // within the tile
+        const uint32_t fm = wm + 16u * (uint32_t)f + 4u * ge;  // within the tile
         const u32x4v sv = split ? u32x4v{0x3f800000u, 0x3f800000u, 0x3f800000u, 0x3f800000u}  // 1.0f
                                 : __builtin_amdgcn_raw_buffer_load_b128(srs, (int)(fm * 4u), 0, 0);
 #pragma unroll
