@@ -848,6 +848,10 @@ def test_matmul_activations_past_the_f16_window(N, M, K, ws):
     (77, [1000, 1, 530], 769, "x16.ksplit2"),
     (140, [4080], 3073, "x16.ksplit2"),                         # 255 tiles, nine passes
     (4096, [100], 1024, "x16.ksplit2"),                         # a pass per CU
+    (48, [4096], 512, "x16.ksplit2"),                           # 3 tile passes per CU, half of the waves without codes
+    (48, [4097], 512, "FB1.PD4.ksplit2"),                       # one more
+    (40, [1000, 33], 767, "x16.ksplit2"),
+    (40, [1000], 511, "FB1.PD4.ksplit2"),
 ])
 def test_matmul_tokens_on_the_ksplit_kernel(N, Ms, K, form):
     """Short prompts on the batched k-split kernel: several projections in one
@@ -879,3 +883,29 @@ def test_matmul_tokens_on_the_ksplit_kernel(N, Ms, K, form):
         assert_bits_equal(again, got, "repeat")
         assert np.all(got[N * M:] == np.float32(7.5)), f"M={M}: written past the output"
         assert_matmul(got[:N * M], a, w, s, N, M, K, rows=rows)
+
+
+@pytest.mark.parametrize("N,M,K,ws", [
+    (100, 4096, 300, False),   # 32-row tiles, a ragged token tile
+    (70, 2048, 5000, False),   # the same past four folds
+    (40, 300, 2100, True),     # K split between workgroups
+    (300, 2048, 520, False),   # 64-row tiles
+])
+def test_matmul_tokens_of_many_scales(N, M, K, ws):
+    """Neighbouring groups of tokens up to 2^90 apart: the short prompts'
+    tiles scale each group of 8 by its own power of two.  Every token within
+    the matmulQ8 bar, under weight scales that keep the sums above its floor."""
+    rng = np.random.default_rng(N + M + K)
+    a = rng.standard_normal((N, K)).astype(np.float32)
+    a *= np.ldexp(np.float32(1), 45 * ((np.arange(N) // 4) % 3) - 45).astype(np.float32)[:, None]
+    w = random_packed(rng, M, K)
+    s = rng.uniform(1e10, 1e11, M).astype(np.float32)
+    ba, bw, bs = (wxo_q8.DeviceBuffer.from_array(v) for v in (a.reshape(-1), w, s))
+    out = wxo_q8.DeviceBuffer(4 * N * M)
+    nbytes = wxo_q8.matmul_q8_workspace_bytes() if ws else 0
+    work = wxo_q8.DeviceBuffer(nbytes) if ws else None
+    wxo_q8.matmul_q8_multi_device(ba, [(bw, bs, out, M)], N, K, workspace=work, workspace_bytes=nbytes)
+    wxo_q8.synchronize()
+    assert "FB" in wxo_q8.last_variant(), wxo_q8.last_variant()
+    rows = np.unique(np.r_[np.arange(0, N, 5), N - 1])
+    assert_matmul(out.download(np.float32, N * M), a, w, s, N, M, K, rows=rows)

@@ -82,7 +82,7 @@ struct Projection {
 };
 hipError_t launch_matvec_q8_multi(const Projection* projections, uint32_t count, const float* x, uint32_t K,
                                   const DeviceInfo& dev, hipStream_t stream, Variant* variant);
-// The same for M vectors x [M, K] (output_p [M, N_p]) on the k-split kernel, 768 <
+// The same for M vectors x [M, K] (output_p [M, N_p]) on the k-split kernel, 512 <=
 // K <= 65536; _pays: whether that beats one call per projection (M >= 5).
 bool matvec_q8_batched_multi_pays(const Projection* projections, uint32_t count, uint32_t K, uint32_t M,
                                   const DeviceInfo& dev);

@@ -235,7 +235,8 @@ __device__ __forceinline__ bool store_split(const uint32_t (&v)[8], float least,
     return bad;
 }
 
-// The tile's power of two, from the sum of |x| over its first 64 x 64
+// The tile's power of two (in matmul_q8_kernel its 8-token groups', which come
+// with 8 times their sums), from the sum of |x| over its first 64 x 64
 // activations: their mean lands in [2^6, 2^7), which leaves 2^9 of it above
 // and 2^-22 below before a step takes the slow form.  All zero or not finite:
 // no scaling.  Every power stays far from the f32 range's ends.
@@ -393,7 +394,7 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     // [step][wave]: nonzero, the wave's tokens of the step are slow_step's
     __shared__ __attribute__((aligned(8))) uint8_t flags[KS][kFlagSteps][8];
-    __shared__ float abssum[KS][8];
+    __shared__ float downs[KS][8];  // the inverse power of two of each wave's 8 tokens
 
     // XCD-aware tile order: workgroup i runs on XCD i % 8; give each XCD a
     // contiguous run of the tile sequence (tile_coords).  A split launch
@@ -496,7 +497,7 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
             v[4 * q + 3] = gb[s][q].w;
         }
     };
-    float up = 1.0f, down = 1.0f;  // the tile's power of two and its inverse
+    float up = 1.0f, down = 1.0f;  // the power of two of this wave's 8 tokens and its inverse
     const float least = btok < ntok ? kPartMin : 0.0f;
     // Writes the converted step into stage st.
     auto convert_store = [&](int s, int st, uint32_t step) {
@@ -584,18 +585,19 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
     for (int q = 0; q < PD; ++q) issue(q, (s0 + (uint32_t)q) * kBK);
     if (ragged && s0 + 1u == steps) mask_b(0, s0 * kBK);
     {
-        // the power of two of this group's run, from its first step
+        // Each wave's 8 tokens have a power of two of their own, from the run's
+        // first step: one for the whole tile met at a barrier and a second
+        // reduction before the first conversion (150 x 2048 x 512 8.0 us, 7.5 so;
+        // 512 x 2048 x 520 12.2 -> 12.0).
         uint32_t v[FPT];
         load_b(0, v);
         float m = 0.0f;
 #pragma unroll
         for (int e = 0; e < (int)FPT; ++e) m += __builtin_fabsf(__uint_as_float(v[e]));
-        m = wave_sum(m);
-        if (lane == 0u) abssum[kg][wv] = m;
-        __syncthreads();
-        const int e = part_exponent(wave_sum(lane < 8u ? abssum[kg][lane] : 0.0f));
+        const int e = part_exponent(wave_sum(m) * 8.0f);
         up = pow2f(e);
         down = pow2f(-e);
+        if (lane == 0u) downs[kg][wv] = down;
     }
     convert_store(0, 0, 0u);
     issue(0, (s0 + (uint32_t)PD) * kBK);
@@ -628,7 +630,7 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
         for (int f = 0; f < FW; ++f)
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
-                fold(sum[f][b], acc[f][b], accl[f][b], down);
+                fold(sum[f][b], acc[f][b], accl[f][b], downs[kg][(wn >> 3) + 2u * (uint32_t)b + (j >> 3)]);
             }
         if (g0 < gs) slow_steps<FW, TB>(flags[kg], wrs, ars, wm, wn, rowbytes, K, s0, g0, min(gend, gs) - g0, [&](int f, int b, f32x4 v) { sum[f][b] += v; });
     }
@@ -1308,11 +1310,15 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // -> 15.3, 256 x 2048 17.4 -> 15.9, 96 x 6144 19.5 -> 18.1 (9 tile passes per CU);
     // past 9 it loses (80 x 8192 19.7 -> 20.8, 160 x 4096 19.7 -> 21.1).  The same
     // line at K = 1024 (64 x 6144 11.7 -> 8.9) and 4096 (64 x 6144 28.7 -> 20.9).
+    // At 512 to 768 codes some of its waves idle and the tiles have few steps: up to
+    // 3 tile passes per CU (40 x 2048 x 520 7.7 -> 6.5, 40 x 4096 x 520 8.4 -> 8.0, x
+    // 768 9.7 -> 7.9; past it 150 x 2048 x 520 8.6 -> 9.9).
     // The forms split through a workspace stay where they apply.
     const uint64_t passes = (N + 15u) / 16u;
     uint64_t t16 = 0;
     for (uint32_t i = 0; i < n; ++i) t16 += (p[i].M + 15ull) / 16u;
-    if (!split4 && !split2 && K > 768u && K <= 4096u && passes <= cus && t16 * passes <= 9ull * cus) {
+    if (!split4 && !split2 && K >= 512u && K <= 4096u && passes <= cus &&
+        t16 * passes <= (K > 768u ? 9ull : 3ull) * cus) {
         const hipError_t e = launch_matvec_q8_batched_multi(pv, n, a, K, N, dev, stream, variant);
         if (variant && e == hipSuccess) {
             variant->kernel = kname;

@@ -1842,7 +1842,7 @@ bool matvec_q8_batched_multi_pays(const Projection* p, uint32_t count, uint32_t 
 
 hipError_t launch_matvec_q8_batched_multi(const Projection* p, uint32_t count, const float* x, uint32_t K, uint32_t M,
                                           const DeviceInfo& dev, hipStream_t stream, Variant* variant) {
-    if (count == 0u || count > kMaxProjections || K <= 768u || K > 65536u) return hipErrorInvalidValue;
+    if (count == 0u || count > kMaxProjections || K < 512u || K > 65536u) return hipErrorInvalidValue;
     if (K > 4096u) return M <= 8u ? launch_ksplit_multi<3, 2, true>(p, count, x, K, M, dev, stream, variant)
                                   : launch_ksplit_multi<3, 1, true>(p, count, x, K, M, dev, stream, variant);
     if (K > 3072u) return M <= 8u ? launch_ksplit_multi<4, 2>(p, count, x, K, M, dev, stream, variant)
