@@ -637,9 +637,9 @@ def cpu_reference_ops(budget_s):
 def run_prefill_suite(stream, steps, warmup, results, check):
     """The prefill side (the next rows after the decode path): matmulQ8 over
     one decoder layer's seven projections for a 512-token prompt, then the
-    dequant / gather ops.  matmulQ8 is compute-bound: its bound is the bf16
-    matrix-core rate at three products per code (the exact split of each
-    activation), i.e. 3 x 2 N M K flops; TFLOP/s counts the 2 N M K useful
+    dequant / gather ops.  matmulQ8 is compute-bound: its bound is the f16
+    matrix-core rate (bf16's) at two products per code (each activation an
+    f16 pair), i.e. 2 x 2 N M K flops; TFLOP/s counts the 2 N M K useful
     flops."""
     L = wxo_q8.lib()
     sp = stream.handle
@@ -665,15 +665,15 @@ def run_prefill_suite(stream, steps, warmup, results, check):
         us = time_loop(stream, lambda i: check(L.wxo_matmul_q8(a.ptr, packed.ptr, scale.ptr, out.ptr, T, N, K, sp)),
                        max(1, steps // 20), max(1, warmup // 20))  # 25+ us per call: never host-bound
         flops = 2.0 * T * N * K
-        bound_us = 3.0 * flops / (PEAK_BF16_MFMA_TFLOPS * 1e12) * 1e6
+        bound_us = 2.0 * flops / (PEAK_BF16_MFMA_TFLOPS * 1e12) * 1e6
         total_flops += flops
         total_us += us
         results.append({"case": f"prefill matmulQ8 {name}: tokens={T} M={N} K={K}", "us": round(us, 3),
-                        "TFLOP/s": round(flops / (us * 1e-6) / 1e12, 1), "bound": "mfma_bf16 (x3 exact split)",
+                        "TFLOP/s": round(flops / (us * 1e-6) / 1e12, 1), "bound": "mfma_f16 (x2: activations in f16 pairs)",
                         "pct_of_bound": round(100 * bound_us / us, 1)})
         log(f"suite prefill matmulQ8 {name} {T}x{N}x{K}: {us:.2f} us  {flops / (us * 1e-6) / 1e12:.1f} TFLOP/s  "
-            f"{100 * bound_us / us:.1f}% of the x3 bf16 bound")
-    bound_us = 3.0 * total_flops / (PEAK_BF16_MFMA_TFLOPS * 1e12) * 1e6
+            f"{100 * bound_us / us:.1f}% of the x2 f16 bound")
+    bound_us = 2.0 * total_flops / (PEAK_BF16_MFMA_TFLOPS * 1e12) * 1e6
     results.append({"case": f"prefill matmulQ8: one decoder layer's 7 projections, {T} tokens", "us": round(total_us, 3),
                     "TFLOP/s": round(total_flops / (total_us * 1e-6) / 1e12, 1),
                     "pct_of_bound": round(100 * bound_us / total_us, 1)})
@@ -741,7 +741,7 @@ def run_prefill_suite(stream, steps, warmup, results, check):
     results.append({"case": f"prefill matmulQ8: one decoder layer, {TL} tokens, as the resident batch issues it "
                             f"(4 launches)", "us": round(long_us, 3),
                     "TFLOP/s": round(long_flops / (long_us * 1e-6) / 1e12, 1),
-                    "pct_of_bound": round(100 * 3.0 * long_flops / (PEAK_BF16_MFMA_TFLOPS * 1e12) * 1e6 / long_us, 1),
+                    "pct_of_bound": round(100 * 2.0 * long_flops / (PEAK_BF16_MFMA_TFLOPS * 1e12) * 1e6 / long_us, 1),
                     "variants": variants})
     log(f"suite prefill layer, {TL} tokens, coalesced: {long_us:.1f} us  {long_flops / (long_us * 1e-6) / 1e12:.1f} "
         f"TFLOP/s")
