@@ -671,6 +671,34 @@ def test_matmul_tile_pairs(N, Ms, K):
         assert_matmul(got[:N * M], a, w, s, N, M, K, rows=rows)
 
 
+@pytest.mark.parametrize("N,Ms,K", [(2048, [6144], 4096), (1024, [12288], 4099), (2030, [4096, 4096], 4096)])
+def test_matmul_long_rows_take_the_larger_tiles(N, Ms, K):
+    """Launches of several rounds of the CUs over long rows, whose 128-row tiles
+    could run in pairs but whose larger tiles cost less (768, 768 and 1024 tiles
+    of 256 rows): 384-row workgroups.  Every 97th token against the oracle,
+    nothing past the outputs."""
+    rng = np.random.default_rng(N + sum(Ms) + K)
+    a = rng.standard_normal(N * K).astype(np.float32)
+    a[3 * K + 5] = np.inf
+    ba = wxo_q8.DeviceBuffer.from_array(a)
+    host, bufs = [], []
+    for M in Ms:
+        w = random_packed(rng, M, K)
+        s = rng.uniform(0.001, 0.05, M).astype(np.float32)
+        out = wxo_q8.DeviceBuffer(4 * (N * M + 64))
+        out.upload(np.full(N * M + 64, 7.5, np.float32))
+        host.append((w, s, M))
+        bufs.append((wxo_q8.DeviceBuffer.from_array(w), wxo_q8.DeviceBuffer.from_array(s), out, M))
+    wxo_q8.matmul_q8_multi_device(ba, bufs, N, K)
+    wxo_q8.synchronize()
+    assert " rows=384 " in wxo_q8.last_variant(), wxo_q8.last_variant()
+    rows = np.unique(np.r_[np.arange(0, N, 97), 3, N - 1])
+    for (w, s, M), (_, _, out, _) in zip(host, bufs):
+        got = out.download(np.float32, N * M + 64)
+        assert np.all(got[N * M:] == np.float32(7.5)), f"M={M}: written past the output"
+        assert_matmul(got[:N * M], a, w, s, N, M, K, rows=rows)
+
+
 def test_matmul_tile_pairs_ragged_tokens_match_one_group():
     """Tile pairs with a partial last token tile (N = 2040: 31 whole 64-token
     tiles and one of 56) over two projections (2176 and 1920 rows: 17 + 15

@@ -1380,10 +1380,13 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
             return launch_direct<4, 2, 1, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)S, 2u);
         }
         // Long rows whose 128-row tiles make two or more whole rounds of two per CU
-        // where 256-row ones do not: one workgroup of 8 waves per two consecutive
-        // tiles of the sequence, 4 waves each (65536 tokens x 128 x 4096: 231.9 ->
-        // 228.4 us).  The same sums in the same order as the one-group form.
-        if (K >= 4096u && t4 >= 4ull * cus && t4 % (2ull * cus) == 0) {
+        // where 256-row ones make neither whole rounds nor 2.75 of them: one
+        // workgroup of 8 waves per two consecutive tiles of the sequence, 4 waves
+        // each.  The same sums in the same order as the one-group form.
+        // Past that line the larger tiles are faster (us, pairs -> 384-row): 4096 x 4096
+        // x 4096 367 -> 281, 2048 x 8192 x 4096 356 -> 274, 1024 x 12288 x 4096 263 ->
+        // 191; below it the two are even at K = 4096 (1024 x 8192: 174, 176).
+        if (K >= 4096u && t4 >= 4ull * cus && t4 % (2ull * cus) == 0 && t8 % cus != 0 && 4u * t8 < 11ull * cus) {
             set_variant(variant, kname, "FB4.pairs", 8, 128, 0, (int)kBN, (uint32_t)((t4 / 2u + 7u) / 8u * 8u));
             return launch_direct<4, 2, 2, kTilePairs>(a, p, n, N, K, stream);
         }
