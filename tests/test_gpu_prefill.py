@@ -10,6 +10,7 @@
   * dequantizePackedQ8, dequantTranspose, gatherDequantRows: bit-exact
     (ops/dequant_transpose/wgsl.test.ts:37 holds its kernel to rel 0, abs 0).
 """
+import ctypes
 import json
 import math
 import os
@@ -832,11 +833,12 @@ def test_matmul_weight_past_4_gib():
     (510, 11200, 330, False),  # 384-row tiles
 ])
 def test_matmul_activations_past_the_f16_window(N, M, K, ws):
-    """Activations that the scaled f16 pair does not hold (large, tiny,
+    """Activations that no one scaled f16 pair holds together (large, tiny,
     subnormal and infinite ones among ordinary ones, and a token tile of tiny
-    ones only) take the exact three-part split.  A third of the weight rows
-    see the tiny ones alone (their other codes are 0), under scales that make
-    those sums of order 1, so the matmulQ8 bar is relative to them."""
+    ones only).  A third of the weight rows see the tiny ones alone (their
+    other codes are 0), under scales that make those sums of order 1, so the
+    matmulQ8 bar is relative to them: they are taken again from the exact
+    three-part split."""
     rng = np.random.default_rng(N + M + K)
     a = rng.standard_normal((N, K)).astype(np.float32)
     tiny = rng.choice(K, 24, replace=False)
@@ -937,3 +939,116 @@ def test_matmul_tokens_of_many_scales(N, M, K, ws):
     assert "FB" in wxo_q8.last_variant(), wxo_q8.last_variant()
     rows = np.unique(np.r_[np.arange(0, N, 5), N - 1])
     assert_matmul(out.download(np.float32, N * M), a, w, s, N, M, K, rows=rows)
+
+
+@pytest.mark.parametrize("N,M,K,ws", [
+    (65, 2048, 300, False),    # 32-row tiles, one token in the second tile
+    (40, 300, 4500, True),     # the same, K split between workgroups
+    (300, 2048, 500, False),   # 64-row tiles, two K groups
+    (379, 2860, 300, False),   # the same, one group
+    (450, 4096, 300, False),   # 128-row tiles, two K groups
+    (19000, 128, 1030, True),  # 128-row tiles, the last ones' K steps split
+    (577, 6100, 1030, False),  # 256-row tiles
+    (510, 11200, 2061, False), # 384-row tiles
+])
+def test_matmul_activations_that_grow(N, M, K, ws):
+    """Tokens whose largest values come late: their powers of two fall during the
+    run, at steps of their own.  Some tokens are zero at first or throughout, some
+    start with an infinity or a NaN; some weight rows have no code at all, or only
+    codes at the small first values (under scales that make those sums of order
+    1)."""
+    rng = np.random.default_rng(N + M + K)
+    a = rng.standard_normal((N, K)).astype(np.float32)
+    first = min(K // 2, 64 * 3)
+    a *= np.ldexp(np.float32(1), 9 * (np.arange(K)[None, :] * 7 // K + np.arange(N)[:, None]) % 80 - 40).astype(np.float32)
+    small = np.sort(rng.choice(first, 24, replace=False))
+    a[:, small] = rng.standard_normal((N, 24)).astype(np.float32) * np.float32(1e-13)
+    a[4::16, :first] = 0          # nothing but zeros in the first steps
+    a[9::32] = 0
+    a[1, 3], a[2, 5], a[3, K - 1] = np.inf, np.nan, -np.inf
+    a[N - 1, K // 2] = np.float32(1e34)
+    codes = rng.integers(-128, 128, (M, K)).astype(np.int32)
+    lone = np.arange(M) % 5 == 0
+    codes[np.ix_(lone, np.setdiff1d(np.arange(K), small))] = 0
+    codes[3::40] = 0
+    s = rng.uniform(0.001, 0.05, M).astype(np.float32)
+    s[lone] = np.float32(1e11)
+    w = oracle.pack_q8(codes.reshape(-1), M, K)
+    ba, bw, bs = (wxo_q8.DeviceBuffer.from_array(v) for v in (a.reshape(-1), w, s))
+    out = wxo_q8.DeviceBuffer(4 * N * M)
+    nbytes = wxo_q8.matmul_q8_workspace_bytes() if ws else 0
+    work = wxo_q8.DeviceBuffer(nbytes) if ws else None
+    wxo_q8.matmul_q8_multi_device(ba, [(bw, bs, out, M)], N, K, workspace=work, workspace_bytes=nbytes)
+    wxo_q8.synchronize()
+    print(wxo_q8.last_variant(), flush=True)
+    assert wxo_q8.last_variant().startswith("matmul_q8 "), wxo_q8.last_variant()
+    rows = np.unique(np.r_[np.arange(0, min(N, 64), 3), np.arange(0, N, 1 + N // 24), 1, 2, 3, 4, 9, N - 1])
+    assert_matmul(out.download(np.float32, N * M), a, w, s, N, M, K, rows=rows)
+
+
+@pytest.mark.parametrize("N,M,K", [(100, 4096, 300), (512, 6100, 1030), (510, 11200, 1030)])
+def test_matmul_tokens_do_not_depend_on_each_other(N, M, K):
+    """A token's sums keep their bits whatever its neighbours hold."""
+    rng = np.random.default_rng(N + M + K)
+    a = rng.standard_normal((N, K)).astype(np.float32)
+    b = a.copy()
+    b[::8] *= np.ldexp(np.float32(1), rng.integers(-60, 60, (b[::8].shape[0], 1))).astype(np.float32)
+    b[::8, 7::64] = 1e30
+    w = random_packed(rng, M, K)
+    s = rng.uniform(0.001, 0.05, M).astype(np.float32)
+    bw, bs = wxo_q8.DeviceBuffer.from_array(w), wxo_q8.DeviceBuffer.from_array(s)
+    got = []
+    for x in (a, b):
+        out = wxo_q8.DeviceBuffer(4 * N * M)
+        wxo_q8.matmul_q8_multi_device(wxo_q8.DeviceBuffer.from_array(x.reshape(-1)), [(bw, bs, out, M)], N, K)
+        wxo_q8.synchronize()
+        got.append(out.download(np.float32, N * M).reshape(N, M))
+    kept = np.arange(N) % 8 != 0
+    assert_bits_equal(got[1][kept].reshape(-1), got[0][kept].reshape(-1), "tokens beside changed ones")
+
+
+def test_matmul_time_does_not_depend_on_the_values():
+    """The same launch over activations of many kinds takes about the same time:
+    GELU and wide SiLU outputs (values of every size down to 1e-30), one large value
+    in every token, nothing but zeros in the first codes, one token of 64 alone.
+    The bar is far above the spread between runs and below what any of these cost
+    where such values took a path of their own (1.6 to 5.7 times)."""
+    N, M, K = 2048, 2048, 5632
+    rng = np.random.default_rng(1)
+    normal = rng.standard_normal((N, K)).astype(np.float32)
+    from scipy.special import erf, expit
+    other = rng.standard_normal((N, K)).astype(np.float32)
+    kinds = {"normal": normal, "gelu": (1.5 * normal * (1 + erf(3 * normal / np.sqrt(2)))).astype(np.float32),
+             "silu": (6 * normal * expit(6 * normal) * other).astype(np.float32)}
+    kinds["outliers"] = normal.copy()
+    kinds["outliers"][np.arange(N), rng.integers(0, K, N)] = 1000
+    kinds["late"] = normal * np.float32(1e-6)
+    kinds["late"][:, :64] = 0
+    kinds["lone"] = (normal * expit(normal) * other).astype(np.float32)
+    kinds["lone"][np.arange(N) % 64 != 0] = 0
+    w = random_packed(rng, M, K)
+    bw, bs = wxo_q8.DeviceBuffer.from_array(w), wxo_q8.DeviceBuffer.from_array(np.full(M, 0.01, np.float32))
+    out = wxo_q8.DeviceBuffer(4 * N * M)
+    L, stream = wxo_q8.lib(), wxo_q8.Stream()
+    start, stop = ctypes.c_void_p(), ctypes.c_void_p()
+    assert L.wxo_event_create_timer(ctypes.byref(start)) == 0 and L.wxo_event_create_timer(ctypes.byref(stop)) == 0
+    us = {}
+    for name, a in kinds.items():
+        ba = wxo_q8.DeviceBuffer.from_array(a.reshape(-1))
+        times = []
+        for _ in range(6):
+            assert L.wxo_event_record(start, stream.handle) == 0
+            for _ in range(5):
+                wxo_q8.matmul_q8_multi_device(ba, [(bw, bs, out, M)], N, K, stream=stream)
+            assert L.wxo_event_record(stop, stream.handle) == 0
+            stream.synchronize()
+            ms = ctypes.c_float()
+            assert L.wxo_event_elapsed_ms(ctypes.byref(ms), start, stop) == 0
+            times.append(ms.value * 200)
+        us[name] = sorted(times)[2]
+        ba.free()
+    L.wxo_event_destroy(start)
+    L.wxo_event_destroy(stop)
+    print(us, flush=True)
+    for name, t in us.items():
+        assert t < 1.5 * us["normal"], us

@@ -12,18 +12,25 @@
 // inside the 1e-5 bar the tests hold.
 //
 // Numerics on the f16 matrix cores: a code q in [-128, 127] is exact in f16;
-// an activation, scaled by a power of two of its run's, becomes a pair of f16 h
-// + l / 2048 (split2: exact to 2^-23 of it over 30 binades), every product
-// q * part is exact in f32, and v_mfma_f32_16x16x32_f16 sums the two planes in
-// two f32 accumulators.  Each 1024-code slice of K is summed there (32
-// accumulations a plane) and then folded into an outer f32 sum, so no rounding
-// chain exceeds 32 + K/1024 steps.  Values outside the 30 binades (infinite,
-// past 65504 after the scale, or nonzero and under 2^-16) flag their step, and
-// their products come from an exact three-part bf16 split instead (slow_steps),
-// so every f32 activation is taken as precisely as before.  Against 64 bits,
-// 2-norm: 1.69e-7 at K = 2048 to 5632, where three bf16 parts in one
-// accumulator (96 accumulations per fold) had 3.1e-7; and a third less matrix
-// work, LDS traffic and splitting.
+// an activation, scaled by its token's power of two, becomes a pair of f16 h +
+// l / 2048, every product q * part is exact in f32, and
+// v_mfma_f32_16x16x32_f16 sums the two planes in two f32 accumulators.  Each
+// 1024-code slice of K is summed there (32 accumulations a plane) and then
+// folded into an outer f32 sum, so no rounding chain exceeds 32 + K/1024 steps.
+// Against 64 bits, 2-norm: 1.7e-7 at K = 2048 to 5632, where three bf16 parts
+// in one accumulator (96 accumulations per fold) had 3.1e-7; and a third less
+// matrix work, LDS traffic and splitting.
+//
+// What the pair holds of one activation: 2^-23 of it at worst (two 11-bit parts
+// and the sign between them: a quarter of all f32 values lose their last bit)
+// from 2^-22 of the token's largest value up, and 2^-45 of the largest one below
+// (the parts turn subnormal).  A token's power of two starts from its first 64
+// codes and falls when a larger value comes (rescale_split): the waves multiply
+// their accumulators by the ratio, exactly, so the time hardly depends on the
+// values and a token's sums depend on no other token.  The values below that
+// window only matter to a weight row that has no code at the larger ones:
+// small_sums takes sums that are small enough for it again, from an exact
+// three-part bf16 split.
 //
 // Tiling (matmul_q8_kernel, short prompts): a workgroup of two K groups of 8
 // waves (2 over the weight rows x 4 over the tokens) owns BM = 32 FB weight
@@ -66,6 +73,7 @@
 // only the activation pairs pass through LDS.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "kernels.hpp"
 #include "wave_ops.hpp"
@@ -181,80 +189,130 @@ __device__ __forceinline__ uint32_t piece_offset(uint32_t p, uint32_t row) {
     return ((((p & 1u) << 2) | (p >> 1)) ^ (row & 7u)) * 16u;
 }
 
-// Two activations -> their f16 pairs.  t = x * 2^s (s the tile's, exact), h =
-// f16(t) and l = f16(2048 (t - h)), both rounded to nearest: t - h is exact,
-// so h + l / 2048 is t to 2^-23 of it while h is a normal f16, i.e. for
-// 2^-14 <= |t| <= 65504, and to 2^-20 from 2^-16 up.  lo and hi collect the
-// smallest and largest |t|.
+// Two activations -> their f16 pairs.  t = x * up (up the token's power of two,
+// exact), h = f16(t) and l = f16(2048 (t - h)), both rounded to nearest: t - h is
+// exact, so h + l / 2048 is t to 2^-23 of it for 2^-13 <= |t| <= 65504, and to
+// 2^-36 below.  hi collects the largest |t|.
 constexpr float kPartScale = 2048.0f;
-constexpr float kPartMin = 1.52587890625e-05f;  // 2^-16
 constexpr float kPartMax = 65504.0f;
-__device__ __forceinline__ void split2(float x0, float x1, float up, uint32_t& h, uint32_t& l, float& lo, float& hi) {
+__device__ __forceinline__ void split2(float x0, float x1, float up, uint32_t& h, uint32_t& l, float& hi) {
     const float t0 = x0 * up, t1 = x1 * up;
     const f16x2 hp = __builtin_convertvector((f32x2v){t0, t1}, f16x2);
     const float r0 = __builtin_fmaf(x0, up, -(float)hp.x), r1 = __builtin_fmaf(x1, up, -(float)hp.y);
     const f16x2 lp = __builtin_convertvector((f32x2v){r0 * kPartScale, r1 * kPartScale}, f16x2);
     h = __builtin_bit_cast(uint32_t, hp);
     l = __builtin_bit_cast(uint32_t, lp);
-    lo = __builtin_fminf(__builtin_fminf(__builtin_fabsf(t0), __builtin_fabsf(t1)), lo);
     hi = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(t0), __builtin_fabsf(t1)), hi);
 }
 
-// True (wave-uniform) if the wave holds a value that its pair does not
-// represent: infinite, past 65504 or, not being 0, under 2^-16 after the scale
-// (lo and hi as split2 collected them over v; least: 2^-16, or 0 for a token
-// past the tile's, whose values are all 0).  Such a wave writes zeros and
-// flags the step, and slow_steps adds its tokens' products from the exact
-// three-part split.  NaNs stay: their token's sums are NaN either way.
-__device__ __forceinline__ bool needs_slow(const uint32_t (&v)[8], float least, float down, float lo, float hi) {
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(lo >= least && hi <= kPartMax)) == 0, 1)) return false;
-    // zeros also read as too small: tell them apart (2 |bits| - 1 wraps for 0)
-    uint32_t small = 0xffffffffu;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) small = min(small, (v[e] << 1) - 1u);
-    const bool bad = small < (__float_as_uint(kPartMin * down) << 1) - 1u || !(hi <= kPartMax);
-    return __builtin_amdgcn_ballot_w64(bad) != 0;
+// A token's power of two 2^(127 - c) stands as the byte c, the exponent field of
+// its inverse.  c = kNoValue: nothing above 2^-113 seen yet.
+constexpr uint32_t kNoValue = 1u;
+constexpr int kTopExponent = 9;  // a new power takes the largest value to [2^9, 2^10): 64 to 128 times of room
+__device__ __forceinline__ float up_of(uint32_t c) { return __uint_as_float((254u - c) << 23); }
+__device__ __forceinline__ float down_of(uint32_t c) { return __uint_as_float(c << 23); }
+__device__ __forceinline__ uint32_t code_of(float up) { return 254u - (__float_as_uint(up) >> 23); }
+
+// The power of two for a token whose largest value is `most`.
+__device__ __forceinline__ float up_for(float most) {
+    const int c = (int)(__float_as_uint(most) >> 23) - kTopExponent;
+    return up_of(c > (int)kNoValue ? (uint32_t)c : kNoValue);
 }
 
-// Eight consecutive activations of one token -> `w` and `w + plane` in LDS
-// (zeros where the step needs slow_steps, which is returned; written over the
-// pairs, so that the conversion stays free of the branch).
-__device__ __forceinline__ bool store_split(const uint32_t (&v)[8], float least, float up, float down, uint8_t* w,
-                                            uint32_t plane) {
-    uint32_t hp[4], lp[4];
-    float lo = kPartMax, hi = 0.0f;
+// The largest of a token's values (not negative) over its 8 lanes.
+__device__ __forceinline__ float token_max(float v) {
+    uint32_t b = __float_as_uint(v);
+    b = max(b, partner_u32<1>(b));
+    b = max(b, partner_u32<2>(b));
+    return __uint_as_float(max(b, partner_u32<4>(b)));
+}
+
+// A token's first power of two, from its first 64 activations (an infinity among
+// them leaves it to rescale_split).
+__device__ __forceinline__ float first_up(const uint32_t (&v)[8]) {
+    float most = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) split2(__uint_as_float(v[2 * e]), __uint_as_float(v[2 * e + 1]), up, hp[e], lp[e], lo, hi);
+    for (int e = 0; e < 8; ++e) most = __builtin_fmaxf(most, __builtin_fabsf(__uint_as_float(v[e])));
+    most = token_max(most);
+    return most <= 3.402823466e38f ? up_for(most) : up_of(kNoValue);
+}
+
+// True (wave-uniform) if a value of the wave passes its token's window.
+__device__ __forceinline__ bool past_window(float hi) {
+    return __builtin_amdgcn_ballot_w64(!(hi <= kPartMax)) != 0;
+}
+
+// Then the pairs again, written over the first ones so that the conversion stays
+// free of the branch (and under the matrix work): a token (8 lanes side by side)
+// whose largest finite value passes 65504 gets its new power of two, and an
+// infinity is h itself, beside l = 0.
+__device__ __forceinline__ void rescale_split(const uint32_t (&v)[8], float& up, uint8_t* w, uint32_t plane) {
+    uint32_t hp[4], lp[4];
+    float most = 0.0f, hi = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const uint32_t b = v[e] & 0x7fffffffu;
+        most = __builtin_fmaxf(most, b == 0x7f800000u ? 0.0f : __uint_as_float(b));
+    }
+    most = token_max(most);
+    if (most * up > kPartMax) up = up_for(most);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t a = v[2 * e], b = v[2 * e + 1];
+        const bool ai = (a & 0x7fffffffu) == 0x7f800000u, bi = (b & 0x7fffffffu) == 0x7f800000u;
+        split2(ai ? 0.0f : __uint_as_float(a), bi ? 0.0f : __uint_as_float(b), up, hp[e], lp[e], hi);
+        if (ai) hp[e] |= 0x7c00u | ((a >> 16) & 0x8000u);
+        if (bi) hp[e] |= 0x7c000000u | (b & 0x80000000u);
+    }
     *reinterpret_cast<u32x4v*>(w) = u32x4v{hp[0], hp[1], hp[2], hp[3]};
     *reinterpret_cast<u32x4v*>(w + plane) = u32x4v{lp[0], lp[1], lp[2], lp[3]};
-    const bool bad = needs_slow(v, least, down, lo, hi);
-    if (bad) {
-        *reinterpret_cast<u32x4v*>(w) = u32x4v{0u, 0u, 0u, 0u};
-        *reinterpret_cast<u32x4v*>(w + plane) = u32x4v{0u, 0u, 0u, 0u};
+}
+
+// What the converting waves tell the others of a K group, for the last four
+// steps: [step][8 tokens] whether a power of two may have changed at the step,
+// and then (at step 0 always) the tokens' codes.
+struct TokenScales {
+    uint8_t changed[4][8];
+    uint8_t code[4][kBN];
+};
+
+// The pairs of a wave's 8 tokens, 8 activations v a lane, are in LDS at `w` and
+// `w + plane`, the largest of them hi: makes them again if one passes its token's
+// window, and notes that for step `step`.
+__device__ __forceinline__ void settle(const uint32_t (&v)[8], float hi, float& up, uint8_t* w, uint32_t plane,
+                                       TokenScales& sc, uint32_t step, uint32_t token) {
+    const bool out = past_window(hi);
+    if (__builtin_expect(out, 0)) {
+        rescale_split(v, up, w, plane);
+        sc.code[step % 4u][token] = (uint8_t)code_of(up);  // the token's 8 lanes alike
     }
-    return bad;
+    if (__lane_id() == 0u) sc.changed[step % 4u][token >> 3] = out ? 1u : 0u;
 }
 
-// The tile's power of two (in matmul_q8_kernel its 8-token groups', which come
-// with 8 times their sums), from the sum of |x| over its first 64 x 64
-// activations: their mean lands in [2^6, 2^7), which leaves 2^9 of it above
-// and 2^-22 below before a step takes the slow form.  All zero or not finite:
-// no scaling.  Every power stays far from the f32 range's ends.
-__device__ __forceinline__ int part_exponent(float abssum) {
-    const int e = (int)((__float_as_uint(abssum) >> 23) & 0xffu);
-    if (e == 0 || e == 0xff) return 0;
-    const int s = 6 + 12 - (e - 127);  // the mean is abssum / 2^12
-    return s > 100 ? 100 : (s < -100 ? -100 : s);
+// Eight consecutive activations of one token -> their pairs in LDS.
+__device__ __forceinline__ void store_split(const uint32_t (&v)[8], float& up, uint8_t* w, uint32_t plane,
+                                            TokenScales& sc, uint32_t step, uint32_t token) {
+    uint32_t hp[4], lp[4];
+    float hi = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split2(__uint_as_float(v[2 * e]), __uint_as_float(v[2 * e + 1]), up, hp[e], lp[e], hi);
+    *reinterpret_cast<u32x4v*>(w) = u32x4v{hp[0], hp[1], hp[2], hp[3]};
+    *reinterpret_cast<u32x4v*>(w + plane) = u32x4v{lp[0], lp[1], lp[2], lp[3]};
+    settle(v, hi, up, w, plane, sc, step, token);
 }
-__device__ __forceinline__ float pow2f(int s) { return __uint_as_float((uint32_t)(127 + s) << 23); }
 
-__device__ __forceinline__ float wave_sum(float v) {
-    v += partner_f32<1>(v);
-    v += partner_f32<2>(v);
-    v += partner_f32<4>(v);
-    v += partner_f32<8>(v);
-    v = swap_add<16>(v, v);
-    return swap_add<32>(v, v);
+// The first step's, with the tokens' first powers of two and their codes.
+__device__ __forceinline__ void store_first(const uint32_t (&v)[8], float& up, uint8_t* w, uint32_t plane,
+                                            TokenScales& sc, uint32_t token) {
+    up = first_up(v);
+    store_split(v, up, w, plane, sc, 0u, token);
+    sc.code[0][token] = (uint8_t)code_of(up);
+}
+
+// The accumulators' factor when a token's code goes from `was` to `now` (>= was).
+__device__ __forceinline__ float scale_ratio(uint32_t was, uint32_t now) {
+    const int e = 127 + (int)was - (int)now;
+    return __uint_as_float((uint32_t)(e > 1 ? e : 1) << 23);  // never 0: an infinite sum stays infinite
 }
 
 // Three bf16 parts of an activation, exactly, whatever its exponent: h keeps
@@ -272,56 +330,34 @@ __device__ __forceinline__ void split3_any(uint32_t bits, uint32_t& h, uint32_t&
     l = __float_as_uint(r - __uint_as_float(m));
 }
 
-// One 64-code step of a wave's FW x TB blocks for the tokens whose converting
-// wave flagged it: `groups` bit i stands for the tile's tokens 8 i .. 8 i + 7.
-// Codes and activations come straight from memory, in the operand's k order,
-// the activations split in three; other tokens' values count as 0, so adding
-// the products (add(f, b, block)) completes the step whatever the other waves found.
-template <int FW, int TB, typename Add>
-__device__ __forceinline__ void slow_step(__amdgpu_buffer_rsrc_t wrs, __amdgpu_buffer_rsrc_t ars, uint32_t wm,
-                                          uint32_t wn, uint32_t rowbytes, uint32_t K, uint32_t k0, uint32_t groups,
-                                          Add&& add) {
-    const uint32_t lane = threadIdx.x & 63u, j = lane & 15u, g = lane >> 4;
-#pragma unroll 1
-    for (int h = 0; h < 2; ++h) {
-        const uint32_t k = k0 + 16u * g + 8u * (uint32_t)h;
+// 0 for a block's sums, and infinity for those of rows past the tile's, which
+// small_sums then leaves alone (they are not stored).
+__device__ __forceinline__ f32x4 no_sums(uint32_t row, uint32_t mrows) {
+    f32x4 s;
 #pragma unroll
-        for (int b = 0; b < TB; ++b) {
-            const uint32_t tk = wn + 16u * (uint32_t)b + j;
-            if (((groups >> ((wn >> 3) + 2u * (uint32_t)b)) & 3u) == 0u) continue;  // uniform
-            const bool mine = ((groups >> (tk >> 3)) & 1u) != 0u;
-            uint32_t x[8], hp[4], mp[4], lp[4];
-            const u32x4v x0 = __builtin_amdgcn_raw_buffer_load_b128(ars, (int)((tk * K + k) * 4u), 0, 0);
-            const u32x4v x1 = __builtin_amdgcn_raw_buffer_load_b128(ars, (int)((tk * K + k) * 4u + 16u), 0, 0);
-            x[0] = x0.x; x[1] = x0.y; x[2] = x0.z; x[3] = x0.w;
-            x[4] = x1.x; x[5] = x1.y; x[6] = x1.z; x[7] = x1.w;
+    for (uint32_t v = 0; v < 4u; ++v) s[v] = row + v < mrows ? 0.0f : __builtin_inff();
+    return s;
+}
+
+// Steps between folds of a run of `steps`: kFoldCodes' worth, and half of a run
+// that is no longer than that (in whole multiples of U), for smallest_of.  Only
+// where the sums are in registers: the second fold of sums in LDS costs what the
+// sums taken again do (1098 x 7216 x 896 52.1 us with it, 51.8 without).
+template <uint32_t U>
+__device__ __forceinline__ uint32_t fold_steps(uint32_t steps) {
+    constexpr uint32_t full = kFoldCodes / 64u;
+    return steps > full ? full : ((steps + 1u) / 2u + U - 1u) / U * U;
+}
+
+// min(least, |now|) over a block's sums, or of the larger of |was| and |now|: for
+// small_sums, a sum after the last fold and, where there are two, before it
+// (either shows that its products are large enough, so that then next to none is
+// small by cancellation).
+__device__ __forceinline__ float smallest_of(f32x4 was, f32x4 now, bool two, float least) {
+    float m[4];
 #pragma unroll
-            for (uint32_t e = 0; e < 8u; ++e)
-                if (!mine || k + e >= K) x[e] = 0u;
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                uint32_t h0, m0, l0, h1, m1, l1;
-                split3_any(x[e], h0, m0, l0);
-                split3_any(x[e + 1], h1, m1, l1);
-                hp[e / 2] = hi_pair(h0, h1);
-                mp[e / 2] = hi_pair(m0, m1);
-                lp[e / 2] = hi_pair(l0, l1);
-            }
-            const bf16x8 bh = __builtin_bit_cast(bf16x8, u32x4v{hp[0], hp[1], hp[2], hp[3]});
-            const bf16x8 bm = __builtin_bit_cast(bf16x8, u32x4v{mp[0], mp[1], mp[2], mp[3]});
-            const bf16x8 bl = __builtin_bit_cast(bf16x8, u32x4v{lp[0], lp[1], lp[2], lp[3]});
-#pragma unroll
-            for (int f = 0; f < FW; ++f) {
-                const bf16x8 af = codes8_to_bf16(__builtin_bit_cast(u32x2v, __builtin_amdgcn_raw_buffer_load_b64(
-                    wrs, (int)((wm + 16u * (uint32_t)f + j) * rowbytes + k), 0, 0)));
-                f32x4 p = f32x4{0.f, 0.f, 0.f, 0.f};
-                p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bh, p, 0, 0, 0);
-                p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bm, p, 0, 0, 0);
-                p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bl, p, 0, 0, 0);
-                add(f, b, p);
-            }
-        }
-    }
+    for (int v = 0; v < 4; ++v) m[v] = two ? __builtin_fmaxf(__builtin_fabsf(was[v]), __builtin_fabsf(now[v])) : __builtin_fabsf(now[v]);
+    return __builtin_fminf(__builtin_fminf(__builtin_fminf(m[0], m[1]), __builtin_fminf(m[2], m[3])), least);
 }
 
 // sum += (acc + accl / 2048) * down, and both accumulators start again.
@@ -335,30 +371,130 @@ __device__ __forceinline__ void fold(f32x4& sum, f32x4& acc, f32x4& accl, float 
     accl = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-// The flagged steps among the `count` steps from step `first` (a fold group's,
-// at most 16): `flags` holds a byte per step of the last 32 and converting
-// wave.  Rare, and once a fold group so that the step loop carries no code or
-// registers for it.
-constexpr uint32_t kFlagSteps = 2u * kFoldCodes / 64u;
-template <int FW, int TB, typename Add>
-__device__ __forceinline__ void slow_steps(const uint8_t (&flags)[kFlagSteps][8], __amdgpu_buffer_rsrc_t wrs,
+// The sums of a wave's FW x TB blocks over its run of `gs` steps from step s0,
+// where the pairs might not hold what they came from.  A pair is off by 2^-36 /
+// up at most where it is off by more than 2^-23 of its value, so a sum of n
+// products by 128 n 2^-36 / up: less than 2^-17 of the sum of the products'
+// sizes unless that is below n 2^-12 / up.  A sum that is not that small itself
+// passes; the others (about one in 10^7 of an ordinary prompt's, by
+// cancellation) are taken again here, straight from memory with the activations
+// in three exact parts, until the products' sizes add up to enough, which the
+// first step shows, or to the end: rows whose only codes meet values far below
+// the token's largest.  smallest[b]: the lane's smallest_of its token b;
+// code(b): that token's code; get and put: a block's sums.
+template <int FW, int TB, typename Code, typename Get, typename Put>
+__device__ __forceinline__ void small_sums(const float (&smallest)[TB], __amdgpu_buffer_rsrc_t wrs,
                                            __amdgpu_buffer_rsrc_t ars, uint32_t wm, uint32_t wn, uint32_t rowbytes,
-                                           uint32_t K, uint32_t s0, uint32_t first, uint32_t count, Add&& add) {
-    const uint32_t lane = threadIdx.x & 63u, step = lane >> 1;
-    const uint32_t fl = step < count ? reinterpret_cast<const uint32_t*>(flags[(first + step) % kFlagSteps])[lane & 1u] : 0u;
-    uint64_t left = __builtin_amdgcn_ballot_w64(fl != 0u);
-#pragma unroll 1
-    while (left != 0u) {  // wave-uniform
-        const int st = __builtin_ctzll(left) >> 1;
-        left &= ~(3ull << (2 * st));
-        uint32_t groups = 0u;
+                                           uint32_t K, uint32_t s0, uint32_t gs, Code&& code, Get&& get, Put&& put) {
+    const uint32_t lane = __lane_id(), j = lane & 15u, g = lane >> 4;
+    // n 2^-12 / up, and 0 for a token without values (down_of(c - 1) is half of down_of(c) but for c = 1)
+    const float per = (float)(gs * 64u) * 0.00048828125f;
+    const auto least_of = [&](int b) { return per * down_of(code(b) - kNoValue); };
+    bool any = false;
 #pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)fl, 2 * st + w);
+    for (int b = 0; b < TB; ++b) any |= smallest[b] < least_of(b);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any) == 0, 1)) return;
+    uint32_t todo = 0u;  // bit f * TB + b: the block has such a sum
 #pragma unroll
-            for (int q = 0; q < 4; ++q) groups |= ((v >> (8 * q)) & 1u) << (4 * w + q);
+    for (int f = 0; f < FW; ++f)
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            const f32x4 y = get(f, b);
+            const float least = least_of(b);
+            bool small = false;
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                small |= __builtin_fabsf(y[v]) < least;
+            todo |= __builtin_amdgcn_ballot_w64(small) != 0 ? 1u << (f * TB + b) : 0u;
         }
-        slow_step<FW, TB>(wrs, ars, wm, wn, rowbytes, K, (s0 + first + (uint32_t)st) * 64u, groups, add);
+#pragma unroll 1
+    while (todo != 0u) {  // wave-uniform
+        const uint32_t at = (uint32_t)__builtin_ctz(todo);
+        todo &= todo - 1u;
+        f32x4 y = {0.f, 0.f, 0.f, 0.f};
+        float least = 0.0f;
+#pragma unroll
+        for (int i = 0; i < FW * TB; ++i)
+            if (at == (uint32_t)i) {
+                y = get(i / TB, i % TB);
+                least = least_of(i % TB);
+            }
+        const uint32_t row0 = wm + 16u * (at / (uint32_t)TB);
+        const uint32_t tk = wn + 16u * (at % (uint32_t)TB) + j;
+        uint32_t left = 0u;  // bit v: sum v of the lane is to be taken again
+#pragma unroll
+        for (uint32_t v = 0; v < 4u; ++v)
+            left |= (__builtin_fabsf(y[v]) < least ? 1u : 0u) << v;
+        f32x4 size = {0.f, 0.f, 0.f, 0.f}, part = size, total = size;
+#pragma unroll 1
+        for (uint32_t st = 0; st < gs; ++st) {
+            const uint32_t k0 = (s0 + st) * 64u + 16u * g;
+            uint32_t x[16];
+            u32x2v w[2];
+#pragma unroll
+            for (uint32_t q = 0; q < 4u; ++q) {
+                const u32x4v t = __builtin_amdgcn_raw_buffer_load_b128(ars, (int)((tk * K + k0 + 4u * q) * 4u), 0, 0);
+                x[4u * q] = t.x; x[4u * q + 1u] = t.y; x[4u * q + 2u] = t.z; x[4u * q + 3u] = t.w;
+            }
+#pragma unroll
+            for (uint32_t h = 0; h < 2u; ++h)
+                w[h] = __builtin_bit_cast(u32x2v, __builtin_amdgcn_raw_buffer_load_b64(
+                    wrs, (int)((row0 + j) * rowbytes + k0 + 8u * h), 0, 0));
+#pragma unroll
+            for (uint32_t e = 0; e < 16u; ++e)
+                if (k0 + e >= K) x[e] = 0u;  // the next token's
+#pragma unroll
+            for (uint32_t h = 0; h < 2u; ++h) {
+                uint32_t hp[4], mp[4], lp[4];
+#pragma unroll
+                for (uint32_t e = 0; e < 4u; ++e) {
+                    uint32_t h0, m0, l0, h1, m1, l1;
+                    split3_any(x[8u * h + 2u * e], h0, m0, l0);
+                    split3_any(x[8u * h + 2u * e + 1u], h1, m1, l1);
+                    hp[e] = hi_pair(h0, h1);
+                    mp[e] = hi_pair(m0, m1);
+                    lp[e] = hi_pair(l0, l1);
+                }
+                const bf16x8 q = codes8_to_bf16(w[h]);
+                const u32x4v qa = __builtin_bit_cast(u32x4v, q) & 0x7fff7fffu, xa = u32x4v{hp[0], hp[1], hp[2], hp[3]} & 0x7fff7fffu;
+                size = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, qa), __builtin_bit_cast(bf16x8, xa), size, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q, __builtin_bit_cast(bf16x8, u32x4v{hp[0], hp[1], hp[2], hp[3]}), part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q, __builtin_bit_cast(bf16x8, u32x4v{mp[0], mp[1], mp[2], mp[3]}), part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q, __builtin_bit_cast(bf16x8, u32x4v{lp[0], lp[1], lp[2], lp[3]}), part, 0, 0, 0);
+            }
+            if (st % (kFoldCodes / 64u) == kFoldCodes / 64u - 1u || st + 1u == gs) {
+                total += part;
+                part = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (uint32_t v = 0; v < 4u; ++v)
+                if (size[v] >= least) left &= ~(1u << v);
+            if (st == 0u && __builtin_amdgcn_ballot_w64(left != 0u) != 0) {
+                // rows without any code need not be walked to the end
+                uint32_t any = 0u;
+#pragma unroll 4
+                for (uint32_t q = 0; q < gs; ++q) {
+                    const uint32_t k = (s0 + q) * 64u + 16u * g;
+                    const u32x4v c = __builtin_amdgcn_raw_buffer_load_b128(wrs, (int)((row0 + j) * rowbytes + k), 0, 0);
+#pragma unroll
+                    for (uint32_t e = 0; e < 4u; ++e) any |= k + 4u * e < rowbytes ? c[e] : 0u;
+                }
+                uint64_t rows = __builtin_amdgcn_ballot_w64(any != 0u);
+                rows |= rows >> 32;
+                rows |= rows >> 16;
+                left &= (uint32_t)rows >> (4u * g);  // row 4 g + v of the block
+            }
+            if (__builtin_amdgcn_ballot_w64(left != 0u) == 0) break;
+        }
+#pragma unroll
+        for (int i = 0; i < FW * TB; ++i)
+            if (at == (uint32_t)i) {
+                f32x4 z = y;
+#pragma unroll
+                for (uint32_t v = 0; v < 4u; ++v)
+                    if ((left >> v) & 1u) z[v] = total[v];
+                put(i / TB, i % TB, z);
+            }
     }
 }
 
@@ -368,13 +504,12 @@ __device__ __forceinline__ void slow_steps(const uint8_t (&flags)[kFlagSteps][8]
 // a long prompt, which would leave some CUs with one tile more than others).
 // The other instances run every tile whole, with no branch on it.
 template <int FB, int NW, int BK, int PD, int KS, bool SPLIT = false>
-__global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __restrict__ a, MatmulProjections P,
+__global__ __launch_bounds__(64 * NW * KS, 4) void matmul_q8_kernel(const float* __restrict__ a, MatmulProjections P,
                                                         uint32_t N, uint32_t K, uint32_t W, uint32_t mtiles,
                                                         uint32_t ntiles) {
     constexpr uint32_t BM = 32u * FB;                 // weight rows per workgroup
     constexpr uint32_t kBK = (uint32_t)BK;            // codes per K step
     constexpr uint32_t kRowBytes = kBK * 2u;          // one LDS row: BK f16
-    constexpr uint32_t kFoldSteps = kFoldCodes / kBK;
     constexpr uint32_t CPR = kBK / 16u;               // 16-code chunks per row and step
     constexpr uint32_t AST = BM * kRowBytes;          // bytes of one A stage
     constexpr uint32_t BST = 2u * kBN * kRowBytes;    // bytes of one B stage (two planes)
@@ -388,13 +523,10 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
     constexpr int FW = (int)(BM / (16u * WR));         // 16-row blocks per wave
     static_assert(NW == 8 && BK == 64, "a wave converts 8 tokens of a 64-code step, 8 activations a thread");
     static_assert(PD == 2 || PD == 4, "2 or 4 register sets of loads in flight");
-    static_assert(kFoldSteps % (uint32_t)PD == 0u, "a fold group starts on register set 0 and stage 0");
     static_assert(KS == 1 || KS == 2, "K split over 1 or 2 groups of NW waves");
     // Per K group: [A0 A1 B0 B1]
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    // [step][wave]: nonzero, the wave's tokens of the step are slow_step's
-    __shared__ __attribute__((aligned(8))) uint8_t flags[KS][kFlagSteps][8];
-    __shared__ float downs[KS][8];  // the inverse power of two of each wave's 8 tokens
+    __shared__ __attribute__((aligned(8))) TokenScales scales[KS];
 
     // XCD-aware tile order: workgroup i runs on XCD i % 8; give each XCD a
     // contiguous run of the tile sequence (tile_coords).  A split launch
@@ -497,10 +629,9 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
             v[4 * q + 3] = gb[s][q].w;
         }
     };
-    float up = 1.0f, down = 1.0f;  // the power of two of this wave's 8 tokens and its inverse
-    const float least = btok < ntok ? kPartMin : 0.0f;
+    float up = up_of(kNoValue);  // the power of two of this thread's token
     // Writes the converted step into stage st.
-    auto convert_store = [&](int s, int st, uint32_t step) {
+    auto convert_store = [&](int s, int st, uint32_t step, auto first) {
         uint8_t* as = lds + gbase + (uint32_t)st * AST;
 #pragma unroll
         for (int u = 0; u < AL; ++u) {
@@ -514,8 +645,8 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
         uint32_t v[FPT];
         load_b(s, v);
         uint8_t* row = lds + gbase + 2u * AST + (uint32_t)st * BST + btok * kRowBytes + piece_offset(bc, btok);
-        const bool bad = store_split(v, least, up, down, row, kBN * kRowBytes);
-        if (lane == 0u) flags[kg][step % kFlagSteps][wv] = bad ? 1u : 0u;
+        if constexpr (first) store_first(v, up, row, kBN * kRowBytes, scales[kg], btok);
+        else store_split(v, up, row, kBN * kRowBytes, scales[kg], step, btok);
     };
 
     const uint32_t steps = (K + kBK - 1u) / kBK;
@@ -538,40 +669,63 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
             sum[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 
-    // Matrix work of one stage: two 32-code halves, lane group g taking codes
-    // 16 g + 8 h .. +7 of the step in half h (the sum's k order is free; this
-    // one is the direct kernel's, whose lanes load 16 consecutive codes).
-    auto compute = [&](int s) {
+    // Operands of half h (32 codes) of a stage: lane group g takes codes 16 g + 8 h
+    // .. +7 of the step (the sum's k order is free; this one is the direct
+    // kernel's, whose lanes load 16 consecutive codes).
+    auto operands = [&](int s, int h, f16x8 (&af)[FW], f16x8 (&bf)[TB][2]) {
         const uint8_t* as = lds + gbase + (uint32_t)s * AST;
         const uint8_t* bs = lds + gbase + 2u * AST + (uint32_t)s * BST;
+        const uint32_t piece = 2u * g + (uint32_t)h;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t piece = 2u * g + (uint32_t)h;
-            f16x8 af[FW], bf[TB][2];
-#pragma unroll
-            for (int f = 0; f < FW; ++f) {
-                const uint32_t r = wm + 16u * (uint32_t)f + j;
-                af[f] = *reinterpret_cast<const f16x8*>(as + r * kRowBytes + piece_offset(piece, r));
-            }
-#pragma unroll
-            for (int b = 0; b < TB; ++b) {
-                const uint32_t tk = wn + 16u * (uint32_t)b + j;
-#pragma unroll
-                for (int p = 0; p < 2; ++p)
-                    bf[b][p] = *reinterpret_cast<const f16x8*>(bs + ((uint32_t)p * kBN + tk) * kRowBytes +
-                                                               piece_offset(piece, tk));
-            }
-#pragma unroll
-            for (int f = 0; f < FW; ++f)
-#pragma unroll
-                for (int b = 0; b < TB; ++b)
-                    acc[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[f], bf[b][0], acc[f][b], 0, 0, 0);
-#pragma unroll
-            for (int f = 0; f < FW; ++f)
-#pragma unroll
-                for (int b = 0; b < TB; ++b)
-                    accl[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[f], bf[b][1], accl[f][b], 0, 0, 0);
+        for (int f = 0; f < FW; ++f) {
+            const uint32_t r = wm + 16u * (uint32_t)f + j;
+            af[f] = *reinterpret_cast<const f16x8*>(as + r * kRowBytes + piece_offset(piece, r));
         }
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            const uint32_t tk = wn + 16u * (uint32_t)b + j;
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                bf[b][p] = *reinterpret_cast<const f16x8*>(bs + ((uint32_t)p * kBN + tk) * kRowBytes +
+                                                           piece_offset(piece, tk));
+        }
+    };
+    auto matrix = [&](const f16x8 (&af)[FW], const f16x8 (&bf)[TB][2]) {
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+                acc[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[f], bf[b][0], acc[f][b], 0, 0, 0);
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+                accl[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[f], bf[b][1], accl[f][b], 0, 0, 0);
+    };
+    // Matrix work of one stage.  Where a token's power of two changed with this
+    // step, the accumulators follow first.
+    uint32_t code = kNoValue;  // of this lane's token
+    static_assert(TB == 1, "one token per lane");
+    auto compute = [&](int s, uint32_t step) {
+        const u32x2v changed = *reinterpret_cast<const u32x2v*>(scales[kg].changed[step % 4u]);
+        f16x8 af[FW], bf[TB][2];
+        operands(s, 0, af, bf);
+        const uint32_t c = __builtin_amdgcn_readfirstlane(wn < 32u ? changed.x : changed.y) >> (wn & 16u);
+        if (__builtin_expect((c & 0xffffu) != 0u && step != 0u, 0)) {  // wave-uniform
+            if ((c >> (j & 8u)) & 1u) {
+                const uint32_t now = scales[kg].code[step % 4u][wn + j];
+                const float r = scale_ratio(code, now);
+                code = now;
+#pragma unroll
+                for (int f = 0; f < FW; ++f) {
+                    acc[f][0] *= r;
+                    accl[f][0] *= r;
+                }
+            }
+        }
+        matrix(af, bf);
+        operands(s, 1, af, bf);
+        matrix(af, bf);
     };
 
     // Software pipeline, one barrier per step: iteration i converts step
@@ -584,40 +738,28 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
 #pragma unroll
     for (int q = 0; q < PD; ++q) issue(q, (s0 + (uint32_t)q) * kBK);
     if (ragged && s0 + 1u == steps) mask_b(0, s0 * kBK);
-    {
-        // Each wave's 8 tokens have a power of two of their own, from the run's
-        // first step: one for the whole tile met at a barrier and a second
-        // reduction before the first conversion (150 x 2048 x 512 8.0 us, 7.5 so;
-        // 512 x 2048 x 520 12.2 -> 12.0).
-        uint32_t v[FPT];
-        load_b(0, v);
-        float m = 0.0f;
-#pragma unroll
-        for (int e = 0; e < (int)FPT; ++e) m += __builtin_fabsf(__uint_as_float(v[e]));
-        const int e = part_exponent(wave_sum(m) * 8.0f);
-        up = pow2f(e);
-        down = pow2f(-e);
-        if (lane == 0u) downs[kg][wv] = down;
-    }
-    convert_store(0, 0, 0u);
+    convert_store(0, 0, 0u, std::true_type{});
     issue(0, (s0 + (uint32_t)PD) * kBK);
     __syncthreads();
+    code = scales[kg].code[0][wn + j];
     // The matrix work comes first in program order: its LDS reads then need
     // not wait behind the conversion's LDS writes, and the scheduler can fill
     // the matrix-core latency with the conversion's VALU work.  q = i % PD.
     auto iter = [&](int q, uint32_t i) {
         const int nx = (q + 1) % PD;
         if (ragged && s0 + i + 2u == steps) mask_b(nx, (s0 + i + 1u) * kBK);  // uniform
-        if (kOneRun || i < gs) compute(q & 1);                                 // uniform
-        convert_store(nx, (q + 1) & 1, i + 1u);
+        if (kOneRun || i < gs) compute(q & 1, i);                              // uniform
+        convert_store(nx, (q + 1) & 1, i + 1u, std::false_type{});
         issue(nx, (s0 + i + 1u + (uint32_t)PD) * kBK);
         __syncthreads();
     };
-    // Steps run in groups of kFoldSteps (a multiple of PD, so a group starts
-    // on register set 0 and stage 0); the accumulator is folded into the
-    // outer sum after each group.
-    for (uint32_t g0 = 0; g0 < iters; g0 += kFoldSteps) {
-        const uint32_t gend = min(g0 + kFoldSteps, iters);
+    // Steps run in groups of a multiple of PD, so a group starts on register
+    // set 0 and stage 0; the accumulator is folded into the outer sum after
+    // each group.
+    const uint32_t group = fold_steps<(uint32_t)PD>(iters);
+    float smallest[TB] = {__builtin_inff()};  // of this lane's sums, at the last fold
+    for (uint32_t g0 = 0; g0 < iters; g0 += group) {
+        const uint32_t gend = min(g0 + group, iters);
         uint32_t i = g0;
         for (; i + (uint32_t)PD <= gend; i += (uint32_t)PD) {
 #pragma unroll
@@ -630,10 +772,21 @@ __global__ __launch_bounds__(64 * NW * KS) void matmul_q8_kernel(const float* __
         for (int f = 0; f < FW; ++f)
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
-                fold(sum[f][b], acc[f][b], accl[f][b], downs[kg][(wn >> 3) + 2u * (uint32_t)b + (j >> 3)]);
+                const f32x4 was = sum[f][b];
+                fold(sum[f][b], acc[f][b], accl[f][b], down_of(code));
+                smallest[b] = smallest_of(was, sum[f][b], true, f == 0 ? __builtin_inff() : smallest[b]);
             }
-        if (g0 < gs) slow_steps<FW, TB>(flags[kg], wrs, ars, wm, wn, rowbytes, K, s0, g0, min(gend, gs) - g0, [&](int f, int b, f32x4 v) { sum[f][b] += v; });
     }
+    if (mrows < BM) {  // uniform
+        smallest[0] = __builtin_inff();
+#pragma unroll
+        for (int f = 0; f < FW; ++f) {
+            sum[f][0] += no_sums(wm + 16u * (uint32_t)f + 4u * g, mrows);
+            smallest[0] = smallest_of(sum[f][0], sum[f][0], false, smallest[0]);
+        }
+    }
+    small_sums<FW, TB>(smallest, wrs, ars, wm, wn, rowbytes, K, s0, gs, [&](int) { return code; },
+                       [&](int f, int b) { return sum[f][b]; }, [&](int f, int b, f32x4 v) { sum[f][b] = v; });
 
     if constexpr (KS > 1) {
         // Group 1's sums through LDS (its stages are done) into group 0's.
@@ -735,18 +888,14 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
     constexpr uint32_t BM = 16u * FW * NW;
     constexpr uint32_t kRowBytes = 128u;              // one LDS row: 64 codes of f16
     constexpr uint32_t BST = 2u * kBN * kRowBytes;    // one stage: two planes of 64 tokens
-    constexpr uint32_t kFoldSteps = kFoldCodes / 64u;
     constexpr bool kSumsInLds = direct_sums_in_lds(NW, KS);
     constexpr bool kOneRun = KS == 1 && MODE == kWholeTiles;  // every workgroup takes all the steps
     static_assert(NW == 4 || NW == 8, "whole chunks per thread");
     static_assert(KS == 1 || KS == 2, "one or two K groups");
     static_assert(MODE != kTilePairs || KS == 2, "pairs are the two groups of a workgroup");
-    static_assert(kFoldSteps % 2u == 0u, "a fold group starts on register set 0");
     // [stages of group 0][stages of group 1][sums]
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    // [group][step][wave]: nonzero, the wave's tokens of the step are slow_step's
-    __shared__ __attribute__((aligned(8))) uint8_t flags[KS][kFlagSteps][8];
-    __shared__ float abssum[KS][8];
+    __shared__ __attribute__((aligned(8))) TokenScales scales[KS];
 
     // XCD-aware order: workgroup i runs on XCD i % 8; each XCD gets a
     // contiguous run of the tile sequence (tile_coords).  A split launch gives
@@ -835,11 +984,8 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
                 if (kb + 4u * (uint32_t)q + 3u >= K) gb[s][c][q].w = 0u;
             }
     };
-    float up = 1.0f, down = 1.0f;  // the run's power of two and its inverse
+    float up[CH];  // the powers of two of this thread's tokens
     constexpr uint32_t kChunkBytes = 8u * NW * kRowBytes;  // from a thread's token to its next in a stage
-    float least[CH];
-#pragma unroll
-    for (int c = 0; c < CH; ++c) least[c] = btok + 8u * NW * (uint32_t)c < ntok ? kPartMin : 0.0f;
     auto take = [&](int s, int c, uint32_t (&v)[8]) {
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -849,16 +995,16 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
             v[4 * q + 3] = gb[s][c][q].w;
         }
     };
-    auto flag = [&](uint32_t step, int c, bool bad) {
-        if (lane == 0u) flags[kg][step % kFlagSteps][wv + NW * (uint32_t)c] = bad ? 1u : 0u;
-    };
     // The two planes of register set s into the stage at `stage`.
-    auto convert_b = [&](int s, uint32_t stage, uint32_t step) {
+    auto convert_b = [&](int s, uint32_t stage, uint32_t step, auto first) {
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             uint32_t v[8];
             take(s, c, v);
-            flag(step, c, store_split(v, least[c], up, down, brow + stage + (uint32_t)c * kChunkBytes, kBN * kRowBytes));
+            uint8_t* const w = brow + stage + (uint32_t)c * kChunkBytes;
+            const uint32_t token = btok + 8u * NW * (uint32_t)c;
+            if constexpr (first) store_first(v, up[c], w, kBN * kRowBytes, scales[kg], token);
+            else store_split(v, up[c], w, kBN * kRowBytes, scales[kg], step, token);
         }
     };
 
@@ -869,7 +1015,9 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
         for (int b = 0; b < TB; ++b) {
             acc[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
             accl[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if constexpr (!kSumsInLds) sum[f][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const f32x4 none = no_sums(wm + 16u * (uint32_t)f + 4u * g, mrows);
+            if constexpr (kSumsInLds) lsum[(uint32_t)(f * TB + b) * NT] = none;
+            else sum[f][b] = none;
         }
 
     // Activation fragments of plane p of half h of a stage: lane group g takes
@@ -921,31 +1069,35 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
 #pragma unroll
     for (int q = 0; q < PD; ++q) issue_a(q, 64u * (s0 + (uint32_t)q));
     if (ragged && s0 + 1u == steps) mask_b(0, 64u * s0);
-    {
-        // the power of two, from the run's first step
-        float m = 0.0f;
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            uint32_t v[8];
-            take(0, c, v);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) m += __builtin_fabsf(__uint_as_float(v[e]));
-        }
-        m = wave_sum(m);
-        if (lane == 0u) abssum[kg][wv] = m;
-        __syncthreads();
-        const int e = part_exponent(wave_sum(lane < (uint32_t)NW ? abssum[kg][lane] : 0.0f));
-        up = pow2f(e);
-        down = pow2f(-e);
-    }
-    convert_b(0, 0u, 0u);
+    convert_b(0, 0u, 0u, std::true_type{});
     if constexpr (GB == 2) issue_b(0, 64u * (s0 + 2u));
     else issue_b(0, 64u * (s0 + 1u));
     if (ragged && s0 + 2u == steps) mask_b(GB - 1, 64u * (s0 + 1u));
-    convert_b(GB - 1, BST, 1u);
+    convert_b(GB - 1, BST, 1u, std::false_type{});
     if constexpr (GB == 2) issue_b(1, 64u * (s0 + 3u));
     else issue_b(0, 64u * (s0 + 2u));
     __syncthreads();
+    // The codes of this lane's tokens 16 b + j, a byte each, and what changes with
+    // the next step (a byte per 8 tokens; wave-uniform).
+    uint32_t code = 0u, changed0 = 0u, changed1 = 0u;  // (step 0 starts from its codes)
+#pragma unroll
+    for (int b = 0; b < TB; ++b) code |= (uint32_t)scales[kg].code[0][16u * (uint32_t)b + j] << (8 * b);
+    auto code_at = [&](int b) { return (code >> (8 * b)) & 255u; };
+    // A token's power of two changed with step `step`: its accumulators follow.
+    auto rescale = [&](uint32_t step) {
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            const uint32_t c = ((b < 2 ? changed0 : changed1) >> (16 * (b & 1) + (j & 8u))) & 1u;
+            const uint32_t now = c ? (uint32_t)scales[kg].code[step % 4u][16u * (uint32_t)b + j] : code_at(b);
+            const float r = scale_ratio(code_at(b), now);
+            code = (code & ~(255u << (8 * b))) | now << (8 * b);
+#pragma unroll
+            for (int f = 0; f < FW; ++f) {
+                acc[f][b] *= r;
+                accl[f][b] *= r;
+            }
+        }
+    };
 
     // One barrier per step.  Iteration i works on stage i % NS, written two
     // iterations earlier, so the fragments of its first phase are read before
@@ -963,18 +1115,18 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
         const int s = q % GB;
         const uint32_t next = cur + BST == kEnd ? 0u : cur + BST, after = next + BST == kEnd ? 0u : next + BST;
         if (ragged && s0 + i + 3u == steps) mask_b(s, (s0 + i + 2u) * 64u);  // uniform
+        if (__builtin_expect((changed0 | changed1) != 0u, 0)) rescale(i);    // uniform
         __builtin_amdgcn_sched_barrier(0);
         uint32_t v[CH][8], hp[CH][4], lp[CH][4];
-        float lo[CH], hi[CH];
+        float hi[CH];
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             take(s, c, v[c]);
-            lo[c] = kPartMax;
             hi[c] = 0.0f;
         }
         auto split = [&](int e) {  // pair e of the thread's 4 CH
             const int c = e >> 2, k = e & 3;
-            split2(__uint_as_float(v[c][2 * k]), __uint_as_float(v[c][2 * k + 1]), up, hp[c][k], lp[c][k], lo[c], hi[c]);
+            split2(__uint_as_float(v[c][2 * k]), __uint_as_float(v[c][2 * k + 1]), up[c], hp[c][k], lp[c][k], hi[c]);
         };
         read_b(cur, 0, 1, by);
         matrix(ax, bx, acc);
@@ -1000,25 +1152,29 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
         }
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            const bool bad = needs_slow(v[c], least[c], down, lo[c], hi[c]);
-            if (bad) {  // wave-uniform
-                *reinterpret_cast<u32x4v*>(w + (uint32_t)c * kChunkBytes) = u32x4v{0u, 0u, 0u, 0u};
-                *reinterpret_cast<u32x4v*>(w + (uint32_t)c * kChunkBytes + kBN * kRowBytes) = u32x4v{0u, 0u, 0u, 0u};
-            }
-            flag(i + 2u, c, bad);
+            settle(v[c], hi[c], up[c], w + (uint32_t)c * kChunkBytes, kBN * kRowBytes, scales[kg], i + 2u,
+                   btok + 8u * NW * (uint32_t)c);
         }
         issue_b(s, (s0 + i + 2u + (uint32_t)GB) * 64u);
         __builtin_amdgcn_sched_barrier(0);
+        const u32x2v changed = *reinterpret_cast<const u32x2v*>(scales[kg].changed[(i + 1u) % 4u]);
         read_b(next, 0, 0, bx);
         matrix(ay, by, accl);
         codes(q ^ 1, 0, ax);
 #pragma unroll
         for (int f = 0; f < FW; ++f) asm volatile("" : "+v"(ax[f]));  // converted here, not past the barrier
         interleave();
+        changed0 = __builtin_amdgcn_readfirstlane(changed.x);
+        changed1 = __builtin_amdgcn_readfirstlane(changed.y);
         cur = next;
     };
-    for (uint32_t g0 = 0; g0 < iters; g0 += kFoldSteps) {
-        const uint32_t gend = min(g0 + kFoldSteps, iters);
+    float smallest[TB];  // of each of this lane's tokens' sums, at the last fold
+#pragma unroll
+    for (int b = 0; b < TB; ++b) smallest[b] = __builtin_inff();
+    // (a group starts on register set 0; whole tiles fold alike in every form)
+    const uint32_t group = KS == 2 && MODE != kTilePairs ? fold_steps<2>(iters) : kFoldCodes / 64u;
+    for (uint32_t g0 = 0; g0 < iters; g0 += group) {
+        const uint32_t gend = min(g0 + group, iters);
         for (uint32_t i = g0; i < gend; i += 2u) {
             if (kOneRun || i < gs) iter(0, i);  // uniform over the group
             __syncthreads();
@@ -1028,23 +1184,35 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
             }
         }
         if (!kOneRun && g0 >= gs) continue;  // nothing since the last fold
-#pragma unroll
-        for (int f = 0; f < FW; ++f)
+        auto fold_all = [&](auto look) {  // look: smallest_of too, of one fold (1) or two (2)
 #pragma unroll
             for (int b = 0; b < TB; ++b) {
-                if constexpr (kSumsInLds) {
-                    f32x4 v = g0 == 0u ? f32x4{0.f, 0.f, 0.f, 0.f} : lsum[(uint32_t)(f * TB + b) * NT];
-                    fold(v, acc[f][b], accl[f][b], down);
-                    lsum[(uint32_t)(f * TB + b) * NT] = v;
-                } else {
-                    fold(sum[f][b], acc[f][b], accl[f][b], down);
+                if constexpr (look != 0) smallest[b] = __builtin_inff();
+#pragma unroll
+                for (int f = 0; f < FW; ++f) {
+                    f32x4 v;
+                    if constexpr (kSumsInLds) v = lsum[(uint32_t)(f * TB + b) * NT];
+                    else v = sum[f][b];
+                    const f32x4 was = v;
+                    fold(v, acc[f][b], accl[f][b], down_of(code_at(b)));
+                    if constexpr (kSumsInLds) lsum[(uint32_t)(f * TB + b) * NT] = v;
+                    else sum[f][b] = v;
+                    if constexpr (look != 0) smallest[b] = smallest_of(was, v, look == 2, smallest[b]);
                 }
             }
-        slow_steps<FW, TB>(flags[kg], wrs, ars, wm, 0u, rowbytes, K, s0, g0, min(gend, gs) - g0, [&](int f, int b, f32x4 v) {
-            if constexpr (kSumsInLds) lsum[(uint32_t)(f * TB + b) * NT] += v;
-            else sum[f][b] += v;
-        });
+        };
+        if (g0 + group < gs) fold_all(std::integral_constant<int, 0>{});
+        else if (g0 == 0u) fold_all(std::integral_constant<int, 1>{});
+        else fold_all(std::integral_constant<int, 2>{});
     }
+    auto get = [&](int f, int b) {
+        if constexpr (kSumsInLds) return lsum[(uint32_t)(f * TB + b) * NT];
+        else return sum[f][b];
+    };
+    small_sums<FW, TB>(smallest, wrs, ars, wm, 0u, rowbytes, K, s0, gs, code_at, get, [&](int f, int b, f32x4 v) {
+        if constexpr (kSumsInLds) lsum[(uint32_t)(f * TB + b) * NT] = v;
+        else sum[f][b] = v;
+    });
 
     if constexpr (KS > 1 && MODE != kTilePairs) {
         // group 1's sums through LDS (every stage is done with) into group 0's
@@ -1080,9 +1248,7 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
         for (int b = 0; b < TB; ++b) {
             const uint32_t tok = 16u * (uint32_t)b + j;
             if (tok >= ntok) continue;
-            f32x4 y;
-            if constexpr (kSumsInLds) y = gs ? lsum[(uint32_t)(f * TB + b) * NT] : f32x4{0.f, 0.f, 0.f, 0.f};
-            else y = sum[f][b];
+            f32x4 y = get(f, b);
             y[0] *= __uint_as_float(sv.x);
             y[1] *= __uint_as_float(sv.y);
             y[2] *= __uint_as_float(sv.z);
