@@ -827,7 +827,7 @@ def test_matmul_weight_past_4_gib():
     (40, 300, 1030, False),    # 32-row tiles, two K groups
     (40, 300, 2100, True),     # the same, K split between workgroups
     (300, 2048, 520, False),   # 64-row tiles
-    (256, 6144, 200, False),   # 128-row tiles, two K groups
+    (256, 6144, 600, False),   # 128-row tiles, two K groups
     (700, 3548, 1030, True),   # 128-row tiles, the last ones' K steps split
     (512, 6100, 330, False),   # 256-row tiles
     (510, 11200, 330, False),  # 384-row tiles
@@ -946,7 +946,7 @@ def test_matmul_tokens_of_many_scales(N, M, K, ws):
     (40, 300, 4500, True),     # the same, K split between workgroups
     (300, 2048, 500, False),   # 64-row tiles, two K groups
     (379, 2860, 300, False),   # the same, one group
-    (450, 4096, 300, False),   # 128-row tiles, two K groups
+    (450, 4096, 600, False),   # 128-row tiles, two K groups
     (19000, 128, 1030, True),  # 128-row tiles, the last ones' K steps split
     (577, 6100, 1030, False),  # 256-row tiles
     (510, 11200, 2061, False), # 384-row tiles
@@ -1052,3 +1052,32 @@ def test_matmul_time_does_not_depend_on_the_values():
     print(us, flush=True)
     for name, t in us.items():
         assert t < 1.5 * us["normal"], us
+
+
+@pytest.mark.parametrize("N,M,K,form", [
+    (500, 4000, 384, "FB2.PD4 waves=8 rows=64"),       # 256 tiles of 128 rows, one per CU: 6 steps
+    (500, 4000, 385, "FB4.ksplit2 waves=8 rows=128"),  # 7
+    (200, 5300, 64, "FB2.PD4 waves=8 rows=64"),        # 168 tiles, one step
+    (200, 5300, 390, "FB4.ksplit2 waves=8 rows=128"),
+    (1300, 7300, 380, "D128 waves=4 rows=128"),        # two rounds of 384-row tiles
+    (1300, 7300, 386, "D128 waves=8 rows=384"),
+    (500, 11200, 100, "D128 waves=8 rows=384"),        # one round
+])
+def test_matmul_few_steps(N, M, K, form):
+    """Rows of at most 384 codes take smaller tiles where several workgroups per CU
+    cover each other's starts: every 29th token against the oracle, nothing past
+    the output."""
+    rng = np.random.default_rng(N + M + K)
+    a = rng.standard_normal(N * K).astype(np.float32)
+    a[3 * K + 5] = np.inf
+    w = random_packed(rng, M, K)
+    s = rng.uniform(0.001, 0.05, M).astype(np.float32)
+    out = wxo_q8.DeviceBuffer(4 * (N * M + 64))
+    out.upload(np.full(N * M + 64, 7.5, np.float32))
+    ba, bw, bs = (wxo_q8.DeviceBuffer.from_array(v) for v in (a, w, s))
+    wxo_q8.matmul_q8_multi_device(ba, [(bw, bs, out, M)], N, K)
+    wxo_q8.synchronize()
+    assert f" {form} " in wxo_q8.last_variant(), wxo_q8.last_variant()
+    got = out.download(np.float32, N * M + 64)
+    assert np.all(got[N * M:] == np.float32(7.5)), "written past the output"
+    assert_matmul(got[:N * M], a, w, s, N, M, K, rows=np.unique(np.r_[np.arange(0, N, 29), 3, N - 1]))

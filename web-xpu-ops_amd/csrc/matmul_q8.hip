@@ -1509,7 +1509,13 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         set_variant(variant, kname, "D256", 8, 256, 0, (int)kBN, (uint32_t)((t8 + 7u) / 8u * 8u));
         return launch_direct<8, 2>(a, p, n, N, K, stream);
     }
-    if (t4 >= cus) {
+    // Up to 6 steps (K <= 384) the two groups' own starts outweigh what they share in
+    // one round of 128-row tiles: 64-row tiles, two workgroups per CU.  Same process,
+    // us, 128 -> 64 rows: 210 x 5406 x 128 9.5 -> 7.5, 995 x 1068 x 256 10.3 -> 9.0,
+    // 512 x 4096 x 256 11.0 -> 10.1, 75 x 11952 x 384 12.9 -> 12.4; past it 75 x 11952
+    // x 448 12.9 -> 13.8.
+    const bool halves = steps > 6u;
+    if (t4 > cus || (t4 == cus && halves)) {
         if (t4 == cus) {
             set_variant(variant, kname, "FB4.ksplit2", 8, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
             return launch_direct<4, 2, 2>(a, p, n, N, K, stream);
@@ -1558,7 +1564,11 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         }
         // Otherwise whole 128-row units: three per workgroup by the rule above,
         // or one per workgroup of 4 waves, two workgroups per CU.
-        if (rows384) {
+        // Up to 6 steps (K <= 384) several rounds of 384-row tiles lose to the smaller
+        // ones, whose two workgroups per CU cover each other's first loads and
+        // stores: 1371 x 7327 x 64 25.2 -> 21.7 us, 519 x 16882 x 192 27.4 -> 24.8,
+        // 928 x 8984 x 384 34.9 -> 34.1; past it 2412 x 3664 x 512 39.4 -> 40.9.
+        if (rows384 && (r12 == 1u || steps > 6u)) {
             set_variant(variant, kname, "D128", 8, 384, 0, (int)kBN, (uint32_t)((t12 + 7u) / 8u * 8u));
             return launch_direct<8, 3>(a, p, n, N, K, stream);
         }
@@ -1585,7 +1595,7 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // waves on the direct kernel, beat smaller tiles that fill them all.  Same
     // process, us, against the 64-row form: 128 tokens gate and up (176 tiles) 32.5 ->
     // 24.8, 256 tokens q, k, v (192) 31.7 -> 24.8, 320 x 5120 x 2048 (200) 32.2 -> 24.9.
-    if (5u * t4 >= 3u * cus) {
+    if (halves && 5u * t4 >= 3u * cus) {
         set_variant(variant, kname, "FB4.ksplit2", 8, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
         return launch_direct<4, 2, 2>(a, p, n, N, K, stream);
     }
