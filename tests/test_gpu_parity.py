@@ -378,6 +378,26 @@ def test_batched_ksplit_long_rows(N, K, M, kernel):
         assert_matvec(ys[m], w, s, xs[m], N, K)
 
 
+@pytest.mark.parametrize("N,K,M", [(4200, 1100, 1376), (4200, 1100, 2064), (5700, 900, 2064), (8200, 1030, 4112),
+                                   (700, 5000, 2064), (4096, 4097, 2064), (1500, 4200, 4112)])
+def test_batched_many_vector_groups(N, K, M):
+    """86, 129 and 257 groups of 16 vectors, which share the CUs badly in one round:
+    the k-split kernel runs several rounds of workgroups that fill them (rows in
+    one pass and in two).  A sample of the vectors against the oracle."""
+    rng = np.random.default_rng(N + 3 * K + M)
+    w = random_weights(rng, N, K, full_range=True)
+    s = rng.uniform(0.001, 0.05, N).astype(np.float32)
+    xs = rng.standard_normal((M, K)).astype(np.float32)
+    xs[M - 1, 5] = np.nan
+    ys = wxo_q8.matvecQ8Batched(weight=w, scale=s, vectors=xs, N=N, K=K, M=M)
+    v = wxo_q8.last_variant()
+    assert v.startswith("matvec_q8_ksplit"), v
+    x, y = (int(t) for t in v.split("grid=")[1].split("x"))
+    assert y == (M + 15) // 16 and x * y / (256 * -(-x * y // 256)) > 0.7, v
+    for m in [0, 15, 16, M // 2, M - 17, M - 1]:
+        assert_matvec(ys[m], w, s, xs[m], N, K)
+
+
 @pytest.mark.parametrize("M,K", [(5, 1030), (8, 64), (12, 2048), (13, 4099), (16, 1024), (17, 1500), (32, 520),
                                  (6, 3000), (14, 1000), (16, 768), (13, 1536), (20, 1024), (33, 1000),
                                  (5, 769), (5, 2047), (6, 897), (7, 1024), (8, 1025), (8, 2048), (9, 1100),

@@ -1586,12 +1586,29 @@ hipError_t launch_mv(const MatvecArgs& a, hipStream_t stream, Variant* variant) 
 // with a contiguous range of 16-row tiles; vector groups of ks_vectors<PACK>()
 // on grid y.  STW adds the store wave (K <= 1024 only: with two steps per
 // wave the x parts need more registers than nine waves per workgroup leave).
-// One round of one workgroup per CU whatever the vector groups, so that each
-// workgroup pays its prologue once (two groups of 16 vectors, N = 5632, K = 2048:
-// 13.2 -> 8.5 us; 11008, 4096: 28.7 -> 18.7).
+//
+// The grid for `groups` vector groups over `tiles` 16-row tiles: whole rounds of one
+// workgroup per CU, as many as cost least where a workgroup's start (its vectors'
+// load and split) takes as long as about 8 of its tiles.  Up to half as many groups
+// as CUs that is one round (two groups of 16 vectors, N = 5632, K = 2048: 13.2 -> 8.5
+// us against a round for each; 11008, 4096: 28.7 -> 18.7); 129 groups, say, would
+// leave 127 of 256 CUs idle (2064 vectors x 11008 x 2048: 627 us, 429 in five rounds
+// of 9 workgroups a group; 1376 x 11008 x 4096 622 -> 508).
 dim3 ks_grid(uint32_t tiles, uint32_t groups, uint32_t cus) {
-    const uint32_t x = groups < cus ? cus / groups : 1u;
-    return dim3(tiles < x ? tiles : x, groups);
+    const uint32_t first = (groups + cus - 1u) / cus;  // rounds
+    uint32_t best_x = 1u;
+    uint64_t best = ~0ull;
+    for (uint32_t r = first; r < first + 16u; ++r) {
+        const uint64_t room = (uint64_t)cus * r / groups;
+        const uint32_t x = room < tiles ? (uint32_t)room : tiles;
+        const uint64_t cost = (uint64_t)r * (8u + (tiles + x - 1u) / x);
+        if (cost < best) {
+            best = cost;
+            best_x = x;
+        }
+        if (x == tiles) break;  // (tiles >= 1: no rows, no launch)
+    }
+    return dim3(best_x, groups);
 }
 
 template <int SW, int PACK, bool STW = false>
