@@ -876,10 +876,14 @@ def test_matmul_activations_past_the_f16_window(N, M, K, ws):
     (33, [300], 1030, "x16.ksplit2"),                           # fewer tiles than workgroups per pass
     (64, [2048, 2048, 2048], 2048, "x16.ksplit2"),              # 6 tile passes per CU
     (77, [1000, 1, 530], 769, "x16.ksplit2"),
-    (140, [4080], 3073, "x16.ksplit2"),                         # 255 tiles, nine passes
+    (140, [3500], 3073, "x16.ksplit2"),                         # 219 tiles, nine passes: 8 tiles a workgroup
+    (140, [4080], 3073, "FB2.PD4.ksplit2"),                     # 10
     (4096, [100], 1024, "x16.ksplit2"),                         # a pass per CU
-    (48, [4096], 512, "x16.ksplit2"),                           # 3 tile passes per CU, half of the waves without codes
-    (48, [4097], 512, "FB1.PD4.ksplit2"),                       # one more
+    (2049, [272], 2048, "FB2.PD4.ksplit2"),                     # 129 workgroups of 17 tiles
+    (2049, [144], 2048, "x16.ksplit2"),                         # of 9
+    (2049, [145], 2048, "FB1.PD4.ksplit2"),                     # of 10
+    (48, [5440], 512, "x16.ksplit2"),                           # 4 tiles a workgroup, half of the waves without codes
+    (48, [5441], 512, "FB1.PD4.ksplit2"),                       # one more
     (40, [1000, 33], 767, "x16.ksplit2"),
     (40, [1000], 511, "FB1.PD4.ksplit2"),
 ])

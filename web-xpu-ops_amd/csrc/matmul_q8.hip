@@ -1471,20 +1471,30 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // Short prompts on the batched k-split kernel, 16 tokens a pass, all passes in
     // one round of the CUs: it splits each activation once per 16-row tile range
     // instead of once per 32- or 64-row tile, and waits for no barrier per step.
-    // From a sweep of 33 to 256 tokens x 1024 to 11264 rows, us, the tiles below ->
-    // this (K = 2048): 64 x 2048 16.8 -> 8.2, 64 x 6144 17.4 -> 12.8, 128 x 4096 17.6
-    // -> 15.3, 256 x 2048 17.4 -> 15.9, 96 x 6144 19.5 -> 18.1 (9 tile passes per CU);
-    // past 9 it loses (80 x 8192 19.7 -> 20.8, 160 x 4096 19.7 -> 21.1).  The same
-    // line at K = 1024 (64 x 6144 11.7 -> 8.9) and 4096 (64 x 6144 28.7 -> 20.9).
-    // At 512 to 768 codes some of its waves idle and the tiles have few steps: up to
-    // 3 tile passes per CU (40 x 2048 x 520 7.7 -> 6.5, 40 x 4096 x 520 8.4 -> 8.0, x
-    // 768 9.7 -> 7.9; past it 150 x 2048 x 520 8.6 -> 9.9).
+    // A workgroup costs its start and its 16-row tiles, each as much as rows of whole
+    // 1024s of codes; the tiles below cost their steps, more past one tile per CU.  So
+    // the line is drawn by a workgroup's tiles times the codes they are priced at, per
+    // code of a row.  From a sweep of 220 shapes of 33 to 4096 tokens, k-split / tiles,
+    // us: at 8, 183 x 2595 x 4096 29.7 / 33.4, 3214 x 115 x 1024 12.1 / 13.4, 191 x 1894 x
+    // 3073 26.3 / 30.3; past 9.5 against 32-row tiles 97 x 3881 x 2112 23.6 / 21.3, 282 x
+    // 1327 x 1088 14.5 / 14.2; against 64-row ones up to 12.5, 43 x 10399 x 1300 17.3 /
+    // 20.3, 2925 x 186 x 4038 38.4 / 47.4, past it 1377 x 400 x 2048 25.9 / 22.3, 2049 x
+    // 272 x 2048 (17 tiles on each of 129 workgroups) 28.9 / 23.3.  Over nine tile
+    // passes per CU in all the weight streams too often (33 x 15122 x 3996, 11: 49.6 /
+    // 42.6).  Rows up to 768 codes have few steps to save: up to 4 tiles, or 7 at whole
+    // rows' price (48 x 4096 x 512 8.0 / 8.4; 3469 x 68 x 640, 5 tiles: 10.5 / 9.4).
     // The forms split through a workspace stay where they apply.
     const uint64_t passes = (N + 15u) / 16u;
     uint64_t t16 = 0;
     for (uint32_t i = 0; i < n; ++i) t16 += (p[i].M + 15ull) / 16u;
-    if (!split4 && !split2 && K >= 512u && K <= 4096u && passes <= cus &&
-        t16 * passes <= (K > 768u ? 9ull : 3ull) * cus) {
+    bool on_ksplit = false;
+    if (!split4 && !split2 && K >= 512u && K <= 4096u && passes <= cus && t16 * passes <= 9ull * cus) {
+        const uint64_t per_pass = cus / passes, load = (t16 + per_pass - 1u) / per_pass;
+        const uint64_t priced = load * 1024u * ((K + 1023u) / 1024u);
+        on_ksplit = K > 768u ? 2u * priced <= (t1 > cus ? 25u : 19u) * (uint64_t)K
+                             : load <= 4u || priced <= 7u * (uint64_t)K;
+    }
+    if (on_ksplit) {
         const hipError_t e = launch_matvec_q8_batched_multi(pv, n, a, K, N, dev, stream, variant);
         if (variant && e == hipSuccess) {
             variant->kernel = kname;
