@@ -314,8 +314,12 @@ def test_batched_same_sign_long_k(M, K):
     (4100, 800, 12, "matvec_q8_ksplit"),
     # fewer tiles than CUs (one per workgroup, its barrier group half empty), ragged rows
     (1000, 900, 32, "matvec_q8_ksplit"), (33, 1024, 48, "matvec_q8_ksplit"), (17, 1000, 35, "matvec_q8_ksplit"),
-    (4096, 2048, 16, "matvec_q8_mv"), (11008, 2048, 4, "matvec_q8_mv"), (2048, 2048, 16, "matvec_q8_mv"),
-    (4096, 2048, 32, "matvec_q8_mv"), (4096, 1024, 24, "matvec_q8_mv"), (5632, 768, 16, "matvec_q8_mv"),
+    (4096, 2048, 16, "matvec_q8_ksplit"), (4096, 2048, 32, "matvec_q8_ksplit"), (4096, 1024, 24, "matvec_q8_ksplit"),
+    (3072, 1024, 12, "matvec_q8_ksplit"), (1500, 2048, 24, "matvec_q8_ksplit"),
+    # the VALU path's: few operations for a pass's start, or rows a little past whole 1024s of codes
+    (11008, 2048, 4, "matvec_q8_mv"), (2048, 2048, 16, "matvec_q8_mv"), (5632, 768, 16, "matvec_q8_mv"),
+    (1024, 2048, 24, "matvec_q8_mv"), (2048, 1025, 9, "matvec_q8_mv"), (4099, 3073, 5, "matvec_q8_mv"),
+    (4200, 4095, 8, "matvec_q8_mv"), (4096, 2049, 2, "matvec_q8_mv"),
 ])
 def test_batched_decoder_sized_weights(N, K, M, kernel):
     # Below 16384 rows the k-split kernel runs where it beats the VALU path
@@ -334,7 +338,7 @@ def test_batched_decoder_sized_weights(N, K, M, kernel):
 @pytest.mark.parametrize("N,K,M", [
     (4097, 2049, 5), (5000, 2500, 8), (4100, 3071, 16), (4096, 3072, 6), (17, 3072, 1500),  # three steps per wave
     (10241, 2100, 3), (10240, 3000, 4),
-    (4099, 3073, 5), (4200, 4095, 8), (5632, 4096, 13), (4096, 4096, 12), (1100, 4000, 35),  # four
+    (5860, 3073, 5), (4400, 4095, 8), (5632, 4096, 13), (4096, 4096, 12), (1100, 4000, 35),  # four
     (16384, 3500, 3),
     (4096, 1000, 5), (5632, 1024, 7), (4097, 1025, 5), (8191, 2048, 6), (16385, 2047, 3), (16384, 900, 4),
 ])

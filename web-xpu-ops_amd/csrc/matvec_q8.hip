@@ -1657,45 +1657,56 @@ hipError_t launch_ksplit_multi(const Projection* p, uint32_t count, const float*
 
 // Batched, K > 768: codes split across a workgroup's waves, x parts in
 // VGPRs (every wave busy from K > 896; at K = 512 half of them would idle and
-// the kernels below win).  Its cost is one pass per round of one workgroup per
-// CU (4.2, 6.0, 7.9, 9.5 us at K = 1024, 2048, 3072, 4096 with 8 vectors, about
-// a tenth more with 16) and the weight's stream; the VALU path's grows with
-// rows x (vectors + 1 per pass of 8).  Same process, launches issued one by one,
-// VALU -> k-split (us):
+// the kernels below win).  Both sides in ns, from 2000 shapes of 500 to 20000
+// rows, 800 to 11008 codes and 2 to 64 vectors: a k-split pass (up to 4096 codes, or
+// 3072 at a time) starts and then walks its tiles, each round of the CUs anew; the
+// VALU path takes its operations, rows x whole 1024s of codes x (vectors, by whole
+// eights past 8, + 1 per eight).  They hold to 7 and 15 %.  VALU -> k-split (us):
+//   vectors x rows x codes 12 x 3072 x 1024 6.7 -> 5.3, 16 x 3833 x 1536 11.9 -> 8.0, 32
+//   x 3072 x 2048 17.4 -> 7.9, 64 x 4097 x 900 22.1 -> 7.6, 12 x 4096 x 4096 15.1 ->
+//   11.3, 33 x 916 x 6144 29.0 -> 19.8; kept: 16 x 2048 x 2048 7.6 (7.8), 8 x 4097 x
+//   3073 11.1 (12.5), 16 x 2048 x 5632 16.5 (18.9), 9 x 2048 x 1025 6.6 (7.6).
+bool ksplit_costs_less(uint64_t N, uint32_t K, uint32_t M, uint32_t gx, uint32_t cus) {
+    const uint64_t groups = (M + 15u) / 16u, tiles = (N + 15u) / 16u, eights = (M + 7u) / 8u;
+    const uint64_t rounds = (gx * groups + cus - 1u) / cus, load = (tiles + gx - 1u) / gx;
+    const uint64_t passes = K > 4096u ? (K + 3071u) / 3072u : 1u, kilos = ((K + passes - 1u) / passes + 1023u) / 1024u;
+    const uint64_t ks = 1100u + rounds * passes * (1900u + 1800u * kilos + load * (460u * kilos + 150u));
+    const uint64_t whole = (K + 1023u) / 1024u * 1024u, vectors = M <= 8u ? M : 8u * eights;
+    const uint64_t valu = 2800u + N * whole * (45u * (vectors + eights) + 27u) / 1000000u + 380u * whole / 1000u + 280u * eights;
+    return 103u * ks < 100u * valu;
+}
+
+// Where the weight streams (more tiles than CUs) the two differ by more than the
+// costs above see, and the lines are drawn from both sides' times (VALU -> k-split):
 //   K = 1024: 4096 rows x 5 / 16 vectors 4.7 -> 4.2 / 5.8 -> 4.4, 16384 x 3 6.1 -> 5.8
-//   K = 2048: 5632 x 5 8.4 -> 6.5, 16384 x 3 8.8 -> 8.0, 2048 x 32 9.9 -> 7.0
-//   K = 3072: 2048 x 16 10.0 -> 9.0, 4096 x 6 8.6 -> 8.3, 11008 x 3 10.9 -> 10.4
-//   K = 4096: 4096 x 8 9.8 -> 10.1, x 12 15.1 -> 11.3; 5632 x 5 11.5 -> 10.0,
-//             11008 x 16 37.9 -> 15.0, 16384 x 3 15.4 -> 13.8
-// Up to 4096 rows at 1024 < K <= 2048 (and past 16 vectors at K <= 1024) the VALU
-// instances keep the calls that they had: their names are checked for there.
+//   K = 2048: 4097 x 5 8.9 -> 6.9, 5632 x 5 8.4 -> 6.5, 16384 x 3 8.8 -> 8.0
+//   K = 3072: 4097 x 5 10.9 -> 8.8, 4096 x 6 8.6 -> 8.3, 11008 x 3 10.9 -> 10.4
+//   K = 3073 to 4096, from 18e6 codes: 5632 x 3200 x 5, 16384 x 4096 x 3 15.4 -> 13.8;
+//       below 4608 x 3073 x 6 11.4 -> 12.3, 4097 x 4096 x 6 11.3 -> 11.9
+//   past 4096, from 125e6 operations a pass: 8 x 5632 x 5632 21.8 -> 17.2, 5 x 8192 x
+//       5632 24.7 -> 16.9, 12 x 4096 x 8192 33.5 -> 27.3; below, 8 x 4096 x 11008 28.8
+//       -> 32.2, 16 x 1000 x 20000 47.7 -> 61.3.
 bool ksplit_pays(uint64_t N, uint32_t K, uint32_t M, const DeviceInfo& dev) {
-    if (K <= 768u || (M + 15u) / 16u > 65535u) return false;
+    if (K <= 768u || K > 65536u || M < 3u || (M + 15u) / 16u > 65535u) return false;
+    const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
+    const uint64_t tiles = (N + 15u) / 16u;
+    const uint32_t gx = ks_grid((uint32_t)tiles, (M + 15u) / 16u, cus).x;
+    const uint64_t ops = N * (M + (M + 7u) / 8u);
     if (K > 4096u) {
-        // Passes of at most 3072 codes; each tile's sums take 1 KiB of LDS between
-        // them.  A pass is a fixed cost per round, the VALU path's the operations
-        // (VALU -> k-split, us): vectors x rows x codes 8 x 5632 x 5632 21.8 -> 17.2,
-        // 5 x 8192 x 5632 24.7 -> 16.9, 16 x 4096 x 4160 24.0 -> 19.9, 12 x 4096 x
-        // 8192 33.5 -> 27.3, 8 x 32000 x 8192 135 -> 57.5; below the line 8 x 4096 x
-        // 11008 28.8 -> 32.2, 16 x 2048 x 5632 16.5 -> 18.9, 16 x 1000 x 20000 47.7 -> 61.3.
-        if (M < 5u || K > 65536u) return false;
-        const uint64_t cus = (uint64_t)(dev.cu_count > 0 ? dev.cu_count : 256), tiles = (N + 15u) / 16u;
-        const uint64_t groups = (M + 15u) / 16u, gx = ks_grid((uint32_t)tiles, (uint32_t)groups, (uint32_t)cus).x;
-        if (kKsLdsBytes + (tiles + gx - 1u) / gx * 1024u > kMfmaLdsBytes) return false;
-        const uint64_t ops = N * K * (M + (M + 7u) / 8u), passes = (K + 3071u) / 3072u;
-        return ops >= passes * 125000000u;
+        // each tile's sums take 1 KiB of LDS between the passes
+        if (M < 5u || kKsLdsBytes + (tiles + gx - 1u) / gx * 1024u > kMfmaLdsBytes) return false;
+        if (ops * K >= (K + 3071u) / 3072u * 125000000ull) return true;
+    } else if (K > 3072u) {
+        if (M < 5u) return N >= 16384u;
+        if (N > 4096u ? N * K >= 18000000u : ops >= 38000u) return true;
+    } else if (K > 2048u) {
+        if ((M >= 5u && (N > 4096u || ops >= 28000u)) || N >= 10240u) return true;
+    } else {
+        if (N >= kMfmaMinRows) return true;
+        if (M >= 32u && (tiles < cus ? tiles : cus) * ((M + 15u) / 16u) <= cus) return true;  // one round
+        if (M >= 5u && (K > 1024u ? N > 4096u : N >= 5632u || (N >= 4096u && M <= 16u))) return true;
     }
-    if (K > 2048u) {
-        const bool three = K <= 3072u;
-        const uint64_t ops = N * (M + (M + 7u) / 8u);
-        return (M >= 5u && (N > 4096u || ops >= (three ? 28000u : 38000u))) ||
-               (M >= 3u && N >= (three ? 10240u : 16384u));
-    }
-    if (N >= kMfmaMinRows) return M >= 3u;
-    const uint64_t cus = (uint64_t)(dev.cu_count > 0 ? dev.cu_count : 256), ntiles = (N + 15u) / 16u;
-    if (M >= 32u && (ntiles < cus ? ntiles : cus) * ((M + 15u) / 16u) <= cus) return true;  // one round
-    if (K > 1024u) return N > 4096u && M >= 5u;
-    return (N >= 5632u && M >= 5u) || (N >= 4096u && M >= 5u && M <= 16u);
+    return ksplit_costs_less(N, K, M, gx, cus);
 }
 
 // Rows per workgroup: the largest R (up to RMAX) that still gives every SIMD
