@@ -420,6 +420,23 @@ def test_long_rows_batched(M):
         assert_matvec(y[m], w, s, xs[m], N, K)
 
 
+def test_long_rows_of_many():
+    """270003 rows of 4100 codes, 5 vectors: more 16-row tiles than one round of
+    workgroups has room to keep the sums of between the passes over K; sampled
+    rows at both ends and at random (one random 4096-row block repeated)."""
+    rng = np.random.default_rng(4100)
+    N, K, M, W = 270003, 4100, 5, 1025
+    block = rng.integers(0, 2 ** 32, 4096 * W, dtype=np.uint64).astype(np.uint32).reshape(4096, W)
+    w = np.ascontiguousarray(np.tile(block, ((N + 4095) // 4096, 1))[:N])
+    s = rng.uniform(1e-3, 1e-1, N).astype(np.float32)
+    xs = rng.standard_normal((M, K)).astype(np.float32)
+    ys = np.asarray(wxo_q8.matvecQ8Batched(weight=w.reshape(-1), scale=s, vectors=xs.reshape(-1), N=N, K=K, M=M)).reshape(M, N)
+    assert wxo_q8.last_variant().startswith("matvec_q8_ksplit.multi "), wxo_q8.last_variant()
+    rows = np.unique(np.concatenate([np.arange(64), np.arange(N - 100, N), rng.integers(0, N, 500)]))
+    for m in range(M):
+        assert_matvec(ys[m][rows], np.ascontiguousarray(w[rows]).reshape(-1), s[rows], xs[m], len(rows), K)
+
+
 def test_long_rows_matmul_with_and_without_workspace():
     """matmulQ8 over K = 65539 (1025 steps of 64 codes, 65 accumulator folds):
     the plain plan and the workspace's K split, each within the bar."""

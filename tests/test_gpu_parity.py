@@ -362,7 +362,8 @@ def test_batched_ksplit_steps(N, K, M):
     (5632, 4097, 9, "matvec_q8_ksplit.multi"), (5000, 6143, 8, "matvec_q8_ksplit.multi"),   # two passes
     (4100, 6144, 16, "matvec_q8_ksplit.multi"), (4099, 6145, 17, "matvec_q8_ksplit.multi"),  # two, three
     (3001, 11008, 33, "matvec_q8_ksplit.multi"), (16390, 9219, 5, "matvec_q8_ksplit.multi"),  # four
-    (2048, 4100, 2048, "matvec_q8_ksplit.multi"), (2049, 4100, 2048, "matvec_q8_mv"),  # 64, 65 tiles per workgroup
+    (2048, 4100, 2048, "matvec_q8_ksplit.multi"),  # 64 tiles per workgroup: all that it has room for
+    (2049, 4100, 2048, "matvec_q8_ksplit.multi"),  # one more: another round
     (150, 65536, 140, "matvec_q8_mv"), (300, 65536, 140, "matvec_q8_ksplit.multi"), (300, 65537, 140, "matvec_q8_mv"),
     (2048, 5632, 16, "matvec_q8_mv"), (8192, 5632, 4, "matvec_q8_mv"),
 ])
@@ -403,32 +404,34 @@ def test_batched_many_vector_groups(N, K, M):
 
 
 @pytest.mark.parametrize("M,K", [(5, 1030), (8, 64), (12, 2048), (13, 4099), (16, 1024), (17, 1500), (32, 520),
-                                 (6, 3000), (14, 1000), (16, 768), (13, 1536), (20, 1024), (33, 1000),
+                                 (6, 3000), (14, 1000), (16, 768), (5, 767), (37, 257), (13, 1536), (20, 1024), (33, 1000),
                                  (5, 769), (5, 2047), (6, 897), (7, 1024), (8, 1025), (8, 2048), (9, 1100),
                                  (16, 2048), (16, 2047), (18, 900), (21, 1999)])
 def test_batched_matrix_core_shapes(M, K):
     # From 16384 rows and 5 vectors the batched call runs on the matrix cores;
     # smaller shapes take the VALU path, which the other batched tests cover.
     # Ragged row tail (N % 16 != 0), ragged K, vector tiles past 16,
-    # full-range codes (-128 included).  768 < K <= 2048 runs the k-split
-    # kernel: 128 codes per wave (K <= 1024) or 256, vectors packed 5 (h|m|l
-    # in one operand), 8 (h|m, l) or 16 per tile (groups on grid y, the last
-    # one partial at 18, 21 and 33); K = 769 and 897 leave waves with no codes
-    # or a partial slice.  Other K run the x-parts-in-LDS kernels.
+    # full-range codes (-128 included).  From 769 codes on the k-split kernel:
+    # 128 codes per wave and step, vectors packed 5 (h|m|l in one operand), 8
+    # (h|m, l) or 16 per tile (groups on grid y, the last one partial at 18, 21
+    # and 33); K = 769 and 897 leave waves with no codes or a partial slice.  Up
+    # to 768 codes the kernel with the x parts in LDS (one to three steps).
     rng = np.random.default_rng(M * 1009 + K)
     N = 16397
     w = random_weights(rng, N, K, full_range=True)
     s = rng.uniform(0.001, 0.05, N).astype(np.float32)
     xs = rng.standard_normal((M, K)).astype(np.float32)
     ys = wxo_q8.matvecQ8Batched(weight=w, scale=s, vectors=xs, N=N, K=K, M=M)
+    head = wxo_q8.last_variant().split(" ")[0]
+    assert head == ("matvec_q8_mfma_dma" if K <= 768 else "matvec_q8_ksplit.multi" if K > 4096 else "matvec_q8_ksplit"), head
     for m in range(M):
         assert_matvec(ys[m], w, s, xs[m], N, K)
 
 
 @pytest.mark.parametrize("M,K", [(5, 5376), (16, 1536), (16, 1024), (13, 1536), (16, 2048), (8, 2048), (5, 2048)])
 def test_batched_matrix_core_same_sign_long_k(M, K):
-    # The longest K whose x parts still fit in LDS for the tile, all terms
-    # positive: the matrix cores' longest accumulation chains.
+    # All terms positive: the matrix cores' accumulation chains, the sums of
+    # rows past one pass of the k-split kernel among them.
     rng = np.random.default_rng(K + M)
     N = 16400
     codes = rng.integers(64, 128, size=(N, K)).astype(np.int32)

@@ -424,8 +424,8 @@ __global__ __launch_bounds__(WAVES * 64) void matvec_q8_multi_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Small-M batched on the matrix cores (M >= 2): y[m, n] for up to 16 vectors
-// per tile (grid y), v_mfma_f32_16x16x32_bf16.
+// Small-M batched on the matrix cores: y[m, n] for up to 16 vectors per tile
+// (grid y), v_mfma_f32_16x16x32_bf16.
 //
 // Exactness: a code q in [-128, 127] is exact in bf16, and x is split into
 // three bf16 parts by truncation, x = h + m + l exactly (8 + 8 + 8 significand
@@ -433,14 +433,11 @@ __global__ __launch_bounds__(WAVES * 64) void matvec_q8_multi_kernel(
 // products do).  Every product q * part is exact in f32; the matrix core sums
 // them in f32.  h-products accumulate in one register set and the (2^-8 and
 // 2^-16 smaller) m, l products in another, so the chain of roundings sits on
-// the h sum alone.  The h sum is folded into an outer sum every 1024 codes,
-// so a chain is at most 32 accumulations plus the matrix core's own 32-term
-// sum and a fold per 1024 codes: under 80 roundings for the largest K that
-// fits, 5e-6 of sum_k |s q x|, inside the 1e-5 bar.
+// the h sum alone: with at most 768 codes 24 accumulations.
 //
 // VALU work is the code conversion only (one v_cvt_f32_i32_sdwa per code,
 // one perm per two codes): 1.5 ops per code whatever M is, against 1 + M on
-// the FMA path.  The x parts for the tile's vectors live in LDS
+// the FMA path.  The x parts for the tile's vectors live in LDS for the whole K
 // (3 x MC x Kp bf16, in B-operand order) and are read per 32-code block as one
 // ds_read_b128 per part per lane.
 //
@@ -475,12 +472,11 @@ __device__ __forceinline__ bf16x8 codes_to_bf16(uint32_t w0, uint32_t w1) {
 
 // Each workgroup takes a contiguous range of 16-row tiles (ranges differ by
 // at most one tile) and its four waves split that range evenly; a wave walks
-// its tiles T at a time over all of K in 256-code steps, the (tile group,
-// step) pairs forming one software pipeline with D - 1 pairs' loads in
-// flight ahead of the one computing.  No wave waits for another after the
-// prologue.  A finished tile's 16 x 16 block of sums goes through a
-// per-wave LDS slot so each lane stores 16 contiguous bytes of one vector's
-// output.
+// its tiles two at a time over all of K in 256-code steps, the (tile group,
+// step) pairs forming one software pipeline with one pair's loads in flight
+// ahead of the one computing.  No wave waits for another after the prologue.
+// A finished tile's 16 x 16 block of sums goes through a per-wave LDS slot so
+// each lane stores 16 contiguous bytes of one vector's output.
 constexpr uint32_t kTileSlotFloats = 16u * 17u;  // one 16 x 16 block, rows skewed by a float
 
 // The bf16 parts of one vector entry as f32 bit patterns (low 16 bits zero):
@@ -537,187 +533,28 @@ __device__ __forceinline__ void store_x_parts(uint16_t* xparts, uint32_t MC, uin
     *reinterpret_cast<u16x4*>(&xparts[2u * Kp * MC + at]) = u16x4{ll[0], ll[1], ll[2], ll[3]};
 }
 
-template <int T, int D>
-__global__ __launch_bounds__(256) void matvec_q8_mfma_kernel(
-    const uint32_t* __restrict__ weight, const float* __restrict__ scale, const float* __restrict__ x,
-    float* __restrict__ y, uint32_t N, uint32_t K, uint32_t W, uint32_t M, uint32_t Kp) {
-    // x parts in B-operand order: [part][32-code block][lane group g][column]
-    // x 8 bf16, so the 64 lanes of one B read cover one contiguous run.
-    extern __shared__ __attribute__((aligned(16))) uint16_t xparts[];  // 3 x Kp x MC bf16, then the tile slots
-    const uint32_t m0 = blockIdx.y * 16u;
-    const uint32_t MC = min(16u, M - m0);
-
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t j = lane & 15u, g = lane >> 4;
-    const uint32_t jb = min(j, MC - 1u);  // B column (lanes past MC compute columns nobody stores)
-    float* slot = reinterpret_cast<float*>(xparts + 3u * MC * Kp) + wv * kTileSlotFloats;
-    const uint32_t rowbytes = W * 4u;
-    const uint32_t ntiles = (N + 15u) / 16u;
-    const uint32_t S = Kp / 256u;  // steps per tile group
-    // this workgroup's tiles, then this wave's quarter of them
-    const uint32_t b0 = (uint32_t)((uint64_t)blockIdx.x * ntiles / gridDim.x);
-    const uint32_t b1 = (uint32_t)((uint64_t)(blockIdx.x + 1u) * ntiles / gridDim.x);
-    const uint32_t t0 = b0 + (b1 - b0) * wv / 4u, t1 = b0 + (b1 - b0) * (wv + 1u) / 4u;
-    const uint32_t ngroups = (t1 - t0 + T - 1) / T;
-    const uint32_t total = ngroups * S;
-    const int voff = (int)(j * rowbytes + g * 16u);
-    const uint32_t r_lane = (lane & 3u) * 4u;  // epilogue: rows r_lane .. r_lane + 3 of column lane / 4
-
-    // Loads of pair i: tile group i / S, step i % S.  Past the last pair the
-    // resource is empty and the loads read 0 without touching memory, so the
-    // issue is unconditional (a conditional issue would make the compiler
-    // join load sequences of different length and wait for all of them).
-    // Codes past K in a row belong to the next row (or read 0 past the
-    // group) and meet x parts that are 0.  The group's scales ride with its
-    // last step (an epilogue load would wait, in issue order, for the next
-    // step's prefetched weights).
-    auto issue = [&](uint32_t i, u32x4v (&d)[T][4], u32x4v (&sc)[T]) {
-        const uint32_t step = i % S;
-        const uint32_t tile0 = i < total ? t0 + (i / S) * T : 0u;
-        const uint32_t rows = i < total ? min((uint32_t)T * 16u, min(t1 * 16u, N) - tile0 * 16u) : 0u;
-        const __amdgpu_buffer_rsrc_t wrs = make_rsrc(weight + (size_t)tile0 * 16u * W, rows * rowbytes);
-        const __amdgpu_buffer_rsrc_t srs = make_rsrc(scale + tile0 * 16u, step == S - 1u ? rows * 4u : 0u);
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int so = (int)((uint32_t)t * 16u * rowbytes + step * 256u);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) d[t][u] = load_nt_b128(wrs, voff + 64 * u, so);
-            sc[t] = __builtin_amdgcn_raw_buffer_load_b128(srs, (int)(((uint32_t)t * 16u + r_lane) * 4u), 0, 0);
-        }
-    };
-
-    // The x parts are staged from up to 16 float4 loads per thread, all issued
-    // before the first weights: a wait for x then never has to wait for the
-    // weight loads queued behind it (vmcnt retires in issue order).
-    constexpr int XU = 16;
-    const uint32_t kq4 = Kp / 4u;  // float4 groups per staged vector row
-    const uint32_t n4 = MC * kq4;
-    const __amdgpu_buffer_rsrc_t xrs = make_rsrc(x + (size_t)m0 * K, MC * K * 4u);
-    u32x4v xv[XU];
-#pragma unroll
-    for (int u = 0; u < XU; ++u) {
-        const uint32_t idx = threadIdx.x + (uint32_t)u * 256u;
-        const uint32_t m = idx / kq4, k = (idx - m * kq4) * 4u;
-        // past the staged range: an offset beyond the resource reads 0
-        const int off = idx < n4 ? (int)((m * K + k) * 4u) : (int)0x7ffffff0;
-        xv[u] = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0);
-    }
-
-    u32x4v buf[D][T][4], sbuf[D][T];
-#pragma unroll
-    for (int q = 0; q < D - 1; ++q) issue((uint32_t)q, buf[q], sbuf[q]);
-
-    auto split_store = [&](uint32_t idx, u32x4v v) {
-        const uint32_t m = idx / kq4, k = (idx - m * kq4) * 4u;
-        store_x_parts(xparts, MC, Kp, K, m, k, v);
-    };
-#pragma unroll
-    for (int u = 0; u < XU; ++u) {
-        const uint32_t idx = threadIdx.x + (uint32_t)u * 256u;
-        if (idx < n4) split_store(idx, xv[u]);
-    }
-    for (uint32_t idx = threadIdx.x + XU * 256u; idx < n4; idx += 256u) {  // only when MC * Kp > 16384
-        const uint32_t m = idx / kq4, k = (idx - m * kq4) * 4u;
-        split_store(idx, __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)((m * K + k) * 4u), 0, 0));
-    }
-    __syncthreads();
-
-    f32x4 hi[T], lo[T], hs[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        hi[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        lo[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        hs[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    const uint16_t* xb = &xparts[(g * MC + jb) * 8u];
-    const uint32_t pstride = Kp * MC;
-    const uint32_t bstride = 32u * MC;  // bf16 elements per block
-
-    auto compute = [&](uint32_t i, const u32x4v (&d)[T][4], const u32x4v (&sc)[T]) {
-        const uint32_t step = i % S;
-        const uint16_t* xs = xb + step * 8u * bstride;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const uint32_t kb = ((uint32_t)u * 2u + (uint32_t)e) * bstride;
-                const bf16x8 bh = *reinterpret_cast<const bf16x8*>(xs + kb);
-                const bf16x8 bm = *reinterpret_cast<const bf16x8*>(xs + pstride + kb);
-                const bf16x8 bl = *reinterpret_cast<const bf16x8*>(xs + 2u * pstride + kb);
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    const bf16x8 av = codes_to_bf16(d[t][u][2 * e], d[t][u][2 * e + 1]);
-                    hi[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bh, hi[t], 0, 0, 0);
-                    lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bm, lo[t], 0, 0, 0);
-                    lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bl, lo[t], 0, 0, 0);
-                }
-            }
-        if (step % 4u == 3u) {  // wave-uniform: fold the h chain every 1024 codes
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                hs[t] += hi[t];
-                hi[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-        }
-        if (step == S - 1u) {  // wave-uniform: the tile group is complete
-            const uint32_t tile0 = t0 + (i / S) * T;
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                // C lane (j, g) holds rows 4g .. 4g+3 of column j: transpose
-                // through the slot so a lane stores 4 rows of one column.
-                const f32x4 v = (hs[t] + hi[t]) + lo[t];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) slot[j * 17u + g * 4u + (uint32_t)q] = v[q];
-                hi[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                lo[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                hs[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                const uint32_t c = lane >> 2;
-                const uint32_t row0 = (tile0 + (uint32_t)t) * 16u;
-                if (c < MC && tile0 + (uint32_t)t < t1) {
-                    float* yo = y + (size_t)(m0 + c) * N + row0 + r_lane;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (row0 + r_lane + (uint32_t)q < N)
-                            yo[q] = slot[c * 17u + r_lane + (uint32_t)q] * __uint_as_float(sc[t][q]);
-                }
-            }
-        }
-    };
-
-    for (uint32_t i = 0; i < total; i += (uint32_t)D) {
-#pragma unroll
-        for (int q = 0; q < D; ++q) {
-            issue(i + (uint32_t)(q + D - 1), buf[(q + D - 1) % D], sbuf[(q + D - 1) % D]);
-            if (q == 0 || i + (uint32_t)q < total) compute(i + (uint32_t)q, buf[q], sbuf[q]);
-        }
-    }
-}
-
-// The same kernel with the weight tiles fetched straight into LDS
-// (buffer_load_dwordx4 ... lds): one instruction moves 1 KiB of whole 128-byte
-// lines (4 rows x 256 bytes, or 8 rows x 128 bytes), where the register form
-// can only fetch 64 bytes of each of 16 rows.  NWV waves (4 or 8) each own D
-// stages of T tiles of 16 rows x SC codes (SC = 256 or 128: a K step).  Piece
-// q (16 bytes) of row j of a tile is stored at position q ^ (j mod pieces per
-// row), so the lanes that read one piece of 16 different rows spread over the
-// bank groups.  128-code steps halve the stages, which lets 8 waves (two per
-// SIMD) share one copy of the x parts of up to 8 vectors: one wave's LDS and
-// load waits then overlap the other's conversion and matrix work.
+// The weight tiles come straight into LDS (buffer_load_dwordx4 ... lds): one
+// instruction moves 1 KiB of whole 128-byte lines (4 rows x 256 bytes), where
+// loads into registers fetch 64 bytes of each of 16 rows.  Each wave owns D
+// stages of T tiles of 16 rows x 256 codes.  Piece q (16 bytes) of row j of a
+// tile is stored at position q ^ j, so the lanes that read one piece of 16
+// different rows spread over the bank groups.
 // Waits are explicit, since the compiler does not track these loads: every
 // LDS read of a stage completes (lgkmcnt(0)) before the stage is refilled,
 // and a stage is read only after its loads have landed (vmcnt, counting the
 // loads issued after it; vector stores count there too, which can only make
 // the wait longer).
+constexpr uint32_t kDmaMaxCodes = 768u;  // the x parts of 16 vectors fit beside the stages; all staged in one go
 constexpr uint32_t kDmaTileBytes = 16u * 256u;  // one tile at 256-code steps
 // Stages per wave.  Three or four (more weight bytes in flight per wave,
 // fewer workgroups per CU) measured slower at every M from 2 to 14.
 constexpr int kDmaStages = 2;
 
-template <int T, int D, int NWV = 4, int SC = 256>
-__global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
+template <int T, int D>
+__global__ __launch_bounds__(256) void matvec_q8_mfma_dma_kernel(
     const uint32_t* __restrict__ weight, const float* __restrict__ scale, const float* __restrict__ x,
     float* __restrict__ y, uint32_t N, uint32_t K, uint32_t W, uint32_t M, uint32_t Kp) {
+    constexpr int NWV = 4, SC = 256;                    // waves; codes per step
     extern __shared__ __attribute__((aligned(16))) uint16_t xparts[];  // x parts, weight stages, tile slots
     const uint32_t m0 = blockIdx.y * 16u;
     const uint32_t MC = min(16u, M - m0);
@@ -727,8 +564,6 @@ __global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
     const uint32_t j = lane & 15u, g = lane >> 4;
     const uint32_t jb = min(j, MC - 1u);
     uint8_t* stages = reinterpret_cast<uint8_t*>(xparts + 3u * MC * Kp);
-    static_assert(NWV == 4 || NWV == 8, "4 or 8 waves");
-    static_assert(SC == 256 || SC == 128, "256- or 128-code steps");
     constexpr uint32_t TBY = 16u * (uint32_t)SC;       // bytes of one tile per step
     constexpr uint32_t PPR = (uint32_t)SC / 16u;        // 16-byte pieces per row
     constexpr uint32_t RPI = 1024u / (uint32_t)SC;      // rows per load instruction
@@ -776,7 +611,8 @@ __global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
         }
     };
 
-    constexpr int XU = 64 / NWV;  // x loads per thread in the first pass (16 KiB of x per pass)
+    constexpr int XU = 64 / NWV;  // x loads per thread
+    static_assert(XU * NT * 4u >= 16u * kDmaMaxCodes, "every vector in one go");
     const uint32_t kq4 = Kp / 4u;
     const uint32_t n4 = MC * kq4;
     const __amdgpu_buffer_rsrc_t xrs = make_rsrc(x + (size_t)m0 * K, MC * K * 4u);
@@ -799,10 +635,6 @@ __global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
             store_x_parts(xparts, MC, Kp, K, m, (idx - m * kq4) * 4u, xv[u]);
         }
     }
-    for (uint32_t idx = threadIdx.x + XU * NT; idx < n4; idx += NT) {
-        const uint32_t m = idx / kq4, k = (idx - m * kq4) * 4u;
-        store_x_parts(xparts, MC, Kp, K, m, k, __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)((m * K + k) * 4u), 0, 0));
-    }
     // The x parts are this workgroup's own LDS writes: wait for them and meet
     // at a plain barrier (a fence here would also wait for the weight stages
     // already in flight).
@@ -811,12 +643,11 @@ __global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
 
-    f32x4 hi[T], lo[T], hs[T];
+    f32x4 hi[T], lo[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         hi[t] = f32x4{0.f, 0.f, 0.f, 0.f};
         lo[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        hs[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     const uint16_t* xb = &xparts[(g * MC + jb) * 8u];
     const uint32_t pstride = Kp * MC;
@@ -849,24 +680,15 @@ __global__ __launch_bounds__(64 * NWV) void matvec_q8_mfma_dma_kernel(
                 }
             }
         }
-        constexpr uint32_t kFoldSteps = 1024u / (uint32_t)SC;  // fold the h sums every 1024 codes
-        if (step % kFoldSteps == kFoldSteps - 1u) {
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                hs[t] += hi[t];
-                hi[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-        }
         if (step == S - 1u) {
             const uint32_t tile0 = t0 + (i / S) * T;
 #pragma unroll
             for (int t = 0; t < T; ++t) {
-                const f32x4 v = (hs[t] + hi[t]) + lo[t];
+                const f32x4 v = hi[t] + lo[t];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) slot[j * 17u + g * 4u + (uint32_t)q] = v[q];
                 hi[t] = f32x4{0.f, 0.f, 0.f, 0.f};
                 lo[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                hs[t] = f32x4{0.f, 0.f, 0.f, 0.f};
                 const uint32_t c = lane >> 2;
                 const uint32_t row0 = (tile0 + (uint32_t)t) * 16u;
                 if (c < MC && tile0 + (uint32_t)t < t1) {
@@ -1587,14 +1409,18 @@ hipError_t launch_mv(const MatvecArgs& a, hipStream_t stream, Variant* variant) 
 // on grid y.  STW adds the store wave (K <= 1024 only: with two steps per
 // wave the x parts need more registers than nine waves per workgroup leave).
 //
+// Rows past 4096 codes keep each tile's sums in 1 KiB of LDS between their passes.
+constexpr uint32_t kKsLongTiles = (kMfmaLdsBytes - kKsLdsBytes) / 1024u;
+
 // The grid for `groups` vector groups over `tiles` 16-row tiles: whole rounds of one
 // workgroup per CU, as many as cost least where a workgroup's start (its vectors'
 // load and split) takes as long as about 8 of its tiles.  Up to half as many groups
 // as CUs that is one round (two groups of 16 vectors, N = 5632, K = 2048: 13.2 -> 8.5
 // us against a round for each; 11008, 4096: 28.7 -> 18.7); 129 groups, say, would
 // leave 127 of 256 CUs idle (2064 vectors x 11008 x 2048: 627 us, 429 in five rounds
-// of 9 workgroups a group; 1376 x 11008 x 4096 622 -> 508).
-dim3 ks_grid(uint32_t tiles, uint32_t groups, uint32_t cus) {
+// of 9 workgroups a group; 1376 x 11008 x 4096 622 -> 508).  most: the tiles a
+// workgroup has room for.
+dim3 ks_grid(uint32_t tiles, uint32_t groups, uint32_t cus, uint32_t most = ~0u) {
     const uint32_t first = (groups + cus - 1u) / cus;  // rounds
     uint32_t best_x = 1u;
     uint64_t best = ~0ull;
@@ -1602,7 +1428,7 @@ dim3 ks_grid(uint32_t tiles, uint32_t groups, uint32_t cus) {
         const uint64_t room = (uint64_t)cus * r / groups;
         const uint32_t x = room < tiles ? (uint32_t)room : tiles;
         const uint64_t cost = (uint64_t)r * (8u + (tiles + x - 1u) / x);
-        if (cost < best) {
+        if (cost < best && (tiles + x - 1u) / x <= most) {
             best = cost;
             best_x = x;
         }
@@ -1643,7 +1469,7 @@ hipError_t launch_ksplit_multi(const Projection* p, uint32_t count, const float*
     }
     several.t0[kMaxProjections] = tiles;
     const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
-    const dim3 grid = ks_grid(tiles, (M + VPB - 1u) / VPB, cus);
+    const dim3 grid = ks_grid(tiles, (M + VPB - 1u) / VPB, cus, LONG ? kKsLongTiles : ~0u);
     // LONG: the fewest passes, of even length in whole 1024s
     const uint32_t passes = (K + 1024u * SW - 1u) / (1024u * SW);
     const uint32_t Kc = (K + 1024u * passes - 1u) / (1024u * passes) * 1024u;
@@ -1690,11 +1516,10 @@ bool ksplit_pays(uint64_t N, uint32_t K, uint32_t M, const DeviceInfo& dev) {
     if (K <= 768u || K > 65536u || M < 3u || (M + 15u) / 16u > 65535u) return false;
     const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
     const uint64_t tiles = (N + 15u) / 16u;
-    const uint32_t gx = ks_grid((uint32_t)tiles, (M + 15u) / 16u, cus).x;
+    const uint32_t gx = ks_grid((uint32_t)tiles, (M + 15u) / 16u, cus, K > 4096u ? kKsLongTiles : ~0u).x;
     const uint64_t ops = N * (M + (M + 7u) / 8u);
     if (K > 4096u) {
-        // each tile's sums take 1 KiB of LDS between the passes
-        if (M < 5u || kKsLdsBytes + (tiles + gx - 1u) / gx * 1024u > kMfmaLdsBytes) return false;
+        if (M < 5u || (tiles + gx - 1u) / gx > kKsLongTiles) return false;
         if (ops * K >= (K + 3071u) / 3072u * 125000000ull) return true;
     } else if (K > 3072u) {
         if (M < 5u) return N >= 16384u;
@@ -1789,73 +1614,22 @@ hipError_t launch_matvec_q8(const MatvecArgs& a, const DeviceInfo& dev, hipStrea
         if (a.M <= 8u) return launch_ksplit<1, 2>(a, dev, stream, variant);
         return launch_ksplit<1, 1>(a, dev, stream, variant);
     }
-    // Batched.  The matrix-core kernels pay a per-workgroup prologue (the x
-    // parts of the whole K for their 16-vector tile, written to LDS) and a
-    // 64-byte-per-row load pattern; they win only on large weights with at
-    // least 5 vectors, where each workgroup streams many tiles and the VALU
-    // path's 1 + M operations per code no longer hide under the streaming.
+    // Short rows (up to 768 codes, where the k-split kernel's waves would idle) of
+    // large weights, from 5 vectors on: the x parts of the whole K in LDS, two tiles
+    // per step, the weight by DMA beside them (they always fit: 16 vectors x 768
+    // codes take 143616 of 163840 bytes).  VALU -> this (us): 5 / 16 vectors x 16384 x 512
+    // 11.0 -> 9.2 / 16.9 -> 11.0, 8 x 151936 x 768 63.7 -> 32.5, 8 x 32000 x 256 16.0 -> 8.2.
     // Everything else runs on the VALU path (up to 8 vectors per pass).
-    // Measured on MI355X over N = 2048 .. 151936, K = 1024 .. 20000, M = 2 .. 16.
-    {
-        const uint32_t Kp = (a.K + 255u) / 256u * 256u;
-        const uint32_t MC = a.M < 16u ? a.M : 16u;
-        const uint64_t lds = 3ull * MC * Kp * 2u + 4ull * kTileSlotFloats * 4u;
-        if (a.M >= 5u && a.N >= kMfmaMinRows && lds <= kMfmaLdsBytes && (a.M + 15u) / 16u <= 65535u) {
-            const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
-            const uint32_t ntiles = (a.N + 15u) / 16u;
-            const uint32_t wgs = (uint32_t)(kMfmaLdsBytes / lds) < 2u ? (uint32_t)(kMfmaLdsBytes / lds) : 2u;
-            const uint32_t grid = min((ntiles + 3u) / 4u, cus * wgs);
-            const dim3 g(grid, (a.M + 15u) / 16u);
-            // The weight tiles go straight into LDS (whole 128-byte lines per
-            // load instruction) whenever the stages fit beside the x parts:
-            // two tiles per step (one B read serves both) when they fit, one
-            // tile per step up to 4 vectors in a tile.
-            {
-                const uint64_t xbytes = 3ull * MC * Kp * 2u + 4ull * kTileSlotFloats * 4u;
-                const uint64_t lds1 = xbytes + 4ull * kDmaStages * 1u * kDmaTileBytes;
-                const uint64_t lds2 = xbytes + 4ull * kDmaStages * 2u * kDmaTileBytes;
-                const bool two = MC > 4u && lds2 <= kMfmaLdsBytes;
-                const uint64_t ldsd = two ? lds2 : lds1;
-                // one tile per step pays a B read per tile: from 5 vectors the
-                // register form (two tiles per step) is faster than that
-                if (two || (MC <= 4u && ldsd <= kMfmaLdsBytes)) {
-                    const uint32_t wg2 = (uint32_t)(kMfmaLdsBytes / ldsd) < 2u ? 1u : 2u;
-                    const dim3 g2(min((ntiles + 3u) / 4u, cus * wg2), (a.M + 15u) / 16u);
-                    if (!two)
-                        hipLaunchKernelGGL((matvec_q8_mfma_dma_kernel<1, kDmaStages>), g2, dim3(256), (size_t)ldsd, stream,
-                                           a.weight, a.scale, a.vector, a.output, a.N, a.K, a.W, a.M, Kp);
-                    else
-                        hipLaunchKernelGGL((matvec_q8_mfma_dma_kernel<2, kDmaStages>), g2, dim3(256), (size_t)ldsd, stream,
-                                           a.weight, a.scale, a.vector, a.output, a.N, a.K, a.W, a.M, Kp);
-                    set_variant(variant, "matvec_q8_mfma_dma", two ? "T2.4waves.256" : "T1.4waves.256", 4, 16 * (two ? 2 : 1),
-                                0, (int)MC, g2.x, g2.y);
-                    return hipGetLastError();
-                }
-                // 13 to 16 vectors: two tiles per step no longer fit beside the
-                // x parts, but one tile per step in 128-code steps does, shared
-                // by 8 waves (two per SIMD): cfg5 (N = 151936, K = 1024) at
-                // 16 vectors in 42.0 us against 45-46 on the register-load
-                // kernel below.
-                const uint64_t lds8 = 3ull * MC * Kp * 2u + 8ull * kTileSlotFloats * 4u +
-                                      8ull * kDmaStages * 1u * 16u * 128u;
-                if (MC > 12u && lds8 <= kMfmaLdsBytes) {
-                    const dim3 g8(min((ntiles + 3u) / 4u, cus), (a.M + 15u) / 16u);
-                    hipLaunchKernelGGL((matvec_q8_mfma_dma_kernel<1, kDmaStages, 8, 128>), g8, dim3(512), (size_t)lds8,
-                                       stream, a.weight, a.scale, a.vector, a.output, a.N, a.K, a.W, a.M, Kp);
-                    set_variant(variant, "matvec_q8_mfma_dma", "T1.8waves.128", 8, 16, 0, (int)MC, g8.x, g8.y);
-                    return hipGetLastError();
-                }
-            }
-            if (MC >= 12u)
-                hipLaunchKernelGGL((matvec_q8_mfma_kernel<2, 2>), g, dim3(256), (size_t)lds, stream, a.weight, a.scale,
-                                   a.vector, a.output, a.N, a.K, a.W, a.M, Kp);
-            else
-                hipLaunchKernelGGL((matvec_q8_mfma_kernel<1, 3>), g, dim3(256), (size_t)lds, stream, a.weight, a.scale,
-                                   a.vector, a.output, a.N, a.K, a.W, a.M, Kp);
-            set_variant(variant, "matvec_q8_mfma", MC >= 12u ? "T2.D2" : "T1.D3", 4, MC >= 12u ? 32 : 16, 0, (int)MC, g.x,
-                        g.y);
-            return hipGetLastError();
-        }
+    if (a.M >= 5u && a.N >= kMfmaMinRows && a.K <= kDmaMaxCodes && (a.M + 15u) / 16u <= 65535u) {
+        const uint32_t Kp = (a.K + 255u) / 256u * 256u, MC = a.M < 16u ? a.M : 16u;
+        const uint64_t lds = 3ull * MC * Kp * 2u + 4ull * kTileSlotFloats * 4u + 4ull * kDmaStages * 2u * kDmaTileBytes;
+        const uint32_t cus = (uint32_t)(dev.cu_count > 0 ? dev.cu_count : 256);
+        const uint32_t ntiles = (a.N + 15u) / 16u, per_cu = kMfmaLdsBytes / lds < 2u ? 1u : 2u;
+        const dim3 g(min((ntiles + 3u) / 4u, cus * per_cu), (a.M + 15u) / 16u);
+        hipLaunchKernelGGL((matvec_q8_mfma_dma_kernel<2, kDmaStages>), g, dim3(256), (size_t)lds, stream, a.weight, a.scale,
+                           a.vector, a.output, a.N, a.K, a.W, a.M, Kp);
+        set_variant(variant, "matvec_q8_mfma_dma", "T2.4waves.256", 4, 32, 0, (int)MC, g.x, g.y);
+        return hipGetLastError();
     }
     if (a.M <= 2) return dispatch_mv<2>(a, dev, stream, variant);
     if (a.M <= 4) return dispatch_mv<4>(a, dev, stream, variant);
