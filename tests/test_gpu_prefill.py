@@ -341,23 +341,20 @@ BALANCE_CASES = [
     (512, [2048, 2048, 2048], 2048, "D256.PD2", "D256.PD2"),  # 512-token q, k, v: 192 256-row tiles
     (256, [5632, 5632], 2048, "D256.PD2", "D256.PD2"),        # 256-token gate, up: 176 256-row tiles
     (500, [3000, 2800], 1030, "D256.PD2", "D256.PD2"),        # ragged tokens, rows and K: 184 256-row tiles
-    (700, [2048, 1500], 1030, "FB4.balance2", "D128"),        # 154 256-row tiles: 308 128-row tiles, 204 split
+    (700, [2048, 1500], 1030, "D256.PD2", "D256.PD2"),        # 154 256-row tiles
 ]
 
 
 @pytest.mark.parametrize("N,Ms,K,form_ws,form_plain", BALANCE_CASES)
 def test_matmul_workspace_balance(N, Ms, K, form_ws, form_plain):
     """Prompts whose 128-row tiles fill one round of two workgroups per CU
-    unevenly.  Where 256-row tiles fill two thirds of the CUs or more they run
-    on the direct kernel, workspace or not; otherwise with a workspace the
-    last 128-row tiles split their K steps in two, so every CU holds the same
-    work, and without one the direct kernel runs the 128-row tiles.  Outputs
-    within the matmulQ8 bar of the oracle (every 5th token, split and whole
-    tiles among them), Inf and NaN activations included; the same bits on
-    every run; nothing written past the outputs."""
+    unevenly: one round of 256-row tiles instead, workspace or not.  Outputs
+    within the matmulQ8 bar of the oracle (every 5th token), Inf and NaN
+    activations included; the same bits on every run; nothing written past the
+    outputs."""
     rng = np.random.default_rng(N + K + sum(Ms))
     a = rng.standard_normal(N * K).astype(np.float32)
-    a[(N - 1) * K + 2] = np.inf   # the last token row is a split tile's
+    a[(N - 1) * K + 2] = np.inf
     a[3 * K + 9] = np.nan
     ba = wxo_q8.DeviceBuffer.from_array(a)
     ws_bytes = wxo_q8.matmul_q8_workspace_bytes()
@@ -396,8 +393,9 @@ def test_matmul_workspace_balance(N, Ms, K, form_ws, form_plain):
     (192, [11008], 1030, "D256.PD2", "D256.PD2"),    # 129 256-row tiles
     (570, [4300], 1000, "D256.PD2", "D256.PD2"),     # 153
     (1216, [2049], 1030, "D256.PD2", "D256.PD2"),    # 171
-    (640, [4200], 1000, "FB4.balance2", "D128"),     # 170
-    (19000, [128], 1030, "FB4.balance2", "D128"),    # 297 tiles of either height, two rounds
+    (640, [4200], 1000, "D256.PD2", "D256.PD2"),     # 170
+    (1024, [4096], 1000, "D256", "D256"),            # 256: whole rounds of either height
+    (19000, [128], 1030, "D128", "D128"),            # 297 tiles of either height: two rounds of 256-row ones
 ])
 def test_matmul_one_round_of_256_row_tiles(N, Ms, K, form_ws, form_plain):
     """The lines of the one-round dispatch, as above."""
@@ -468,8 +466,8 @@ def random_packed(rng, M, K):
 
 def test_matmul_random_shapes_every_plan():
     """Seeded random shapes across the dispatch's plans (32-, 64- and 128-row
-    tiles, one or two K groups, splits in 2 or 4 parts, the balanced round,
-    several projections), with and without a workspace: every output row
+    tiles, one or two K groups, splits in 2 or 4 parts, several projections),
+    with and without a workspace: every output row
     sampled is within the matmulQ8 bar of the oracle, and nothing is written
     past the outputs."""
     rng = np.random.default_rng(20261202)
@@ -746,30 +744,27 @@ def test_matmul_tile_pairs_ragged_tokens_match_one_group():
 
 def test_matmul_256_row_tiles_match_the_one_group_form():
     """Launches whose 256-row tiles make whole rounds of the CUs take them on
-    the direct kernel (8 waves of 32 rows): 2048 tokens x 2048 x 2048 is 256
-    such tiles.  The bits of its first 1280 tokens equal a launch of those
-    tokens alone, whose 320 tiles of 128 rows (160 of 256 rows: under two
-    thirds of the CUs) take the 128-row direct form; every 41st token against
-    the oracle."""
-    N, M, K = 2048, 2048, 2048
+    the direct kernel (8 waves of 32 rows): 16384 tokens x 256 x 1100 is 256
+    such tiles.  Their bits equal those of the same tokens in a launch of
+    19200, whose 300 tiles would leave a second round mostly empty and which
+    takes the 128-row direct form; every 411th token against the oracle."""
+    N, n, M, K = 19200, 16384, 256, 1100
     rng = np.random.default_rng(256)
-    a = rng.standard_normal(N * K).astype(np.float32)
+    a = rng.standard_normal(N * K, dtype=np.float32)
     w = oracle.pack_q8(rng.integers(-128, 128, (M, K)).astype(np.int32).reshape(-1), M, K)
     s = rng.uniform(0.001, 0.05, M).astype(np.float32)
     bw, bs = wxo_q8.DeviceBuffer.from_array(w), wxo_q8.DeviceBuffer.from_array(s)
     out = wxo_q8.DeviceBuffer(4 * N * M)
     wxo_q8.matmul_q8_multi_device(wxo_q8.DeviceBuffer.from_array(a), [(bw, bs, out, M)], N, K)
     wxo_q8.synchronize()
-    assert " D256 " in wxo_q8.last_variant(), wxo_q8.last_variant()
+    assert " D128 waves=4 rows=128 " in wxo_q8.last_variant(), wxo_q8.last_variant()
     got = out.download(np.float32, N * M)
-    assert_matmul(got, a, w, s, N, M, K, rows=np.unique(np.r_[np.arange(0, N, 41), N - 1]))
-    n = 1280
+    assert_matmul(got, a, w, s, N, M, K, rows=np.unique(np.r_[np.arange(0, N, 411), N - 1]))
     half = wxo_q8.DeviceBuffer(4 * n * M)
     wxo_q8.matmul_q8_multi_device(wxo_q8.DeviceBuffer.from_array(a[:n * K]), [(bw, bs, half, M)], n, K)
     wxo_q8.synchronize()
-    variant = wxo_q8.last_variant()
-    assert " D128 " in variant, variant
-    assert_bits_equal(got[:n * M], half.download(np.float32, n * M), "256-row tiles vs the one-group 128-row form")
+    assert " D256 " in wxo_q8.last_variant(), wxo_q8.last_variant()
+    assert_bits_equal(half.download(np.float32, n * M), got[:n * M], "256-row tiles vs the one-group 128-row form")
 
 
 def test_matmul_256_row_tiles_ragged():
@@ -828,7 +823,7 @@ def test_matmul_weight_past_4_gib():
     (40, 300, 2100, True),     # the same, K split between workgroups
     (300, 2048, 520, False),   # 64-row tiles
     (256, 6144, 600, False),   # 128-row tiles, two K groups
-    (700, 3548, 1030, True),   # 128-row tiles, the last ones' K steps split
+    (512, 2048, 4096, True),   # 256-row tiles, K split between workgroups
     (512, 6100, 330, False),   # 256-row tiles
     (510, 11200, 330, False),  # 384-row tiles
 ])
@@ -951,7 +946,8 @@ def test_matmul_tokens_of_many_scales(N, M, K, ws):
     (300, 2048, 500, False),   # 64-row tiles, two K groups
     (379, 2860, 300, False),   # the same, one group
     (450, 4096, 600, False),   # 128-row tiles, two K groups
-    (19000, 128, 1030, True),  # 128-row tiles, the last ones' K steps split
+    (19000, 128, 1030, True),  # 128-row tiles, two workgroups per CU
+    (512, 2048, 4096, True),   # 256-row tiles, K split between workgroups
     (577, 6100, 1030, False),  # 256-row tiles
     (510, 11200, 2061, False), # 384-row tiles
 ])

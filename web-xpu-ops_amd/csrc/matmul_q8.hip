@@ -58,11 +58,10 @@
 // one token tile and every weight row) streamed the whole weight through
 // every XCD's L2: 512-token layer 215 -> 182 us, 2048 tokens 629 -> 570.
 //
-// With a caller's workspace, a launch may also split some tiles' K steps
-// between 2, 4 or 8 workgroups (a short prompt's tiles, which would leave most
-// CUs idle; the last tiles of a round that would load the CUs unevenly):
-// part 0 stores its unscaled sums into the output, the other parts into
-// tile-sized workspace blocks, and a second launch adds them in part order
+// With a caller's workspace, a short prompt's launch, whose tiles would leave most
+// CUs idle, may also split the tiles' K steps between 2, 4 or 8 workgroups: part 0
+// stores its unscaled sums into the output, the other parts into tile-sized
+// workspace blocks, and a second launch adds them in part order
 // and scales them.  The stream order between the two launches is the only
 // synchronisation, so every run gives the same bits.
 //
@@ -95,11 +94,10 @@ constexpr uint32_t kMaxMatmulProjections = 4;
 
 // Up to four projections of the same activations in one launch: projection p
 // owns weight-row tiles [mt0[p], mt0[p + 1]) of the launch's tile sequence
-// (mt0[p] = 0xffffffff past the last one).  A split launch runs its first
-// `whole` tiles whole and splits the other `splits` tiles' K steps into
-// `parts` runs, one workgroup each: part 0 stores its unscaled sums into the
-// output, part j >= 1 into the workspace block (j - 1) * splits + (tile -
-// whole) of BM x kBN floats ([token][row] within the tile), and
+// (mt0[p] = 0xffffffff past the last one).  A split launch splits the K steps of
+// its `tiles` tiles into `parts` runs, one workgroup each: part 0 stores its
+// unscaled sums into the output, part j >= 1 into the workspace block (j - 1) *
+// tiles + tile of BM x kBN floats ([token][row] within the tile), and
 // split_sum_kernel adds the parts in part order and scales them.
 struct MatmulProjections {
     const uint32_t* weight[kMaxMatmulProjections];
@@ -108,7 +106,7 @@ struct MatmulProjections {
     uint32_t M[kMaxMatmulProjections];
     uint32_t mt0[kMaxMatmulProjections];
     float* part;
-    uint32_t whole, splits, parts;
+    uint32_t tiles, parts;
 };
 
 
@@ -498,11 +496,7 @@ __device__ __forceinline__ void small_sums(const float (&smallest)[TB], __amdgpu
     }
 }
 
-// SPLIT instances take the split launch above: whole tiles plus split tiles
-// whose K steps are shared by `parts` workgroups (a short prompt's few tiles,
-// which would leave most CUs idle, or the tiles past the last whole round of
-// a long prompt, which would leave some CUs with one tile more than others).
-// The other instances run every tile whole, with no branch on it.
+// SPLIT instances take the split launch above.
 template <int FB, int NW, int BK, int PD, int KS, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW * KS, 4) void matmul_q8_kernel(const float* __restrict__ a, MatmulProjections P,
                                                         uint32_t N, uint32_t K, uint32_t W, uint32_t mtiles,
@@ -529,10 +523,8 @@ __global__ __launch_bounds__(64 * NW * KS, 4) void matmul_q8_kernel(const float*
     __shared__ __attribute__((aligned(8))) TokenScales scales[KS];
 
     // XCD-aware tile order: workgroup i runs on XCD i % 8; give each XCD a
-    // contiguous run of the tile sequence (tile_coords).  A split launch
-    // gives each XCD a run of the whole tiles first and then a run of the
-    // split tiles' parts, so every XCD holds its share of both and the whole
-    // tiles are dispatched first.  Workgroups past the end return whole (no
+    // contiguous run of the tile sequence (tile_coords), of a split launch with a
+    // tile's parts side by side.  Workgroups past the end return whole (no
     // barrier is skipped by part of one).
     const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
     uint32_t tile, xs = 0u, np = (uint32_t)KS;  // np: runs of this tile's K steps
@@ -542,19 +534,11 @@ __global__ __launch_bounds__(64 * NW * KS, 4) void matmul_q8_kernel(const float*
         if (lin >= total) return;
         tile = lin;
     } else {
-        const uint32_t wpx = (P.whole + 7u) / 8u;
-        if (slot < wpx) {
-            const uint32_t i = xcd * wpx + slot;
-            if (i >= P.whole) return;
-            tile = i;
-        } else {
-            const uint32_t np_all = P.splits * P.parts;
-            const uint32_t q = xcd * ((np_all + 7u) / 8u) + (slot - wpx);
-            if (q >= np_all) return;
-            tile = P.whole + q / P.parts;
-            xs = q % P.parts;
-            np = (uint32_t)KS * P.parts;
-        }
+        const uint32_t all = P.tiles * P.parts, q = xcd * ((all + 7u) / 8u) + slot;
+        if (q >= all) return;
+        tile = q / P.parts;
+        xs = q % P.parts;
+        np = (uint32_t)KS * P.parts;
     }
     uint32_t mt, nt;
     tile_coords(tile, mtiles, ntiles, mt, nt);
@@ -818,14 +802,13 @@ __global__ __launch_bounds__(64 * NW * KS, 4) void matmul_q8_kernel(const float*
     // The lane group is read again: kept from the start it costs the 64-row form on
     // two K groups (128 registers a lane) a spill.
     const uint32_t ge = __lane_id() >> 4;
-    const bool split = SPLIT && tile >= P.whole;
-    const __amdgpu_buffer_rsrc_t srs = make_rsrc(scale + m0, split ? 0u : mrows * 4u);
+    const __amdgpu_buffer_rsrc_t srs = make_rsrc(scale + m0, SPLIT ? 0u : mrows * 4u);
     float* const blk = SPLIT && xs > 0u
-        ? P.part + ((size_t)(xs - 1u) * P.splits + (tile - P.whole)) * (size_t)(BM * kBN) : nullptr;
+        ? P.part + ((size_t)(xs - 1u) * P.tiles + tile) * (size_t)(BM * kBN) : nullptr;
 #pragma unroll
     for (int f = 0; f < FW; ++f) {
         const uint32_t fm = wm + 16u * (uint32_t)f + 4u * ge;  // within the tile
-        const u32x4v sv = split ? u32x4v{0x3f800000u, 0x3f800000u, 0x3f800000u, 0x3f800000u}  // 1.0f
+        const u32x4v sv = SPLIT ? u32x4v{0x3f800000u, 0x3f800000u, 0x3f800000u, 0x3f800000u}  // 1.0f
                                 : __builtin_amdgcn_raw_buffer_load_b128(srs, (int)(fm * 4u), 0, 0);
 #pragma unroll
         for (int b = 0; b < TB; ++b) {
@@ -861,11 +844,9 @@ constexpr bool direct_sums_in_lds(int NW, int KS) { return NW == 8 && KS == 1; }
 // the activations go through a ring of three LDS stages, split into their f16
 // pairs once per group.  KS = 2: two groups share the tile and split its K steps
 // in halves (their sums meet in LDS), or, as kTilePairs, each take a tile of
-// their own.  kSplitTiles splits the last P.splits tiles' K steps into P.parts
-// runs, one workgroup each: part 0 stores its unscaled sums into the output,
-// part j >= 1 into workspace block (j - 1) * P.splits + tile, and
-// split_sum_kernel adds them in part order and scales them.  Every form sums a
-// run in the same order, so whole tiles have the same bits in all of them.
+// their own.  kSplitTiles splits the P.tiles tiles' K steps into P.parts runs,
+// one workgroup each.  Every form sums a run in the same order, so whole tiles
+// have the same bits in all of them.
 //
 // What bounds it: at 2048 x 2048 x 5632 (256 tiles of 256 rows, one per CU) the
 // step takes 1.1 us where its matrix ops alone, at the clock they leave (they
@@ -898,15 +879,14 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
     __shared__ __attribute__((aligned(8))) TokenScales scales[KS];
 
     // XCD-aware order: workgroup i runs on XCD i % 8; each XCD gets a
-    // contiguous run of the tile sequence (tile_coords).  A split launch gives
-    // each XCD a run of the whole tiles first and then a run of the split
-    // tiles' parts (a tile's parts adjacent).  Workgroups past the end return
-    // whole (no barrier is skipped by part of one).
+    // contiguous run of the tile sequence (tile_coords), of a split launch with a
+    // tile's parts side by side.  Workgroups past the end return whole (no barrier
+    // is skipped by part of one).
     const uint32_t kg = KS == 1 ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
     const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
     uint32_t tile, xs = 0u, np = (uint32_t)KS;  // np: runs of this tile's K steps
     if constexpr (MODE == kTilePairs) {
-        const uint32_t pairs = P.whole / 2u;
+        const uint32_t pairs = mtiles * ntiles / 2u;
         const uint32_t i = xcd * ((pairs + 7u) / 8u) + slot;
         if (i >= pairs) return;
         tile = 2u * i + kg;
@@ -916,18 +896,11 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
         tile = xcd * ((total + 7u) / 8u) + slot;
         if (tile >= total) return;
     } else {
-        const uint32_t wpx = (P.whole + 7u) / 8u;
-        if (slot < wpx) {
-            tile = xcd * wpx + slot;
-            if (tile >= P.whole) return;
-        } else {
-            const uint32_t np_all = P.splits * P.parts;
-            const uint32_t q = xcd * ((np_all + 7u) / 8u) + (slot - wpx);
-            if (q >= np_all) return;
-            tile = P.whole + q / P.parts;
-            xs = q % P.parts;
-            np = (uint32_t)KS * P.parts;
-        }
+        const uint32_t all = P.tiles * P.parts, q = xcd * ((all + 7u) / 8u) + slot;
+        if (q >= all) return;
+        tile = q / P.parts;
+        xs = q % P.parts;
+        np = (uint32_t)KS * P.parts;
     }
     uint32_t mt, nt;
     tile_coords(tile, mtiles, ntiles, mt, nt);
@@ -1235,10 +1208,10 @@ __global__ __launch_bounds__(64 * NW * KS, 2) void matmul_q8_direct_kernel(const
     // lane (j, g) of block (f, b): rows m0 + wm + 16 f + 4 g .. +3 of token
     // n0 + 16 b + j.  A split tile's parts store unscaled sums: part 0 into
     // the output, part xs into its workspace block ([token][row] in the tile).
-    const bool split = MODE == kSplitTiles && tile >= P.whole;
+    constexpr bool split = MODE == kSplitTiles;
     const __amdgpu_buffer_rsrc_t srs = make_rsrc(scale + m0, split ? 0u : mrows * 4u);
     float* const blk = MODE == kSplitTiles && xs > 0u
-        ? P.part + ((size_t)(xs - 1u) * P.splits + (tile - P.whole)) * (size_t)(BM * kBN) : nullptr;
+        ? P.part + ((size_t)(xs - 1u) * P.tiles + tile) * (size_t)(BM * kBN) : nullptr;
 #pragma unroll
     for (int f = 0; f < FW; ++f) {
         const uint32_t fm = wm + 16u * (uint32_t)f + 4u * g;
@@ -1273,7 +1246,7 @@ template <uint32_t BM>
 __global__ __launch_bounds__(256) void split_sum_kernel(MatmulProjections P, uint32_t N, uint32_t mtiles) {
     constexpr uint32_t G = BM / 4u;  // 4-row groups per token
     static_assert(kBN * G == 256u * (BM / 16u), "one group per thread");
-    const uint32_t st = blockIdx.x, tile = P.whole + st;
+    const uint32_t tile = blockIdx.x;
     uint32_t mt, nt;
     tile_coords(tile, mtiles, (N + kBN - 1u) / kBN, mt, nt);
     const uint32_t pj = (mt >= P.mt0[1] ? 1u : 0u) + (mt >= P.mt0[2] ? 1u : 0u) + (mt >= P.mt0[3] ? 1u : 0u);
@@ -1286,14 +1259,14 @@ __global__ __launch_bounds__(256) void split_sum_kernel(MatmulProjections P, uin
     float* y = P.out[pj] + (size_t)(n0 + t) * M + m0 + r;
     const float* sc = P.scale[pj] + m0 + r;
     const uint32_t parts = P.parts;
-    const size_t blk = (size_t)BM * kBN, off = (size_t)st * blk + (size_t)t * BM + r;
+    const size_t blk = (size_t)BM * kBN, off = (size_t)tile * blk + (size_t)t * BM + r;
     if (r + 3u < mrows) {
         f32x4 v = *reinterpret_cast<const f32x4_a4*>(y);
         const f32x4 s4 = *reinterpret_cast<const f32x4_a4*>(sc);
         f32x4 q[7];
 #pragma unroll
         for (uint32_t j = 1; j < 8u; ++j)
-            if (j < parts) q[j - 1u] = *reinterpret_cast<const f32x4*>(P.part + (size_t)(j - 1u) * P.splits * blk + off);
+            if (j < parts) q[j - 1u] = *reinterpret_cast<const f32x4*>(P.part + (size_t)(j - 1u) * P.tiles * blk + off);
 #pragma unroll
         for (uint32_t j = 1; j < 8u; ++j)
             if (j < parts) v += q[j - 1u];
@@ -1301,7 +1274,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(MatmulProjections P, uin
     } else {
         for (uint32_t k = 0; k < mrows - r; ++k) {
             float v = y[k];
-            for (uint32_t j = 1; j < parts; ++j) v += P.part[(size_t)(j - 1u) * P.splits * blk + off + k];
+            for (uint32_t j = 1; j < parts; ++j) v += P.part[(size_t)(j - 1u) * P.tiles * blk + off + k];
             y[k] = v * sc[k];
         }
     }
@@ -1332,12 +1305,12 @@ uint32_t fill_projections(const MatmulProjection* p, uint32_t count, uint32_t BM
 }
 
 // One launch of matmul_q8_direct_kernel over `count` projections of the same
-// activations.  kSplitTiles: the last `splits` tiles of the sequence have their K
-// steps split into `parts` runs, the workspace `part` holding (parts - 1) x splits
-// blocks of BM x kBN floats, and split_sum_kernel sums them in a second launch.
+// activations.  kSplitTiles: the tiles' K steps split into `parts` runs, the
+// workspace `part` holding (parts - 1) blocks of BM x kBN floats per tile, and
+// split_sum_kernel sums them in a second launch.
 template <int NW, int FW, int KS = 1, int MODE = kWholeTiles>
 hipError_t launch_direct(const float* a, const MatmulProjection* p, uint32_t count, uint32_t N, uint32_t K,
-                         hipStream_t stream, float* part = nullptr, uint32_t splits = 0, uint32_t parts = 1) {
+                         hipStream_t stream, float* part = nullptr, uint32_t parts = 1) {
     constexpr uint32_t BM = 16u * FW * NW;
     const uint32_t W = (uint32_t)(((uint64_t)K + 3) / 4);
     MatmulProjections P = {};
@@ -1345,11 +1318,10 @@ hipError_t launch_direct(const float* a, const MatmulProjection* p, uint32_t cou
     const uint32_t ntiles = (N + kBN - 1u) / kBN;
     const uint32_t tiles = mtiles * ntiles;
     P.part = part;
-    P.whole = tiles - splits;
-    P.splits = splits;
+    P.tiles = tiles;
     P.parts = parts;
     uint32_t grid = ((tiles + 7u) / 8u) * 8u;
-    if constexpr (MODE == kSplitTiles) grid = 8u * ((P.whole + 7u) / 8u + (splits * parts + 7u) / 8u);
+    if constexpr (MODE == kSplitTiles) grid = ((tiles * parts + 7u) / 8u) * 8u;
     if constexpr (MODE == kTilePairs) grid = 8u * ((tiles / 2u + 7u) / 8u);
     const size_t lds = KS * 3u * 2u * kBN * 128u + (direct_sums_in_lds(NW, KS) ? BM * kBN * 4u : 0u);
     hipLaunchKernelGGL((matmul_q8_direct_kernel<NW, FW, KS, MODE>), dim3(grid), dim3(64 * NW * KS), lds, stream, a, P, N,
@@ -1357,19 +1329,15 @@ hipError_t launch_direct(const float* a, const MatmulProjection* p, uint32_t cou
     if constexpr (MODE == kSplitTiles) {
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
-        hipLaunchKernelGGL(split_sum_kernel<BM>, dim3(splits, BM / 16u), dim3(256), 0, stream, P, N, mtiles);
+        hipLaunchKernelGGL(split_sum_kernel<BM>, dim3(tiles, BM / 16u), dim3(256), 0, stream, P, N, mtiles);
     }
     return hipGetLastError();
 }
 
-// One launch over `count` (1 to 4) projections of the same activations.  With
-// splits > 0 (a SPLIT instance) the last `splits` tiles of the sequence have
-// their K steps split into `parts` runs, with the workspace `part` holding
-// (parts - 1) x splits blocks of BM x kBN floats, and a second launch sums
-// them.
+// One launch of matmul_q8_kernel, alike.
 template <int FB, int NW, int BK, int PD, int KS = 1, bool SPLIT = false>
 hipError_t launch_fb(const float* a, const MatmulProjection* p, uint32_t count, uint32_t N, uint32_t K,
-                     hipStream_t stream, float* part = nullptr, uint32_t splits = 0, uint32_t parts = 1) {
+                     hipStream_t stream, float* part = nullptr, uint32_t parts = 1) {
     constexpr uint32_t kRowBytes = (uint32_t)BK * 2u;
     constexpr uint32_t BM = 32u * FB;
     const uint32_t W = (uint32_t)(((uint64_t)K + 3) / 4);
@@ -1378,18 +1346,17 @@ hipError_t launch_fb(const float* a, const MatmulProjection* p, uint32_t count, 
     const uint32_t ntiles = (N + kBN - 1u) / kBN;
     const uint32_t tiles = mtiles * ntiles;
     P.part = part;
-    P.whole = tiles - splits;
-    P.splits = splits;
+    P.tiles = tiles;
     P.parts = parts;
     uint32_t grid = ((tiles + 7u) / 8u) * 8u;
-    if constexpr (SPLIT) grid = 8u * ((P.whole + 7u) / 8u + (splits * parts + 7u) / 8u);
+    if constexpr (SPLIT) grid = ((tiles * parts + 7u) / 8u) * 8u;
     const size_t lds = (size_t)KS * (2u * BM * kRowBytes + 2u * 2u * kBN * kRowBytes);
     hipLaunchKernelGGL((matmul_q8_kernel<FB, NW, BK, PD, KS, SPLIT>), dim3(grid), dim3(64 * NW * KS), lds, stream, a,
                        P, N, K, W, mtiles, ntiles);
     if constexpr (SPLIT) {
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
-        hipLaunchKernelGGL(split_sum_kernel<BM>, dim3(splits, BM / 16u), dim3(256), 0, stream, P, N, mtiles);
+        hipLaunchKernelGGL(split_sum_kernel<BM>, dim3(tiles, BM / 16u), dim3(256), 0, stream, P, N, mtiles);
     }
     return hipGetLastError();
 }
@@ -1530,36 +1497,16 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
             set_variant(variant, kname, "FB4.ksplit2", 8, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
             return launch_direct<4, 2, 2>(a, p, n, N, K, stream);
         }
-        // Two workgroups per CU.  Between cus and 2 x cus tiles, some CUs
-        // take two tiles and the others one (384 tiles: half and half).  With
-        // a workspace, the last S = 2 x cus - tiles tiles split their K steps
-        // in two, so that whole tiles plus halves fill the 2 x cus slots and
-        // every CU holds the same work (384 tiles -> 256 whole and 256 halves,
-        // one of each per CU).  The halves' sum is a second launch (~5 us
-        // with its launch), so this pays for long rows only (320 x 7680 tokens x
-        // rows: 101.7 -> 91.3 us at K = 5632, 41.9 -> 42.6 at 2048); with more
-        // tiles the rounds even the CUs out by themselves.
-        const uint64_t slots = 2ull * cus;
-        const uint64_t S = t4 < slots ? slots - t4 : 0u;
-        const size_t blk = (size_t)128u * kBN * 4u;
-        // One round of 256-row tiles on the direct kernel beats both the split and
-        // the uneven round, with or without a workspace: a 128-row workgroup beside
-        // another takes longer than a 256-row one alone.  Same process, us, split ->
-        // 256-row: 512 tokens q, k, v (192 tiles) 41.0 -> 34.3, 256 tokens gate and up
-        // (176) 41.4 -> 34.3, 320 x 7168 x 2048 (140) 42.4 -> 33.7 (x 1024: 30.4 ->
-        // 20.6, x 5632: 90.1 -> 80.7), 300 x 6700 x 4096 (135) 74.5 -> 59.6; without a
-        // workspace 320 x 7168 x 1024 24.5 -> 20.6.  From 0.6 to 2/3 of the CUs the
-        // 128-row forms are kept for their names, which tests check at 154 and 160
-        // tiles, not for their time (154 tiles, K = 1030: 31.8 us against 22.1).
-        // More 256-row tiles than CUs (19000 x 128 x 2048, every tile half empty)
-        // would take two rounds: 67.9 us against 48.2 without a workspace, 58.2 with.
-        if (S > 0 && t8 <= cus && (5u * t8 < 3ull * cus || 3u * t8 >= 2ull * cus)) {
+        // One round of 256-row tiles beats an uneven round of 128-row ones, two
+        // workgroups per CU: a 128-row workgroup beside another takes longer than a
+        // 256-row one alone (us, 128 -> 256 rows: 700 x 3548 x 1030 28.0 -> 24.7, 640 x
+        // 4200 x 2048 42.4 -> 36.7, 1280 x 2048 x 8192 142 -> 118, 320 x 7168 x 1024 24.5 ->
+        // 20.6), and beats their last tiles' K steps split through a workspace as well
+        // (33.2, 48.3, 127, 30.4).  More 256-row tiles than CUs (19000 x 128 x 2048, every
+        // tile half empty) would take two rounds: 67.9 against 41.9.
+        if (t4 < 2ull * cus && t8 <= cus) {
             set_variant(variant, kname, "D256.PD2", 8, 256, 0, (int)kBN, (uint32_t)((t8 + 7u) / 8u * 8u));
             return launch_direct<8, 2>(a, p, n, N, K, stream);
-        }
-        if (workspace && S > 0 && steps >= 8u && S * blk <= workspace_bytes) {
-            set_variant(variant, kname, "FB4.balance2", 4, 128, 0, (int)kBN, (uint32_t)(t4 + S));
-            return launch_direct<4, 2, 1, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)S, 2u);
         }
         // Long rows whose 128-row tiles make two or more whole rounds of two per CU
         // where 256-row ones make neither whole rounds nor 2.75 of them: one
@@ -1598,7 +1545,7 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
             (xs - 1u) * t8 * blk <= workspace_bytes) {
             set_variant(variant, kname, xs == 4u ? "D256.split4" : "D256.split8", 8, 256, 0, (int)kBN,
                         (uint32_t)(t8 * xs));
-            return launch_direct<8, 2, 1, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)t8, xs);
+            return launch_direct<8, 2, 1, kSplitTiles>(a, p, n, N, K, stream, workspace, xs);
         }
     }
     // 128-row tiles that fill most of the CUs, one per CU with two K groups of 4
@@ -1620,17 +1567,17 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
             (xs - 1u) * t4 * blk <= workspace_bytes) {
             set_variant(variant, kname, xs == 4u ? "FB4.ksplit2.wgsplit4" : "FB4.ksplit2.wgsplit2", 8, 128, 0, (int)kBN,
                         (uint32_t)(t4 * xs));
-            return launch_direct<4, 2, 2, kSplitTiles>(a, p, n, N, K, stream, workspace, (uint32_t)t4, xs);
+            return launch_direct<4, 2, 2, kSplitTiles>(a, p, n, N, K, stream, workspace, xs);
         }
     }
     if (t1 <= cus) {
         if (split4) {
             set_variant(variant, kname, "FB1.PD4.ksplit2.wgsplit4", 16, 32, 0, (int)kBN, (uint32_t)(4u * t1));
-            return launch_fb<1, 8, 64, 4, 2, true>(a, p, n, N, K, stream, workspace, (uint32_t)t1, 4u);
+            return launch_fb<1, 8, 64, 4, 2, true>(a, p, n, N, K, stream, workspace, 4u);
         }
         if (split2) {
             set_variant(variant, kname, "FB1.PD4.ksplit2.wgsplit2", 16, 32, 0, (int)kBN, (uint32_t)(2u * t1));
-            return launch_fb<1, 8, 64, 4, 2, true>(a, p, n, N, K, stream, workspace, (uint32_t)t1, 2u);
+            return launch_fb<1, 8, 64, 4, 2, true>(a, p, n, N, K, stream, workspace, 2u);
         }
         set_variant(variant, kname, "FB1.PD4.ksplit2", 16, 32, 0, (int)kBN, (uint32_t)((t1 + 7u) / 8u * 8u));
         return launch_fb<1, 8, 64, 4, 2>(a, p, n, N, K, stream);
