@@ -287,14 +287,16 @@ def test_matmul_short_prompt_is_deterministic(N, M, K):
 
 SPLIT_CASES = [
     # (N, Ms, K, form): tokens, the projections' rows, columns, the expected split
-    (64, [2048], 2048, "wgsplit4"),     # 64 tiles of 32 rows: four workgroups per tile
-    (33, [300], 4099, "wgsplit4"),      # ragged rows and K, a one-token second tile row
-    (200, [256], 2048, "wgsplit4"),
-    (100, [1000], 1030, "wgsplit2"),    # 17 steps: two runs of at least 4 per K group
-    (128, [2048], 5632, "wgsplit2"),    # 128 tiles: two workgroups per tile
-    (64, [512, 256, 256], 2048, "wgsplit4"),  # three projections (q, k, v of a small model)
-    (64, [2048, 2048, 2048], 2048, "ksplit2"),  # 192 tiles: no room to split
-    (40, [96, 32, 32], 520, "ksplit2"),  # 9 steps: too few to split
+    (64, [2048], 4160, "FB1.PD4.ksplit2.wgsplit4"),     # 64 tiles of 32 rows: four workgroups per tile
+    (33, [300], 4099, "FB1.PD4.ksplit2.wgsplit4"),      # ragged rows and K, a one-token second tile row
+    (200, [256], 4200, "FB1.PD4.ksplit2.wgsplit4"),
+    (100, [2000], 4100, "FB1.PD4.ksplit2.wgsplit2"),    # 65 steps in two runs
+    (128, [2048], 5632, "FB1.PD4.ksplit2.wgsplit2"),    # 128 tiles: two workgroups per tile
+    (64, [512, 256, 256], 4160, "FB1.PD4.ksplit2.wgsplit4"),  # three projections (q, k, v of a small model)
+    (64, [2048, 2048, 2048], 4160, "FB1.PD4.ksplit2"),  # 192 tiles: no room to split
+    (40, [96, 32, 32], 500, "FB1.PD4.ksplit2"),         # 8 steps: too few to split
+    (64, [2048], 2048, "x16.ksplit2"),                  # up to 4096 codes the k-split kernel, a workspace or not
+    (100, [1000], 1030, "x16.ksplit2"),
 ]
 
 
@@ -325,7 +327,7 @@ def test_matmul_workspace_split(N, Ms, K, form):
     for _ in range(3):
         wxo_q8.matmul_q8_multi_device(ba, bufs, N, K, workspace=ws, workspace_bytes=ws_bytes)
         wxo_q8.synchronize()
-        assert wxo_q8.last_variant().split()[1].endswith(form), wxo_q8.last_variant()
+        assert wxo_q8.last_variant().split()[1] == form, wxo_q8.last_variant()
         runs.append([b[2].download(np.float32, N * b[3] + 64) for b in bufs])
     for r in runs[1:]:
         for got, first in zip(r, runs[0]):
@@ -535,7 +537,7 @@ def test_matmul_workspace_size_sets_the_split():
     """A workspace too small for four parts splits in two; one too small for
     that (or none) does not split; the results agree within the bar either
     way."""
-    N, M, K = 64, 2048, 2048
+    N, M, K = 64, 2048, 4160
     rng = np.random.default_rng(5)
     a = rng.standard_normal(N * K).astype(np.float32)
     codes = rng.integers(-128, 128, (M, K)).astype(np.int32)
@@ -820,7 +822,7 @@ def test_matmul_weight_past_4_gib():
 
 @pytest.mark.parametrize("N,M,K,ws", [
     (40, 300, 1030, False),    # 32-row tiles, two K groups
-    (40, 300, 2100, True),     # the same, K split between workgroups
+    (40, 300, 4500, True),     # the same, K split between workgroups
     (300, 2048, 520, False),   # 64-row tiles
     (256, 6144, 600, False),   # 128-row tiles, two K groups
     (512, 2048, 4096, True),   # 256-row tiles, K split between workgroups
@@ -917,7 +919,7 @@ def test_matmul_tokens_on_the_ksplit_kernel(N, Ms, K, form):
 @pytest.mark.parametrize("N,M,K,ws", [
     (100, 4096, 300, False),   # 32-row tiles, a ragged token tile
     (70, 2048, 5000, False),   # the same past four folds
-    (40, 300, 2100, True),     # K split between workgroups
+    (40, 300, 4500, True),     # K split between workgroups
     (300, 2048, 520, False),   # 64-row tiles
 ])
 def test_matmul_tokens_of_many_scales(N, M, K, ws):

@@ -35,11 +35,11 @@ def test_no_alloc_matches_the_workspace_entry():
     rng = np.random.default_rng(2024)
     ws_bytes = min(wxo_q8.matmul_q8_workspace_bytes(), SCRATCH_BYTES)
     ws = wxo_q8.DeviceBuffer(ws_bytes)
-    # 700 tokens over two projections (204 of their 308 tiles split in two:
-    # 6.4 MiB of the array), then a 64-token projection (every tile in four
-    # parts), then a smaller one over two projections (two parts)
-    for N, Ms, K, form in [(512, [2048], 4096, "D256.split4"), (64, [2048], 2048, "wgsplit4"),
-                           (40, [512, 256], 1030, "wgsplit2")]:
+    # 512 tokens (64 tiles of 256 rows in four parts: 12 MiB of the array), then a
+    # 64-token projection (every 32-row tile in four parts), then one over two
+    # projections (two parts)
+    for N, Ms, K, form in [(512, [2048], 4096, "D256.split4"), (64, [2048], 4160, "wgsplit4"),
+                           (100, [1500, 500], 4100, "wgsplit2")]:
         a = rng.standard_normal(N * K).astype(np.float32)
         a[1] = np.inf
         ba = wxo_q8.DeviceBuffer.from_array(a)
@@ -88,10 +88,10 @@ def test_no_alloc_entry_in_a_captured_graph():
         s = rng.uniform(0.001, 0.05, M).astype(np.float32)
         return w, s, wxo_q8.DeviceBuffer.from_array(w), wxo_q8.DeviceBuffer.from_array(s)
 
-    N, M, K = 64, 2048, 2048
+    N, M, K = 64, 2048, 4160
     w, s, bw, bs = projection(N, M, K)
     ba, out, ref = wxo_q8.DeviceBuffer(4 * N * K), wxo_q8.DeviceBuffer(4 * N * M), wxo_q8.DeviceBuffer(4 * N * M)
-    N2, M2, K2 = 40, 512, 1030  # the eager call between replays: two parts per tile
+    N2, M2, K2 = 100, 2000, 4100  # the eager call between replays: two parts per tile
     _, _, bw2, bs2 = projection(N2, M2, K2)
     ba2 = wxo_q8.DeviceBuffer.from_array(rng.standard_normal(N2 * K2).astype(np.float32))
     out2 = wxo_q8.DeviceBuffer(4 * N2 * M2)

@@ -1429,12 +1429,6 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     }
     const uint32_t steps = (uint32_t)(((uint64_t)K + 63u) / 64u);
     const char* kname = n > 1 ? "matmul_q8.multi" : "matmul_q8";
-    // With a workspace, short prompts whose 32-row tiles fill at most a quarter (a
-    // half) of the CUs split their K steps between 4 (2) workgroups, each run at
-    // least 4 steps per K group; the parts' sums meet in a second launch.
-    const size_t blk32 = (size_t)32u * kBN * 4u;
-    const bool split4 = workspace && 4u * t1 <= cus && steps >= 32u && 3u * t1 * blk32 <= workspace_bytes;
-    const bool split2 = workspace && 2u * t1 <= cus && steps >= 16u && t1 * blk32 <= workspace_bytes;
     // Short prompts on the batched k-split kernel, 16 tokens a pass, all passes in
     // one round of the CUs: it splits each activation once per 16-row tile range
     // instead of once per 32- or 64-row tile, and waits for no barrier per step.
@@ -1450,12 +1444,13 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     // passes per CU in all the weight streams too often (33 x 15122 x 3996, 11: 49.6 /
     // 42.6).  Rows up to 768 codes have few steps to save: up to 4 tiles, or 7 at whole
     // rows' price (48 x 4096 x 512 8.0 / 8.4; 3469 x 68 x 640, 5 tiles: 10.5 / 9.4).
-    // The forms split through a workspace stay where they apply.
+    // A workspace changes nothing here (64 x 2048 x 2048 8.2 us; its 32-row tiles split
+    // in 4 parts 13.0, 425 x 128 x 1024 in 2 13.1 against 6.6).
     const uint64_t passes = (N + 15u) / 16u;
     uint64_t t16 = 0;
     for (uint32_t i = 0; i < n; ++i) t16 += (p[i].M + 15ull) / 16u;
     bool on_ksplit = false;
-    if (!split4 && !split2 && K >= 512u && K <= 4096u && passes <= cus && t16 * passes <= 9ull * cus) {
+    if (K >= 512u && K <= 4096u && passes <= cus && t16 * passes <= 9ull * cus) {
         const uint64_t per_pass = cus / passes, load = (t16 + per_pass - 1u) / per_pass;
         const uint64_t priced = load * 1024u * ((K + 1023u) / 1024u);
         on_ksplit = K > 768u ? 2u * priced <= (t1 > cus ? 25u : 19u) * (uint64_t)K
@@ -1571,11 +1566,15 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         }
     }
     if (t1 <= cus) {
-        if (split4) {
+        // With a workspace, 32-row tiles that fill at most a quarter (a half) of the
+        // CUs also split their K steps between 4 (2) workgroups, each run at least 4
+        // steps per K group; the parts' sums meet in a second launch.
+        const size_t blk32 = (size_t)32u * kBN * 4u;
+        if (workspace && 4u * t1 <= cus && steps >= 32u && 3u * t1 * blk32 <= workspace_bytes) {
             set_variant(variant, kname, "FB1.PD4.ksplit2.wgsplit4", 16, 32, 0, (int)kBN, (uint32_t)(4u * t1));
             return launch_fb<1, 8, 64, 4, 2, true>(a, p, n, N, K, stream, workspace, 4u);
         }
-        if (split2) {
+        if (workspace && 2u * t1 <= cus && steps >= 16u && t1 * blk32 <= workspace_bytes) {
             set_variant(variant, kname, "FB1.PD4.ksplit2.wgsplit2", 16, 32, 0, (int)kBN, (uint32_t)(2u * t1));
             return launch_fb<1, 8, 64, 4, 2, true>(a, p, n, N, K, stream, workspace, 2u);
         }
