@@ -597,7 +597,7 @@ def test_threads_on_their_own_streams():
         elif kind == 1:  # 8 vectors on the k-split kernel
             N, K, M = 20000, 1024, 8
         elif kind == 2:  # prefill GEMM with its own workspace
-            N, K, M = 128, 2048, 1000
+            N, K, M = 128, 4160, 1000
         else:            # quantize + pack
             N, K, M = 512, 5000, 0
         job = {"kind": kind, "N": N, "K": K, "M": M, "outs": [], "error": None}

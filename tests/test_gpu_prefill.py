@@ -258,7 +258,8 @@ def test_matmul_multi_projection(N, K, Ms):
     wxo_q8.matmul_q8_multi_device(ba, bufs, N, K)
     wxo_q8.synchronize()
     if N > 32 and 1 < sum(1 for M in Ms if M) <= 4:  # one launch over all of them
-        assert wxo_q8.last_variant().startswith("matmul_q8.multi "), wxo_q8.last_variant()
+        head = wxo_q8.last_variant().split()[0]
+        assert head == ("matvec_q8_ksplit.multi" if (N, K) in ((100, 2048), (33, 1000)) else "matmul_q8.multi"), head
     for (w, s, M), (_, _, out, _) in zip(host, bufs):
         got = out.download(np.float32, N * M + 64)
         assert np.all(got[N * M:] == np.float32(7.5)), f"M={M}: written past the output"
@@ -266,11 +267,16 @@ def test_matmul_multi_projection(N, K, Ms):
             assert_matmul(got[:N * M], a, w, s[:M], N, M, K)
 
 
-@pytest.mark.parametrize("N,M,K", [(64, 2048, 5632), (100, 2048, 2048), (33, 300, 1030), (200, 1000, 4099)])
-def test_matmul_short_prompt_is_deterministic(N, M, K):
-    """Short prompts run one workgroup per tile with the tile's K steps split
-    between two groups of waves, whose sums meet in LDS in a fixed order: every
-    run gives the same bits, within the bar of the oracle."""
+@pytest.mark.parametrize("N,M,K,form", [(64, 2048, 5632, "FB1.PD4.ksplit2"), (100, 2048, 500, "FB1.PD4.ksplit2"),
+                                        (33, 300, 4100, "FB1.PD4.ksplit2"), (200, 1000, 4099, "FB1.PD4.ksplit2"),
+                                        (300, 2048, 4099, "FB2.PD4.ksplit2"),
+                                        (100, 2048, 2048, "matmul.tokens_as_vectors"),
+                                        (33, 300, 1030, "matmul.tokens_as_vectors")])
+def test_matmul_short_prompt_is_deterministic(N, M, K, form):
+    """Short prompts over rows past 4096 codes or of few run one workgroup per
+    tile with the tile's K steps split between two groups of waves, whose sums
+    meet in LDS in a fixed order, the others on the k-split kernel: every run
+    gives the same bits, within the bar of the oracle."""
     rng = np.random.default_rng(N * M + K)
     codes = rng.integers(-128, 128, (M, K)).astype(np.int32)
     w = oracle.pack_q8(codes.reshape(-1), M, K)
@@ -279,7 +285,7 @@ def test_matmul_short_prompt_is_deterministic(N, M, K):
     a[5] = np.nan
     a[K + 7] = np.inf
     first = wxo_q8.matmulQ8(a=a, weight=w, scale=s, N=N, M=M, K=K)
-    assert "ksplit2" in wxo_q8.last_variant(), wxo_q8.last_variant()
+    assert wxo_q8.last_variant().split()[1] == form, wxo_q8.last_variant()
     for _ in range(3):
         assert_bits_equal(wxo_q8.matmulQ8(a=a, weight=w, scale=s, N=N, M=M, K=K), first, "repeat")
     assert_matmul(first, a, w, s, N, M, K)
@@ -295,8 +301,8 @@ SPLIT_CASES = [
     (64, [512, 256, 256], 4160, "FB1.PD4.ksplit2.wgsplit4"),  # three projections (q, k, v of a small model)
     (64, [2048, 2048, 2048], 4160, "FB1.PD4.ksplit2"),  # 192 tiles: no room to split
     (40, [96, 32, 32], 500, "FB1.PD4.ksplit2"),         # 8 steps: too few to split
-    (64, [2048], 2048, "x16.ksplit2"),                  # up to 4096 codes the k-split kernel, a workspace or not
-    (100, [1000], 1030, "x16.ksplit2"),
+    (64, [2048], 2048, "matmul.tokens_as_vectors"),                  # up to 4096 codes the k-split kernel, a workspace or not
+    (100, [1000], 1030, "matmul.tokens_as_vectors"),
 ]
 
 
@@ -340,10 +346,10 @@ def test_matmul_workspace_split(N, Ms, K, form):
 BALANCE_CASES = [
     # (N, Ms, K, form with a workspace, form without): between cus and 2 x cus
     # 128-row tiles
-    (512, [2048, 2048, 2048], 2048, "D256.PD2", "D256.PD2"),  # 512-token q, k, v: 192 256-row tiles
-    (256, [5632, 5632], 2048, "D256.PD2", "D256.PD2"),        # 256-token gate, up: 176 256-row tiles
-    (500, [3000, 2800], 1030, "D256.PD2", "D256.PD2"),        # ragged tokens, rows and K: 184 256-row tiles
-    (700, [2048, 1500], 1030, "D256.PD2", "D256.PD2"),        # 154 256-row tiles
+    (512, [2048, 2048, 2048], 2048, "D256", "D256"),  # 512-token q, k, v: 192 256-row tiles
+    (256, [5632, 5632], 2048, "D256", "D256"),        # 256-token gate, up: 176 256-row tiles
+    (500, [3000, 2800], 1030, "D256", "D256"),        # ragged tokens, rows and K: 184 256-row tiles
+    (700, [2048, 1500], 1030, "D256", "D256"),        # 154 256-row tiles
 ]
 
 
@@ -392,10 +398,10 @@ def test_matmul_workspace_balance(N, Ms, K, form_ws, form_plain):
 
 
 @pytest.mark.parametrize("N,Ms,K,form_ws,form_plain", [
-    (192, [11008], 1030, "D256.PD2", "D256.PD2"),    # 129 256-row tiles
-    (570, [4300], 1000, "D256.PD2", "D256.PD2"),     # 153
-    (1216, [2049], 1030, "D256.PD2", "D256.PD2"),    # 171
-    (640, [4200], 1000, "D256.PD2", "D256.PD2"),     # 170
+    (192, [11008], 1030, "D256", "D256"),    # 129 256-row tiles
+    (570, [4300], 1000, "D256", "D256"),     # 153
+    (1216, [2049], 1030, "D256", "D256"),    # 171
+    (640, [4200], 1000, "D256", "D256"),     # 170
     (1024, [4096], 1000, "D256", "D256"),            # 256: whole rounds of either height
     (19000, [128], 1030, "D128", "D128"),            # 297 tiles of either height: two rounds of 256-row ones
 ])
@@ -515,9 +521,8 @@ def test_matmul_random_shapes_every_plan():
 
 
 def test_matmul_workspace_leaves_several_rounds_unsplit():
-    """704 tiles (a 512-token gate and up) take several rounds of two
-    workgroups per CU: the dispatch evens the CUs out itself and the split
-    does not pay, so a workspace changes nothing there."""
+    """A 512-token gate and up (240 tiles of 384 rows, one round) fills the CUs: a
+    workspace changes nothing there."""
     N, M, K = 512, 5632, 2048
     rng = np.random.default_rng(11)
     ba = wxo_q8.DeviceBuffer.from_array(rng.standard_normal(N * K).astype(np.float32))
@@ -529,7 +534,7 @@ def test_matmul_workspace_leaves_several_rounds_unsplit():
     wxo_q8.matmul_q8_multi_device(ba, [(bw, bs, outs[0], M), (bw, bs, outs[1], M)], N, K, workspace=ws,
                                   workspace_bytes=ws_bytes)
     wxo_q8.synchronize()
-    assert wxo_q8.last_variant().split()[1] == "D128", wxo_q8.last_variant()
+    assert wxo_q8.last_variant().split()[1] == "D384", wxo_q8.last_variant()
     assert_bits_equal(outs[1].download(np.float32, N * M), outs[0].download(np.float32, N * M), "same weight")
 
 
@@ -820,16 +825,17 @@ def test_matmul_weight_past_4_gib():
     assert_matmul(np.ascontiguousarray(y[:, cols]), a, wsub, s[cols], T, len(cols), K)
 
 
-@pytest.mark.parametrize("N,M,K,ws", [
-    (40, 300, 1030, False),    # 32-row tiles, two K groups
-    (40, 300, 4500, True),     # the same, K split between workgroups
-    (300, 2048, 520, False),   # 64-row tiles
-    (256, 6144, 600, False),   # 128-row tiles, two K groups
-    (512, 2048, 4096, True),   # 256-row tiles, K split between workgroups
-    (512, 6100, 330, False),   # 256-row tiles
-    (510, 11200, 330, False),  # 384-row tiles
+@pytest.mark.parametrize("N,M,K,ws,form", [
+    (40, 300, 1030, False, "matmul.tokens_as_vectors"),        # the k-split kernel
+    (40, 300, 4100, False, "FB1.PD4.ksplit2"),                 # 32-row tiles, two K groups
+    (40, 300, 4500, True, "FB1.PD4.ksplit2.wgsplit4"),         # the same, K split between workgroups
+    (300, 2048, 520, False, "FB2.PD4.ksplit2"),                # 64-row tiles
+    (256, 6144, 600, False, "FB4.ksplit2"),                    # 128-row tiles, two K groups
+    (512, 2048, 4096, True, "D256.split4"),                    # 256-row tiles, K split between workgroups
+    (512, 6100, 330, False, "D256"),
+    (510, 11200, 330, False, "D384"),
 ])
-def test_matmul_activations_past_the_f16_window(N, M, K, ws):
+def test_matmul_activations_past_the_f16_window(N, M, K, ws, form):
     """Activations that no one scaled f16 pair holds together (large, tiny,
     subnormal and infinite ones among ordinary ones, and a token tile of tiny
     ones only).  A third of the weight rows see the tiny ones alone (their
@@ -860,6 +866,7 @@ def test_matmul_activations_past_the_f16_window(N, M, K, ws):
     wxo_q8.matmul_q8_multi_device(ba, [(bw, bs, out, M)], N, K, workspace=work, workspace_bytes=nbytes)
     wxo_q8.synchronize()
     print(wxo_q8.last_variant(), flush=True)
+    assert wxo_q8.last_variant().split()[1] == form, wxo_q8.last_variant()
     rows = np.unique(np.r_[np.arange(0, N, 23), 1, 5 % N, 7 % N, N // 2, min(N - 1, 70), N - 1])
     assert_matmul(out.download(np.float32, N * M), a, w, s, N, M, K, rows=rows)
 
@@ -870,18 +877,18 @@ def test_matmul_activations_past_the_f16_window(N, M, K, ws):
     (17, [3000, 2000, 700, 15], 1000, "matmul.tokens_as_vectors"),  # two passes, the second with one token
     (32, [2500, 2500], 3072, "matmul.tokens_as_vectors"),
     (16, [4200, 500], 4095, "matmul.tokens_as_vectors"),
-    (33, [300], 1030, "x16.ksplit2"),                           # fewer tiles than workgroups per pass
-    (64, [2048, 2048, 2048], 2048, "x16.ksplit2"),              # 6 tile passes per CU
-    (77, [1000, 1, 530], 769, "x16.ksplit2"),
-    (140, [3500], 3073, "x16.ksplit2"),                         # 219 tiles, nine passes: 8 tiles a workgroup
+    (33, [300], 1030, "matmul.tokens_as_vectors"),                           # fewer tiles than workgroups per pass
+    (64, [2048, 2048, 2048], 2048, "matmul.tokens_as_vectors"),              # 6 tile passes per CU
+    (77, [1000, 1, 530], 769, "matmul.tokens_as_vectors"),
+    (140, [3500], 3073, "matmul.tokens_as_vectors"),                         # 219 tiles, nine passes: 8 tiles a workgroup
     (140, [4080], 3073, "FB2.PD4.ksplit2"),                     # 10
-    (4096, [100], 1024, "x16.ksplit2"),                         # a pass per CU
+    (4096, [100], 1024, "matmul.tokens_as_vectors"),                         # a pass per CU
     (2049, [272], 2048, "FB2.PD4.ksplit2"),                     # 129 workgroups of 17 tiles
-    (2049, [144], 2048, "x16.ksplit2"),                         # of 9
+    (2049, [144], 2048, "matmul.tokens_as_vectors"),                         # of 9
     (2049, [145], 2048, "FB1.PD4.ksplit2"),                     # of 10
-    (48, [5440], 512, "x16.ksplit2"),                           # 4 tiles a workgroup, half of the waves without codes
+    (48, [5440], 512, "matmul.tokens_as_vectors"),                           # 4 tiles a workgroup, half of the waves without codes
     (48, [5441], 512, "FB1.PD4.ksplit2"),                       # one more
-    (40, [1000, 33], 767, "x16.ksplit2"),
+    (40, [1000, 33], 767, "matmul.tokens_as_vectors"),
     (40, [1000], 511, "FB1.PD4.ksplit2"),
 ])
 def test_matmul_tokens_on_the_ksplit_kernel(N, Ms, K, form):
@@ -907,7 +914,7 @@ def test_matmul_tokens_on_the_ksplit_kernel(N, Ms, K, form):
         wxo_q8.matmul_q8_multi_device(ba, bufs, N, K)
         wxo_q8.synchronize()
         v = wxo_q8.last_variant().split()
-        assert v[1] == form and (v[0].startswith("matvec_q8_ksplit") or N > 32), v
+        assert v[1] == form and v[0].startswith("matvec_q8_ksplit" if form.startswith("matmul.") else "matmul_q8"), v
         runs.append([b[2].download(np.float32, N * b[3] + 64) for b in bufs])
     rows = np.arange(N) if N <= 140 else np.unique(np.r_[np.arange(0, N, 61), 3, N - 1])
     for (w, s, M), got, again in zip(host, *runs):
@@ -942,18 +949,19 @@ def test_matmul_tokens_of_many_scales(N, M, K, ws):
     assert_matmul(out.download(np.float32, N * M), a, w, s, N, M, K, rows=rows)
 
 
-@pytest.mark.parametrize("N,M,K,ws", [
-    (65, 2048, 300, False),    # 32-row tiles, one token in the second tile
-    (40, 300, 4500, True),     # the same, K split between workgroups
-    (300, 2048, 500, False),   # 64-row tiles, two K groups
-    (379, 2860, 300, False),   # the same, one group
-    (450, 4096, 600, False),   # 128-row tiles, two K groups
-    (19000, 128, 1030, True),  # 128-row tiles, two workgroups per CU
-    (512, 2048, 4096, True),   # 256-row tiles, K split between workgroups
-    (577, 6100, 1030, False),  # 256-row tiles
-    (510, 11200, 2061, False), # 384-row tiles
+@pytest.mark.parametrize("N,M,K,ws,form", [
+    (65, 2048, 300, False, "FB1.PD4.ksplit2"),                 # 32-row tiles, one token in the second tile
+    (40, 300, 4500, True, "FB1.PD4.ksplit2.wgsplit4"),         # the same, K split between workgroups
+    (300, 2048, 500, False, "FB2.PD4.ksplit2"),                # 64-row tiles, two K groups
+    (379, 2860, 300, False, "FB2.PD4"),                        # the same, one group
+    (450, 4096, 600, False, "FB4.ksplit2"),                    # 128-row tiles, two K groups
+    (19000, 128, 1030, True, "D128"),                          # 128-row tiles, two workgroups per CU
+    (2048, 4096, 4100, False, "D256"),
+    (512, 2048, 4096, True, "D256.split4"),                    # 256-row tiles, K split between workgroups
+    (577, 6100, 1030, False, "D256"),
+    (510, 11200, 2061, False, "D384"),
 ])
-def test_matmul_activations_that_grow(N, M, K, ws):
+def test_matmul_activations_that_grow(N, M, K, ws, form):
     """Tokens whose largest values come late: their powers of two fall during the
     run, at steps of their own.  Some tokens are zero at first or throughout, some
     start with an infinity or a NaN; some weight rows have no code at all, or only
@@ -983,7 +991,7 @@ def test_matmul_activations_that_grow(N, M, K, ws):
     wxo_q8.matmul_q8_multi_device(ba, [(bw, bs, out, M)], N, K, workspace=work, workspace_bytes=nbytes)
     wxo_q8.synchronize()
     print(wxo_q8.last_variant(), flush=True)
-    assert wxo_q8.last_variant().startswith("matmul_q8 "), wxo_q8.last_variant()
+    assert wxo_q8.last_variant().split()[1] == form, wxo_q8.last_variant()
     rows = np.unique(np.r_[np.arange(0, min(N, 64), 3), np.arange(0, N, 1 + N // 24), 1, 2, 3, 4, 9, N - 1])
     assert_matmul(out.download(np.float32, N * M), a, w, s, N, M, K, rows=rows)
 
@@ -1062,8 +1070,8 @@ def test_matmul_time_does_not_depend_on_the_values():
     (200, 5300, 64, "FB2.PD4 waves=8 rows=64"),        # 168 tiles, one step
     (200, 5300, 390, "FB4.ksplit2 waves=8 rows=128"),
     (1300, 7300, 380, "D128 waves=4 rows=128"),        # two rounds of 384-row tiles
-    (1300, 7300, 386, "D128 waves=8 rows=384"),
-    (500, 11200, 100, "D128 waves=8 rows=384"),        # one round
+    (1300, 7300, 386, "D384 waves=8 rows=384"),
+    (500, 11200, 100, "D384 waves=8 rows=384"),        # one round
 ])
 def test_matmul_few_steps(N, M, K, form):
     """Rows of at most 384 codes take smaller tiles where several workgroups per CU

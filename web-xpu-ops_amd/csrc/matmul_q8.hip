@@ -1458,10 +1458,7 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
     }
     if (on_ksplit) {
         const hipError_t e = launch_matvec_q8_batched_multi(pv, n, a, K, N, dev, stream, variant);
-        if (variant && e == hipSuccess) {
-            variant->kernel = kname;
-            variant->form = "x16.ksplit2";  // K split over a workgroup's waves, two tiles per barrier
-        }
+        if (variant && e == hipSuccess) variant->form = "matmul.tokens_as_vectors";
         return e;
     }
     // One workgroup of 8 waves per CU on the direct kernel, each wave 32 or 48
@@ -1500,7 +1497,7 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         // (33.2, 48.3, 127, 30.4).  More 256-row tiles than CUs (19000 x 128 x 2048, every
         // tile half empty) would take two rounds: 67.9 against 41.9.
         if (t4 < 2ull * cus && t8 <= cus) {
-            set_variant(variant, kname, "D256.PD2", 8, 256, 0, (int)kBN, (uint32_t)((t8 + 7u) / 8u * 8u));
+            set_variant(variant, kname, "D256", 8, 256, 0, (int)kBN, (uint32_t)((t8 + 7u) / 8u * 8u));
             return launch_direct<8, 2>(a, p, n, N, K, stream);
         }
         // Long rows whose 128-row tiles make two or more whole rounds of two per CU
@@ -1521,7 +1518,7 @@ hipError_t launch_matmul_q8_multi(const float* a, const MatmulProjection* projec
         // stores: 1371 x 7327 x 64 25.2 -> 21.7 us, 519 x 16882 x 192 27.4 -> 24.8,
         // 928 x 8984 x 384 34.9 -> 34.1; past it 2412 x 3664 x 512 39.4 -> 40.9.
         if (rows384 && (r12 == 1u || steps > 6u)) {
-            set_variant(variant, kname, "D128", 8, 384, 0, (int)kBN, (uint32_t)((t12 + 7u) / 8u * 8u));
+            set_variant(variant, kname, "D384", 8, 384, 0, (int)kBN, (uint32_t)((t12 + 7u) / 8u * 8u));
             return launch_direct<8, 3>(a, p, n, N, K, stream);
         }
         set_variant(variant, kname, "D128", 4, 128, 0, (int)kBN, (uint32_t)((t4 + 7u) / 8u * 8u));
