@@ -274,9 +274,11 @@ int wxo_quantize_pack_q8_multi(const float* const* inputs, const uint32_t* Ns, u
 
 /* matmulQ8: output[n*M + m] = (sum_{k<K} a[n*K + k] * sext8(byte k of weight row m)) * scale[m]
  * for n < N (tokens), m < M (weight rows).  a f32 [N, K], weight u32 [M, ceil(K/4)],
- * scale f32 [M], output f32 [N, M].  f32 accumulation on the matrix cores (each
- * activation as a scaled f16 pair, exact to 2^-23, or exactly where it has no
- * such pair); |y - y_ref| <= 1e-5 * sum_k |a * q * s| + 1e-7 against the reference's f64
+ * scale f32 [M], output f32 [N, M].  f32 accumulation on the matrix cores.  Each
+ * activation is exact for up to 32 tokens and where the k-split kernel runs (512 <=
+ * K <= 4096, few tokens); otherwise it is a scaled f16 pair, within 2^-23 of it, or
+ * within 2^-45 of its token's largest one where it is under 2^-22 of that (sums
+ * small enough for this to show are taken again exactly).  |y - y_ref| <= 1e-5 * sum_k |a * q * s| + 1e-7 against the reference's f64
  * sum of per-term dequantized products.  K = 0 gives zeros.  K <= 2^22. */
 int wxo_matmul_q8(const float* a, const uint32_t* weight, const float* scale, float* output, uint32_t N,
                   uint32_t M, uint32_t K, wxo_stream_t stream);
@@ -296,11 +298,10 @@ int wxo_matmul_q8_multi(const float* a, const uint32_t* const* weights, const fl
  * counterpart in the reference, which has no workspace.  With room in it,
  * some tiles split their K steps between workgroups whose partial sums meet in
  * a second launch (added in a fixed order: deterministic, and within the same
- * bound of the reference): all of a short prompt's tiles, which would leave
- * most CUs idle, and the last tiles of a prompt whose tiles fill one round of
- * the CUs unevenly, so that every CU holds the same work.  wxo_matmul_q8_workspace_bytes gives the size that allows every
- * split on the current device; less (or NULL and 0) allows fewer splits or
- * none, never an error.  The workspace's contents are scratch between calls;
+ * bound of the reference): those of prompts whose tiles would leave most CUs
+ * idle, over rows long enough for it.  wxo_matmul_q8_workspace_bytes gives the
+ * size that allows every split on the current device; less (or NULL and 0)
+ * allows fewer splits or none, never an error.  The workspace's contents are scratch between calls;
  * calls that share one workspace must not overlap in time. */
 int wxo_matmul_q8_multi_ws(const float* a, const uint32_t* const* weights, const float* const* scales,
                            float* const* outputs, const uint32_t* Ms, uint32_t count, uint32_t N, uint32_t K,

@@ -1091,3 +1091,25 @@ def test_matmul_few_steps(N, M, K, form):
     got = out.download(np.float32, N * M + 64)
     assert np.all(got[N * M:] == np.float32(7.5)), "written past the output"
     assert_matmul(got[:N * M], a, w, s, N, M, K, rows=np.unique(np.r_[np.arange(0, N, 29), 3, N - 1]))
+
+
+@pytest.mark.parametrize("N,M,K", [(100, 520, 500), (300, 2600, 520), (130, 2600, 4100), (512, 6100, 520), (500, 11200, 520)])
+def test_matmul_holds_an_activation_to_23_bits(N, M, K):
+    """Rows with one code of 1 (or -128) and a scale of 1 return what the kernel holds
+    of one activation: the f16 pair is within 2^-23 of it, three quarters of all
+    values exactly, and values far below their token's largest are taken again
+    exactly."""
+    rng = np.random.default_rng(N + M + K)
+    a = rng.standard_normal((N, K)).astype(np.float32)
+    a[:, ::3] *= np.ldexp(np.float32(1), rng.integers(-40, 5, (N, (K + 2) // 3))).astype(np.float32)
+    a *= np.ldexp(np.float32(1), rng.integers(-60, 60, (N, 1))).astype(np.float32)
+    at = rng.integers(0, K, M)
+    codes = np.zeros((M, K), np.int32)
+    codes[np.arange(M), at] = np.where(np.arange(M) % 4 == 3, -128, 1)
+    w = oracle.pack_q8(codes.reshape(-1), M, K)
+    y = np.asarray(wxo_q8.matmulQ8(a=a.reshape(-1), weight=w, scale=np.ones(M, np.float32), N=N, M=M, K=K)).reshape(N, M)
+    assert wxo_q8.last_variant().startswith("matmul_q8"), wxo_q8.last_variant()
+    want = a[:, at].astype(np.float64) * codes[np.arange(M), at]
+    off = np.abs(y.astype(np.float64) - want)
+    assert (off <= 2.0 ** -23 * np.abs(want)).all(), (off / np.abs(want)).max()
+    assert 0.7 < np.mean(off == 0) , np.mean(off == 0)
