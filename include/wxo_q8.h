@@ -276,10 +276,11 @@ int wxo_quantize_pack_q8_multi(const float* const* inputs, const uint32_t* Ns, u
  * for n < N (tokens), m < M (weight rows).  a f32 [N, K], weight u32 [M, ceil(K/4)],
  * scale f32 [M], output f32 [N, M].  f32 accumulation on the matrix cores.  Each
  * activation is exact for up to 32 tokens and where the k-split kernel runs (512 <=
- * K <= 4096, few tokens); otherwise it is a scaled f16 pair, within 2^-23 of it, or
- * within 2^-45 of its token's largest one where it is under 2^-22 of that (sums
- * small enough for this to show are taken again exactly).  |y - y_ref| <= 1e-5 * sum_k |a * q * s| + 1e-7 against the reference's f64
- * sum of per-term dequantized products.  K = 0 gives zeros.  K <= 2^22. */
+ * K <= 4096, few tokens or few rows); otherwise it is a scaled f16 pair, within
+ * 2^-23 of it, or within 2^-45 of its token's largest one where it is under 2^-22
+ * of that (sums small enough for this to show are taken again exactly).
+ * |y - y_ref| <= 1e-5 * sum_k |a * q * s| + 1e-7 against the reference's f64 sum of
+ * per-term dequantized products.  K = 0 gives zeros.  K <= 2^22. */
 int wxo_matmul_q8(const float* a, const uint32_t* weight, const float* scale, float* output, uint32_t N,
                   uint32_t M, uint32_t K, wxo_stream_t stream);
 /* matmulQ8 of several weights on the same activations a [N, K]: outputs[p]
