@@ -109,8 +109,6 @@ struct MatmulProjections {
     uint32_t tiles, parts;
 };
 
-
-
 // Tile `tile` of the launch's sequence -> weight-row tile mt, token tile nt.
 // The sequence takes kTileGroup row tiles at a time (fewer in the last
 // group) and walks all token tiles of the group, its row tiles innermost:
